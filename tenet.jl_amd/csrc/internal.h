@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <string>
+#include <vector>
 
 namespace tenet {
 
@@ -33,6 +34,20 @@ struct GemmTables {
   const int64_t* bC;
 };
 
+// How one contraction runs, chosen when its plan is made (gemm_form): the
+// kernel and tile shape, which operand's free index runs over the lanes, and
+// the tables' strides when all nine are index * stride.
+struct GemmForm {
+  int cfg = 0;
+  int j_is_m = 1;
+  int order = 0;   // one-thread-per-element kernel: fastest class (0: m, 1: n, 2: batch)
+  int affine = 0;
+  int64_t st[9] = {};
+};
+// v: the nine tables (rowA, kA, bA, kB, colB, bB, rowC, colC, bC)
+void gemm_form(const std::vector<int64_t> v[9], int64_t M, int64_t N, int64_t K, int64_t batch, int dtype, int prec,
+               GemmForm* f);
+
 struct GemmLaunch {
   const void* A;
   const void* B;
@@ -40,8 +55,7 @@ struct GemmLaunch {
   GemmTables t;
   int64_t M, N, K, batch;
   int conjA, conjB;
-  int a_mfast;  // rowA has unit stride: load A tiles with consecutive lanes along m
-  int b_nfast;  // colB has unit stride: load B tiles with consecutive lanes along n
+  const GemmForm* form;
   double alpha_re, alpha_im, beta_re, beta_im;
 };
 

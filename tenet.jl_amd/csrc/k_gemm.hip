@@ -17,29 +17,11 @@
 // with i = 4*(l/16) + r for FP32 and i = 4*r + l/16 for FP64.
 #include "../../include/tenet_hip.h"
 #include "internal.h"
+#include "gemm_direct.h"
+
+#include <algorithm>
 
 namespace tenet {
-
-typedef double d4v __attribute__((ext_vector_type(4)));
-typedef float f4v __attribute__((ext_vector_type(4)));
-
-template <typename R>
-struct Acc4;
-template <>
-struct Acc4<double> {
-  using T = d4v;
-};
-template <>
-struct Acc4<float> {
-  using T = f4v;
-};
-
-__device__ __forceinline__ d4v mfma16x16x4(double a, double b, d4v c) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-}
-__device__ __forceinline__ f4v mfma16x16x4(float a, float b, f4v c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 constexpr int BK = 16, PADK = 4;
 
@@ -343,69 +325,227 @@ __device__ __forceinline__ void partial_sum(const R* __restrict__ part, int nchu
       }
 }
 
-// One Cfg::BM x Cfg::BN output tile (tm, tn) of batch entry z over the whole K range.
-template <typename S2, typename R, typename Cfg>
-__device__ __forceinline__ void gemm_tile(const TileView& p, int64_t tm, int64_t tn, int64_t z, GemmSmem<R>& sm) {
-  TileAcc<R, Cfg> acc;
-  gemm_accumulate<S2, R, Cfg>(p, tm, tn, z, 0, p.K, sm, acc);
-  gemm_store<S2, R, Cfg>(p, tm, tn, z, acc);
-}
+// ---- one contraction per launch -----------------------------------------------
+// Workgroup shapes of the direct kernel: four waves, either all on the same
+// TI x TJ blocks with the K steps dealt round robin (WK = 4: short chains and
+// four times the waves where a product has few tiles), or side by side along
+// j (WK = 1: a short K has no steps to deal).
+struct DirectCfg {
+  int ti, tj, wj, wk;
+  double eff;  // share of its modelled rate that the shape reaches (fitted, see choose_direct)
+};
+enum { D16 = 0, D16x32, D32, D32x64, S32, S16, DIRECT_CFGS, ELEMENTS = DIRECT_CFGS };
+static constexpr DirectCfg kDirect[DIRECT_CFGS] = {
+    {1, 1, 1, 4, 0.65}, {1, 2, 1, 4, 0.75}, {2, 2, 1, 4, 0.75},
+    {2, 4, 1, 4, 0.80}, {2, 2, 4, 1, 0.85}, {1, 2, 4, 1, 0.75}};
+
+struct DirectArgs {
+  const void* X;
+  const void* Y;
+  void* C;
+  // offsets of rowX, kX, batchX, rowY, kY, batchY, rowC, colC, batchC
+  const int64_t* tab[9];
+  int64_t st[9];
+  int64_t I, J, K;
+  int64_t tiles_i, tiles_j;
+  int conjX, conjY;
+  Scalars sc;
+};
 
 // Map a physical workgroup id to a logical tile so that the tiles one XCD
 // receives (ids congruent mod 8 are dispatched to the same XCD) are
-// neighbours in the tile grid and share A/B panels in that XCD's L2.
+// neighbours in the tile grid and share X / Y panels in that XCD's L2.
 __device__ __forceinline__ int64_t xcd_remap(int64_t pid, int64_t total) {
   constexpr int64_t NXCD = 8;
   if (total % NXCD != 0) return pid;
   return (pid % NXCD) * (total / NXCD) + pid / NXCD;
 }
 
-template <typename S2, typename R, typename Cfg>
-__global__ __launch_bounds__(256) void gemm_kernel(TileView p, int64_t tiles_m, int64_t tiles_n, int64_t batch) {
-  __shared__ GemmSmem<R> sm;
-  const int64_t per_batch = tiles_m * tiles_n;
-  const int64_t total = per_batch * batch;
-  const int64_t lid = xcd_remap((int64_t)blockIdx.x, total);
-  const int64_t z = lid / per_batch;
-  const int64_t t = lid - z * per_batch;
-  gemm_tile<S2, R, Cfg>(p, t % tiles_m, t / tiles_m, z, sm);
+template <typename S2, typename R, int TI, int TJ, int WJ, int WK, int U, bool AFF>
+__global__ __launch_bounds__(256, 2) void gemm_direct_kernel(DirectArgs p) {
+  static_assert(WJ * WK == 4, "four waves");
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wk = wave % WK, wj = wave / WK;
+  const int64_t total = gridDim.x, id = xcd_remap((int64_t)blockIdx.x, total);
+  const int64_t per = p.tiles_i * p.tiles_j;
+  const int64_t z = per == total ? 0 : id / per, t = id - z * per;
+  const int64_t tj = t / p.tiles_i, ti = t - tj * p.tiles_i;
+  const int64_t i0 = ti * (16 * TI), j0 = (tj * WJ + wj) * (16 * TJ);
+  auto off = [&](int k) { return Offsets<AFF>{p.tab[k], p.st[k]}; };
+  const S2* X = static_cast<const S2*>(p.X) + off(2)[z];
+  const S2* Y = static_cast<const S2*>(p.Y) + off(5)[z];
+  BlockAcc<R, TI, TJ> acc;
+  direct_accumulate<S2, R, TI, TJ, WK, U, AFF>(X, Y, off(0), off(1), off(3), off(4), i0, p.I, j0, p.J, 0, p.K, wk,
+                                               p.conjX != 0, p.conjY != 0, acc);
+  if constexpr (WK > 1) {
+    __shared__ R red[WK / 2 * TI * TJ * 512];
+    direct_fold<R, TI, TJ, WK>(red, wk, acc);
+    if (wk > 0) return;
+  }
+  direct_store<S2, R, TI, TJ, AFF>(static_cast<S2*>(p.C) + off(8)[z], off(6), off(7), i0, p.I, j0, p.J, p.sc, acc);
 }
 
-template <typename S2, typename R>
-static int launch_gemm_t(const GemmLaunch& g, hipStream_t s) {
-  TileView p;
-  p.A = g.A;
-  p.B = g.B;
-  p.C = g.C;
-  p.t = g.t;
-  p.M = g.M;
-  p.N = g.N;
-  p.K = g.K;
-  p.a_mfast = g.a_mfast;
-  p.b_nfast = g.b_nfast;
-  p.conjA = g.conjA;
-  p.conjB = g.conjB;
-  p.alpha_re = g.alpha_re;
-  p.alpha_im = g.alpha_im;
-  p.beta_re = g.beta_re;
-  p.beta_im = g.beta_im;
-  // 64 x 64 tiles, or 32 x 32 when 64 x 64 would leave most of the 256 CUs idle
-  // (a 512 x 512 product: 64 workgroups against 256)
-  const bool small = ((g.M + 63) / 64) * ((g.N + 63) / 64) * g.batch < 128;
-  const int64_t bt = small ? 32 : 64;
-  const int64_t tm = (g.M + bt - 1) / bt, tn = (g.N + bt - 1) / bt;
-  const int64_t total = tm * tn * g.batch;
-  if (total <= 0) return TENET_OK;
+// One thread per output element, for products of so few terms that an MFMA
+// block would be mostly padding (permutations, Hadamard scalings): consecutive
+// threads take consecutive entries of the index class whose entries of C are
+// closest (order 0: m, 1: n, 2: batch).
+template <typename S2, typename R, typename IT>
+__global__ __launch_bounds__(256) void gemm_elements_kernel(GemmTables t, const S2* __restrict__ A,
+                                                            const S2* __restrict__ B, S2* __restrict__ C, IT total,
+                                                            IT ext0, IT ext1, int K, int order, int conjA, int conjB,
+                                                            Scalars sc) {
+  const R sa = conjA ? (R)-1 : (R)1, sb = conjB ? (R)-1 : (R)1;
+  for (IT e = (IT)blockIdx.x * 256 + threadIdx.x; e < total; e += (IT)gridDim.x * 256) {
+    const IT rest = e / ext0, i0 = e - rest * ext0;
+    const IT i2 = rest / ext1, i1 = rest - i2 * ext1;
+    const int64_t m = order == 0 ? i0 : i1;
+    const int64_t n = order == 0 ? i1 : (order == 1 ? i0 : i2);
+    const int64_t z = order == 2 ? i0 : i2;
+    const S2* a0 = A + (t.rowA[m] + t.bA[z]);
+    const S2* b0 = B + (t.colB[n] + t.bB[z]);
+    R cr = 0, ci = 0;
+    for (int k = 0; k < K; ++k) {
+      const S2 a = a0[t.kA[k]], b = b0[t.kB[k]];
+      const R ar = (R)a.x, ai = sa * (R)a.y, br = (R)b.x, bi = sb * (R)b.y;
+      cr += ar * br - ai * bi;
+      ci += ar * bi + ai * br;
+    }
+    store_scaled<S2>(C + (t.rowC[m] + t.colC[n] + t.bC[z]), (double)cr, (double)ci, sc);
+  }
+}
+
+// The workgroup shape with the least modelled time, in cycles of one CU: per
+// K step the larger of its MFMAs (64 cycles each in FP64, 32 in FP32) and
+// its operand loads (24 cycles of the CU's address unit per wave and block,
+// twice that where 16 lanes read 16 rows instead of neighbours), over the
+// rounds the 256 CUs need, plus the epilogue of a tile.  On 45 measured shapes
+// (K 4..3840, 24 x 38 to 590000 x 20, both types) the choice is 2% slower than
+// the best of the six in the mean, 26% at worst (complex64 300 x 600 x 300,
+// 11.8 against 9.4 us).  From K = 128 on the WK = 1 shapes never won.
+static int choose_direct(double cyc, int64_t I, int64_t J, int64_t K, int64_t batch, bool x_adj, bool y_adj) {
+  const double clx = x_adj ? 24 : 48, cly = y_adj ? 24 : 48;
+  int best = 0;
+  double best_t = 0.0;
+  for (int c = 0; c < DIRECT_CFGS; ++c) {
+    const DirectCfg& f = kDirect[c];
+    if (f.wk == 1 && K >= 128) continue;
+    const int64_t ei = 16 * f.ti, ej = 16 * f.tj * f.wj;
+    const double tiles = (double)((I + ei - 1) / ei) * (double)((J + ej - 1) / ej) * (double)batch;
+    const double rounds = tiles > 1024 ? tiles / 256 : std::ceil(tiles / 256);
+    const double steps = (double)((K + 4 * f.wk - 1) / (4 * f.wk));
+    const double step = std::max(4 * cyc * f.ti * f.tj, 4 * (f.ti * clx + f.tj * cly));
+    const double t = rounds * (steps * step / f.eff + 200.0 * f.ti * f.tj);
+    if (c == 0 || t < best_t) {
+      best = c;
+      best_t = t;
+    }
+  }
+  return best;
+}
+
+void gemm_form(const std::vector<int64_t> v[9], int64_t M, int64_t N, int64_t K, int64_t batch, int dtype, int prec,
+               GemmForm* f) {
+  auto stride_of = [](const std::vector<int64_t>& t, int64_t* st) {
+    *st = t.size() > 1 ? t[1] - t[0] : 0;
+    for (size_t i = 0; i < t.size(); ++i)
+      if (t[i] != (int64_t)i * *st) return false;
+    return true;
+  };
+  f->affine = 1;
+  for (int i = 0; i < 9; ++i)
+    if (!stride_of(v[i], &f->st[i])) f->affine = 0;
+  auto gap = [&](int i) { return v[i].size() > 1 ? std::llabs(v[i][1] - v[i][0]) : INT64_MAX; };
+  const int64_t gm = gap(6), gn = gap(7), gz = gap(8);
+  f->order = (gm <= gn && gm <= gz) ? 0 : (gn <= gz ? 1 : 2);
+  f->j_is_m = gm <= gn ? 1 : 0;
+  // up to two outputs per gathered row: 160000 x 8 by 8 x 2 in 9.4 us either
+  // way, a Hadamard scaling of 51200 entries 2.1 us (MFMA blocks 4.5), a dot
+  // of 8 terms per row over 4e6 rows 115 us (434); with three or more columns
+  // the MFMA blocks win (160000 x 4 by 4 x 4: 7.4 against 11.8 us)
+  if (K <= 8 && std::min(M, N) <= 2) {
+    f->cfg = ELEMENTS;
+    return;
+  }
+  const bool a_adj = gap(0) == 1 || M == 1, b_adj = gap(4) == 1 || N == 1;
+  const double cyc = dtype == TENET_C128 && prec == TENET_PREC_NATIVE ? 64 : 32;
+  if (f->j_is_m)
+    f->cfg = choose_direct(cyc, N, M, K, batch, b_adj, a_adj);
+  else
+    f->cfg = choose_direct(cyc, M, N, K, batch, a_adj, b_adj);
+}
+
+template <typename S2, typename R, int TI, int TJ, int WJ, int WK, int U>
+static int launch_direct(DirectArgs& p, const GemmLaunch& g, hipStream_t s) {
+  p.tiles_i = (p.I + 16 * TI - 1) / (16 * TI);
+  p.tiles_j = (p.J + 16 * TJ * WJ - 1) / (16 * TJ * WJ);
+  const double total = (double)p.tiles_i * (double)p.tiles_j * (double)g.batch;
   if (total > 0x7fffffffLL) {
     set_error("contraction too large for one launch");
     return TENET_ERR_UNSUPPORTED;
   }
-  if (small)
-    hipLaunchKernelGGL((gemm_kernel<S2, R, Tile32>), dim3((unsigned)total), dim3(256), 0, s, p, tm, tn, g.batch);
+  if (g.form->affine)
+    hipLaunchKernelGGL((gemm_direct_kernel<S2, R, TI, TJ, WJ, WK, U, true>), dim3((unsigned)total), dim3(256), 0, s,
+                       p);
   else
-    hipLaunchKernelGGL((gemm_kernel<S2, R, Tile64>), dim3((unsigned)total), dim3(256), 0, s, p, tm, tn, g.batch);
+    hipLaunchKernelGGL((gemm_direct_kernel<S2, R, TI, TJ, WJ, WK, U, false>), dim3((unsigned)total), dim3(256), 0, s,
+                       p);
   TENET_HIP_CHECK(hipGetLastError());
   return TENET_OK;
+}
+
+template <typename S2, typename R, typename IT>
+static int launch_elements(const GemmLaunch& g, const Scalars& sc, hipStream_t s) {
+  const int order = g.form->order;
+  const int64_t total = g.M * g.N * g.batch;
+  const int64_t ext0 = order == 0 ? g.M : (order == 1 ? g.N : g.batch), ext1 = order == 0 ? g.N : g.M;
+  const int64_t blocks = std::min<int64_t>((total + 255) / 256, 1 << 20);
+  hipLaunchKernelGGL((gemm_elements_kernel<S2, R, IT>), dim3((unsigned)blocks), dim3(256), 0, s, g.t,
+                     (const S2*)g.A, (const S2*)g.B, (S2*)g.C, (IT)total, (IT)ext0, (IT)ext1, (int)g.K, order,
+                     g.conjA, g.conjB, sc);
+  TENET_HIP_CHECK(hipGetLastError());
+  return TENET_OK;
+}
+
+template <typename S2, typename R>
+static int launch_gemm_t(const GemmLaunch& g, hipStream_t s) {
+  const Scalars sc{g.alpha_re, g.alpha_im, g.beta_re, g.beta_im};
+  if (g.form->cfg == ELEMENTS) {
+    if (g.M * g.N * g.batch <= (int64_t)INT32_MAX) return launch_elements<S2, R, uint32_t>(g, sc, s);
+    return launch_elements<S2, R, int64_t>(g, sc, s);
+  }
+  // i and j are A's and B's free indices, or B's and A's when C's entries are
+  // adjacent along m (a store instruction then writes neighbours)
+  DirectArgs p{};
+  p.C = g.C;
+  p.K = g.K;
+  p.sc = sc;
+  const int64_t* tab[9] = {g.t.rowA, g.t.kA, g.t.bA, g.t.kB, g.t.colB, g.t.bB, g.t.rowC, g.t.colC, g.t.bC};
+  static const int from[2][9] = {{0, 1, 2, 4, 3, 5, 6, 7, 8}, {4, 3, 5, 0, 1, 2, 7, 6, 8}};
+  const int jm = g.form->j_is_m;
+  for (int k = 0; k < 9; ++k) {
+    p.tab[k] = tab[from[jm][k]];
+    p.st[k] = g.form->st[from[jm][k]];
+  }
+  p.X = jm ? g.B : g.A;
+  p.Y = jm ? g.A : g.B;
+  p.conjX = jm ? g.conjB : g.conjA;
+  p.conjY = jm ? g.conjA : g.conjB;
+  p.I = jm ? g.N : g.M;
+  p.J = jm ? g.M : g.N;
+  switch (g.form->cfg) {
+    case D16:
+      return launch_direct<S2, R, 1, 1, 1, 4, 1>(p, g, s);
+    case D16x32:
+      return launch_direct<S2, R, 1, 2, 1, 4, 2>(p, g, s);
+    case D32:
+      return launch_direct<S2, R, 2, 2, 1, 4, 1>(p, g, s);
+    case D32x64:
+      return launch_direct<S2, R, 2, 4, 1, 4, 1>(p, g, s);
+    case S32:
+      return launch_direct<S2, R, 2, 2, 4, 1, 1>(p, g, s);
+    default:
+      return launch_direct<S2, R, 1, 2, 4, 1, 2>(p, g, s);
+  }
 }
 
 int launch_split_gemm(const GemmLaunch& g, int dtype, int prec, hipStream_t s, void* ws, size_t ws_bytes);

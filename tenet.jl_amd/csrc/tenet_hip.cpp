@@ -76,7 +76,7 @@ struct tenet_plan_s {
   tenet_ctx ctx = nullptr;
   int dtype = 0, prec = 0;
   int64_t M = 0, N = 0, K = 0, batch = 0;
-  int a_mfast = 0, b_nfast = 0;
+  GemmForm form;
   int64_t* tables = nullptr;
   GemmTables t{};
   size_t ws_bytes = 0;
@@ -964,6 +964,23 @@ static void set_tables(GemmTables& t, int64_t* T, const size_t* off) {
   t.bC = T + off[8];
 }
 
+// Where the vendor library's GEMM beats the direct kernel (measured, library
+// against direct, us).  complex128: large products whose 64 x 64 tiles fill the
+// rounds of 256 CUs (1024^3, N/T 126 : 145, C/N 136 : 145; 4096^3 7640 : 8090);
+// a last round mostly empty costs the library more than the tiles' rate gains
+// (3072 x 768 x 3840, 2.25 rounds, 1300 : 1140; 1536^3 538 : 500).  complex64:
+// A contiguous along K from 400^3 on (13.5 : 15.7; 700^3 26 : 40; but
+// 300 x 300 x 600 19.6 : 11.7), otherwise only very large ones (2048^3
+// 538 : 612; 1024^3 157 : 92, 250 x 1250 x 462 42 : 20).
+static bool lib_pays(int dtype, rocblas_operation opA, int64_t M, int64_t N, int64_t K, int64_t batch) {
+  const double fl = 8.0 * M * N * K * batch;
+  if (dtype == TENET_C128) {
+    const double rounds = (double)((M + 63) / 64) * ((N + 63) / 64) * batch / 256.0;
+    return fl >= 5e9 && rounds >= 0.92 * std::ceil(rounds);
+  }
+  return fl >= (opA == rocblas_operation_none ? 3e10 : 5e8);
+}
+
 static int build_plan(tenet_ctx ctx, int dtype, int prec, const tenet_tdesc* a, const tenet_tdesc* b,
                       const tenet_tdesc* c, tenet_plan p) {
   HostPlan hp;
@@ -975,13 +992,14 @@ static int build_plan(tenet_ctx ctx, int dtype, int prec, const tenet_tdesc* a, 
   p->N = hp.N;
   p->K = hp.K;
   p->batch = hp.batch;
-  p->a_mfast = hp.a_mfast;
-  p->b_nfast = hp.b_nfast;
+  gemm_form(hp.v, hp.M, hp.N, hp.K, hp.batch, dtype, prec, &p->form);
   p->spanA = hp.spanA;
   p->spanB = hp.spanB;
   p->spanC = hp.spanC;
-  if (prec == TENET_PREC_NATIVE && 8.0 * hp.M * hp.N * hp.K * hp.batch >= LIB_MIN_FLOPS)
+  if (prec == TENET_PREC_NATIVE && 8.0 * hp.M * hp.N * hp.K * hp.batch >= LIB_MIN_FLOPS) {
     p->lib = plain_layout(hp);
+    p->lib.ok = p->lib.ok && lib_pays(dtype, p->lib.opA, hp.M, hp.N, hp.K, hp.batch);
+  }
   std::vector<int64_t> host;
   size_t off[9];
   for (int i = 0; i < 9; ++i) {
@@ -1092,8 +1110,7 @@ static int exec_plan(tenet_plan p, hipStream_t s, const void* A, const void* B, 
   g.batch = p->batch;
   g.conjA = conj_a;
   g.conjB = conj_b;
-  g.a_mfast = p->a_mfast;
-  g.b_nfast = p->b_nfast;
+  g.form = &p->form;
   g.alpha_re = alpha ? alpha[0] : 1.0;
   g.alpha_im = alpha ? alpha[1] : 0.0;
   g.beta_re = beta ? beta[0] : 0.0;
