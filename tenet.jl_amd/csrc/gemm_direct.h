@@ -61,13 +61,24 @@ struct Offsets {
   }
 };
 
+// Two neighbouring entries of a complex64 operand, loaded at once (rows of odd
+// length leave them 8-byte aligned).
+typedef float f4pair __attribute__((ext_vector_type(4), aligned(8)));
+
 // acc = sum over this wave's share of k in [k_lo, k_hi) for the blocks at
 // rows i0.. (of I) and columns j0.. (of J): WK waves take the K steps of 4
 // round robin (this one is number wk), U steps per load group, the next
 // group's loads in flight during the current group's products.  Rows and
 // columns past the edge read the last valid one (their results are never
 // stored); k past the end contributes zeros.
-template <typename S2, typename R, int TI, int TJ, int WK, int U, bool AFF>
+//
+// PX / PY (complex64): that operand's entries k, k + 1 (k even) are adjacent,
+// and each lane takes them with one 16-byte load.  A lane group then covers
+// k = 2 g, 2 g + 1 of a span of 8 instead of k = g of spans of 4; the sum does
+// not care which lane group holds which k.  An operand read along its rows
+// costs one cache-line access per row and load whatever the width, so this
+// halves the accesses that bound it.
+template <typename S2, typename R, int TI, int TJ, int WK, int U, bool AFF, bool PX, bool PY>
 __device__ __forceinline__ void direct_accumulate(const S2* __restrict__ X, const S2* __restrict__ Y,
                                                   const Offsets<AFF>& rowX, const Offsets<AFF>& kX,
                                                   const Offsets<AFF>& rowY, const Offsets<AFF>& kY, int64_t i0,
@@ -87,51 +98,82 @@ __device__ __forceinline__ void direct_accumulate(const S2* __restrict__ X, cons
       acc.r[a][b] = typename BlockAcc<R, TI, TJ>::V4{0, 0, 0, 0};
       acc.i[a][b] = typename BlockAcc<R, TI, TJ>::V4{0, 0, 0, 0};
     }
+  constexpr bool PAIR = PX || PY;
+  static_assert(!PAIR || (U == 2 && sizeof(S2) == 8), "pairs: two steps per group, complex64");
   struct Group {
     S2 x[U][TI], y[U][TJ];
   };
   struct KOff {
     int64_t x[U], y[U];
   };
-  constexpr int CK = 4 * WK * U;             // k range of one group over the WK waves
-  const int64_t kb = k_lo + 4 * wk + g;      // this lane's first k
+  constexpr int CK = 4 * WK * U;                               // k range of one group over the WK waves
+  constexpr int KU = PAIR ? 1 : 4 * WK;                        // k distance of a lane's steps
+  const int64_t kb = k_lo + (PAIR ? 8 * wk + 2 * g : 4 * wk + g);  // this lane's first k
   const int64_t k_last = k_hi - 1;
   auto offs = [&](int64_t c, KOff& o) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const int64_t k = min(c * CK + u * 4 * WK + kb, k_last);
-      o.x[u] = kX[k];
-      o.y[u] = kY[k];
+      const int64_t k = c * CK + u * KU + kb;
+      // a pair ends at the last entry: past it the second of the two is the
+      // one wanted (tail)
+      if (!PX || u == 0) o.x[u] = kX[min(k, PX ? k_last - 1 : k_last)];
+      if (!PY || u == 0) o.y[u] = kY[min(k, PY ? k_last - 1 : k_last)];
       // opaque: otherwise every (block, step) address of the affine form
       // becomes a 64-bit induction variable of its own, 80 registers more
       // and half the resident waves
-      if constexpr (AFF) asm("" : "+v"(o.x[u]), "+v"(o.y[u]));
+      if constexpr (AFF) {
+        if (!PX || u == 0) asm("" : "+v"(o.x[u]));
+        if (!PY || u == 0) asm("" : "+v"(o.y[u]));
+      }
     }
   };
+  auto load2 = [](const S2* q, S2& e0, S2& e1) {
+    const f4pair v = *reinterpret_cast<const f4pair*>(q);
+    e0.x = v[0];
+    e0.y = v[1];
+    e1.x = v[2];
+    e1.y = v[3];
+  };
   auto load = [&](const KOff& o, Group& f) {
+    if constexpr (PX) {
+#pragma unroll
+      for (int a = 0; a < TI; ++a) load2(px[a] + o.x[0], f.x[0][a], f.x[U - 1][a]);
+    }
+    if constexpr (PY) {
+#pragma unroll
+      for (int b = 0; b < TJ; ++b) load2(py[b] + o.y[0], f.y[0][b], f.y[U - 1][b]);
+    }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
+      if constexpr (!PX) {
 #pragma unroll
-      for (int a = 0; a < TI; ++a) f.x[u][a] = px[a][o.x[u]];
+        for (int a = 0; a < TI; ++a) f.x[u][a] = px[a][o.x[u]];
+      }
+      if constexpr (!PY) {
 #pragma unroll
-      for (int b = 0; b < TJ; ++b) f.y[u][b] = py[b][o.y[u]];
+        for (int b = 0; b < TJ; ++b) f.y[u][b] = py[b][o.y[u]];
+      }
     }
   };
   const R sx = conjX ? (R)-1 : (R)1, sy = conjY ? (R)-1 : (R)1;
   auto mul = [&](int64_t c, const Group& f, bool tail) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      const bool in = !tail || c * CK + u * 4 * WK + kb < k_hi;
+      const int64_t k = c * CK + u * KU + kb;
+      const bool in = !tail || k < k_hi;
+      const bool second = PAIR && tail && u == 0 && k == k_last;  // the pair loaded was (k - 1, k)
       R xr[TI], xi[TI], yr[TJ], yi[TJ];
 #pragma unroll
       for (int a = 0; a < TI; ++a) {
-        xr[a] = in ? (R)f.x[u][a].x : (R)0;
-        xi[a] = in ? sx * (R)f.x[u][a].y : (R)0;
+        const S2 v = PX && second ? f.x[U - 1][a] : f.x[u][a];
+        xr[a] = in ? (R)v.x : (R)0;
+        xi[a] = in ? sx * (R)v.y : (R)0;
       }
 #pragma unroll
       for (int b = 0; b < TJ; ++b) {
-        yr[b] = in ? (R)f.y[u][b].x : (R)0;
-        yi[b] = in ? sy * (R)f.y[u][b].y : (R)0;
+        const S2 v = PY && second ? f.y[U - 1][b] : f.y[u][b];
+        yr[b] = in ? (R)v.x : (R)0;
+        yi[b] = in ? sy * (R)v.y : (R)0;
       }
 #pragma unroll
       for (int a = 0; a < TI; ++a)

@@ -42,8 +42,10 @@ struct GemmForm {
   int j_is_m = 1;
   int order = 0;   // one-thread-per-element kernel: fastest class (0: m, 1: n, 2: batch)
   int affine = 0;
+  bool pair_a = false, pair_b = false;  // the operand's K entries come in adjacent pairs (k_pairs)
   int64_t st[9] = {};
 };
+bool k_pairs(const std::vector<int64_t>& t);
 // v: the nine tables (rowA, kA, bA, kB, colB, bB, rowC, colC, bC)
 void gemm_form(const std::vector<int64_t> v[9], int64_t M, int64_t N, int64_t K, int64_t batch, int dtype, int prec,
                GemmForm* f);
@@ -79,16 +81,16 @@ constexpr int64_t SMALLK_ELEMS = 4096;
 struct GroupedProblem {
   GemmTables t;
   int64_t M, N, K, batch;
-  int32_t a_mfast, b_nfast;
   int32_t conjA, conjB;     // conjugate operand A / B
   int32_t shape;            // GROUPED_TILE_* / GROUPED_SMALLK
   int32_t kchunks;          // K chunks per tile (1: no split)
   int32_t order;            // GROUPED_SMALLK: fastest index class (0: m, 1: n, 2: batch), C's unit-stride one
+  int32_t j_is_m;           // tiles: the lanes run along m (C adjacent along m), else along n
+  int32_t pairs;            // bit 0 / 1: A's / B's K entries come in adjacent pairs (k_pairs)
   int32_t pad0;
   int64_t tiles_m, tiles_n;
   int64_t kc;               // chunk length (multiple of 16)
   int64_t part_base;        // first partial element (complex) of this problem
-  int64_t ctr_base;         // first tile arrival counter of this problem
 };
 struct GroupedUnit {
   int32_t prob;
@@ -101,7 +103,9 @@ struct GroupedLaunch {
   int64_t nunits;
   const uint64_t* ptrs;
   void* partials;
-  uint32_t* counters;  // [0] queue head, [64 + i] tile arrival counters
+  const GroupedUnit* split;  // tiles with K chunks (their sums follow in a second launch)
+  int64_t nsplit;
+  uint32_t* queue;  // next unit; zero between launches
   int64_t grid;
   int dtype, prec;
 };

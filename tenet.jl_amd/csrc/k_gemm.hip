@@ -4,326 +4,18 @@
 //   C[m, n, z] = sum_k A[m, k, z] * B[k, n, z].
 // The permutation that matricisation needs is never materialised: the host
 // planner turns every label class into a table of element offsets
-// (rowA[m], kA[k], bA[z], ...), and the tile loaders below gather straight
-// from the caller's strided tensors into LDS ("permute-into-LDS").  Complex
-// products run as four real MFMA products (no 3M trick: it cancels badly at
-// the 1e-8 accuracy this path is held to).
-//
-// Tiles: 64x64 output per 256-thread workgroup, four waves each owning a
-// 32x32 quadrant made of 2x2 16x16 MFMA blocks, K step 16.
-//   FP64: v_mfma_f64_16x16x4_f64      FP32: v_mfma_f32_16x16x4_f32
-// MFMA 16x16x4 operand layout (lane l): A[i = l%16][k = l/16],
-// B[k = l/16][j = l%16]; result register r of lane l holds D[i][j = l%16]
-// with i = 4*(l/16) + r for FP32 and i = 4*r + l/16 for FP64.
+// (rowA[m], kA[k], bA[z], ...), and the kernels gather straight from the
+// caller's strided tensors (gemm_direct.h).  Complex products run as four
+// real MFMA products (no 3M trick: it cancels badly at the 1e-8 accuracy this
+// path is held to).
 #include "../../include/tenet_hip.h"
 #include "internal.h"
 #include "gemm_direct.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace tenet {
-
-constexpr int BK = 16, PADK = 4;
-
-// Tile variants.  A workgroup of four waves computes one BM x BN output tile;
-// the waves form a WGM x WGN grid over the tile and, when WGK > 1, also split
-// each K step of 16 (k sub-steps of 4 taken round robin) with an LDS
-// reduction at the end.  Each wave owns TM x TN MFMA blocks of 16 x 16.
-template <int BM_, int BN_, int WGM_, int WGN_, int WGK_>
-struct TileCfg {
-  static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, WGK = WGK_;
-  static constexpr int TM = BM / (16 * WGM), TN = BN / (16 * WGN);
-  static constexpr int NA = BM * BK / 256, NB = BN * BK / 256;  // loads per thread
-  static_assert(WGM * WGN * WGK == 4, "four waves");
-  static_assert(TM >= 1 && TN >= 1 && NA >= 1 && NB >= 1, "tile too small");
-};
-using Tile64 = TileCfg<64, 64, 2, 2, 1>;
-using Tile32 = TileCfg<32, 32, 2, 2, 1>;
-using Tile16 = TileCfg<16, 16, 1, 1, 4>;
-
-template <typename R>
-struct GemmSmem {
-  R ar[BK][64 + PADK];
-  R ai[BK][64 + PADK];
-  R br[BK][64 + PADK];
-  R bi[BK][64 + PADK];
-};
-
-struct TileView {
-  const void* A;
-  const void* B;
-  void* C;
-  GemmTables t;
-  int64_t M, N, K;
-  int a_mfast, b_nfast, conjA, conjB;
-  double alpha_re, alpha_im, beta_re, beta_im;
-};
-
-template <typename R, typename Cfg>
-struct TileAcc {
-  using V4 = typename Acc4<R>::T;
-  V4 r[Cfg::TM][Cfg::TN], i[Cfg::TM][Cfg::TN];
-};
-
-// Accumulate the (tm, tn) tile of batch entry z over k in [k_lo, k_hi).
-// On return every wave holds its TM x TN blocks; for WGK > 1 the sum over
-// the K-splitting waves has been folded into wave 0 (the others hold zeros).
-// CONJ = false: the operands are never conjugated (p.conjA / p.conjB are
-// not read), so the loads carry no per-element sign select.
-template <typename S2, typename R, typename Cfg, bool CONJ = true>
-__device__ __forceinline__ void gemm_accumulate(const TileView& p, int64_t tm, int64_t tn, int64_t z, int64_t k_lo,
-                                                int64_t k_hi, GemmSmem<R>& sm, TileAcc<R, Cfg>& acc) {
-  const bool conjA = CONJ && p.conjA, conjB = CONJ && p.conjB;
-  constexpr int BM = Cfg::BM, BN = Cfg::BN, NA = Cfg::NA, NB = Cfg::NB;
-  const S2* __restrict__ A = static_cast<const S2*>(p.A);
-  const S2* __restrict__ B = static_cast<const S2*>(p.B);
-  const int tid = threadIdx.x;
-  const int lane = tid & 63;
-  const int wave = tid >> 6;
-  const int wk = wave % Cfg::WGK;
-  const int wmn = wave / Cfg::WGK;
-  const int wm = wmn % Cfg::WGM, wn = wmn / Cfg::WGM;
-  const int64_t m0 = tm * BM, n0 = tn * BN;
-  const int64_t M = p.M, N = p.N;
-  const int64_t offAz = p.t.bA[z], offBz = p.t.bB[z];
-
-  // Per-thread loader coordinates.  The dimension a thread keeps fixed over
-  // the K loop has its table offset cached in registers.
-  int la_m[NA], la_k[NA], lb_n[NB], lb_k[NB];
-  int64_t la_fixed[NA], lb_fixed[NB];
-  bool la_ok[NA], lb_ok[NB];
-#pragma unroll
-  for (int j = 0; j < NA; ++j) {
-    if (p.a_mfast) {
-      la_m[j] = tid % BM;
-      la_k[j] = tid / BM + (256 / BM) * j;
-    } else {
-      la_m[j] = (tid >> 4) + 16 * j;
-      la_k[j] = tid & 15;
-    }
-    const int64_t gm = m0 + la_m[j];
-    la_ok[j] = gm < M;
-    la_fixed[j] = la_ok[j] ? p.t.rowA[gm] + offAz : 0;
-  }
-#pragma unroll
-  for (int j = 0; j < NB; ++j) {
-    if (p.b_nfast) {
-      lb_n[j] = tid % BN;
-      lb_k[j] = tid / BN + (256 / BN) * j;
-    } else {
-      lb_n[j] = (tid >> 4) + 16 * j;
-      lb_k[j] = tid & 15;
-    }
-    const int64_t gn = n0 + lb_n[j];
-    lb_ok[j] = gn < N;
-    lb_fixed[j] = lb_ok[j] ? p.t.colB[gn] + offBz : 0;
-  }
-
-  R ra_r[NA], ra_i[NA], rb_r[NB], rb_i[NB];
-  auto gload = [&](int64_t k0) {
-#pragma unroll
-    for (int j = 0; j < NA; ++j) {
-      const int64_t gka = k0 + la_k[j];
-      if (la_ok[j] && gka < k_hi) {
-        const S2 v = A[la_fixed[j] + p.t.kA[gka]];
-        ra_r[j] = (R)v.x;
-        ra_i[j] = conjA ? -(R)v.y : (R)v.y;
-      } else {
-        ra_r[j] = 0;
-        ra_i[j] = 0;
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      const int64_t gkb = k0 + lb_k[j];
-      if (lb_ok[j] && gkb < k_hi) {
-        const S2 v = B[lb_fixed[j] + p.t.kB[gkb]];
-        rb_r[j] = (R)v.x;
-        rb_i[j] = conjB ? -(R)v.y : (R)v.y;
-      } else {
-        rb_r[j] = 0;
-        rb_i[j] = 0;
-      }
-    }
-  };
-  auto sstore = [&]() {
-#pragma unroll
-    for (int j = 0; j < NA; ++j) {
-      sm.ar[la_k[j]][la_m[j]] = ra_r[j];
-      sm.ai[la_k[j]][la_m[j]] = ra_i[j];
-    }
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      sm.br[lb_k[j]][lb_n[j]] = rb_r[j];
-      sm.bi[lb_k[j]][lb_n[j]] = rb_i[j];
-    }
-  };
-
-#pragma unroll
-  for (int i = 0; i < Cfg::TM; ++i)
-#pragma unroll
-    for (int j = 0; j < Cfg::TN; ++j) {
-      acc.r[i][j] = typename TileAcc<R, Cfg>::V4{0, 0, 0, 0};
-      acc.i[i][j] = typename TileAcc<R, Cfg>::V4{0, 0, 0, 0};
-    }
-
-  gload(k_lo);
-  __syncthreads();  // previous tile's readers are done with the LDS buffers
-  sstore();
-  __syncthreads();
-  for (int64_t k0 = k_lo; k0 < k_hi; k0 += BK) {
-    const bool more = (k0 + BK) < k_hi;
-    if (more) gload(k0 + BK);
-#pragma unroll
-    for (int kk = 0; kk < BK / 4; ++kk) {
-      if (kk % Cfg::WGK != wk) continue;
-      const int kr = kk * 4 + (lane >> 4);
-      R xr[Cfg::TM], xi[Cfg::TM], yr[Cfg::TN], yi[Cfg::TN];
-#pragma unroll
-      for (int i = 0; i < Cfg::TM; ++i) {
-        xr[i] = sm.ar[kr][(wm * Cfg::TM + i) * 16 + (lane & 15)];
-        xi[i] = sm.ai[kr][(wm * Cfg::TM + i) * 16 + (lane & 15)];
-      }
-#pragma unroll
-      for (int j = 0; j < Cfg::TN; ++j) {
-        yr[j] = sm.br[kr][(wn * Cfg::TN + j) * 16 + (lane & 15)];
-        yi[j] = sm.bi[kr][(wn * Cfg::TN + j) * 16 + (lane & 15)];
-      }
-#pragma unroll
-      for (int i = 0; i < Cfg::TM; ++i)
-#pragma unroll
-        for (int j = 0; j < Cfg::TN; ++j) {
-          acc.r[i][j] = mfma16x16x4(xr[i], yr[j], acc.r[i][j]);
-          acc.r[i][j] = mfma16x16x4(-xi[i], yi[j], acc.r[i][j]);
-          acc.i[i][j] = mfma16x16x4(xr[i], yi[j], acc.i[i][j]);
-          acc.i[i][j] = mfma16x16x4(xi[i], yr[j], acc.i[i][j]);
-        }
-    }
-    __syncthreads();
-    if (more) {
-      sstore();
-      __syncthreads();
-    }
-  }
-
-  if constexpr (Cfg::WGK > 1) {
-    // fold the K-splitting waves into wave 0 in a fixed order (deterministic);
-    // the LDS operand buffers are free after the loop's final barrier
-    static_assert(Cfg::TM == 1 && Cfg::TN == 1, "K-split tiles hold one block per wave");
-    R* red = &sm.ar[0][0];  // (WGK - 1) * 8 * 64 values <= the 4 operand planes
-    if (wave > 0) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        red[((wave - 1) * 8 + r) * 64 + lane] = acc.r[0][0][r];
-        red[((wave - 1) * 8 + 4 + r) * 64 + lane] = acc.i[0][0][r];
-        acc.r[0][0][r] = 0;
-        acc.i[0][0][r] = 0;
-      }
-    }
-    __syncthreads();
-    if (wave == 0) {
-      for (int w = 1; w < Cfg::WGK; ++w)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          acc.r[0][0][r] += red[((w - 1) * 8 + r) * 64 + lane];
-          acc.i[0][0][r] += red[((w - 1) * 8 + 4 + r) * 64 + lane];
-        }
-    }
-    __syncthreads();
-  }
-}
-
-// Does this wave hold final accumulators (all waves, or wave 0 of a K-split tile)?
-template <typename Cfg>
-__device__ __forceinline__ bool holds_result() {
-  return Cfg::WGK == 1 || (threadIdx.x >> 6) == 0;
-}
-
-// Epilogue: C = alpha * acc + beta * C, scattered through the C tables.
-template <typename S2, typename R, typename Cfg>
-__device__ __forceinline__ void gemm_store(const TileView& p, int64_t tm, int64_t tn, int64_t z,
-                                           const TileAcc<R, Cfg>& acc) {
-  if (!holds_result<Cfg>()) return;
-  S2* __restrict__ C = static_cast<S2*>(p.C);
-  const int lane = threadIdx.x & 63;
-  const int wmn = (threadIdx.x >> 6) / Cfg::WGK;
-  const int wm = wmn % Cfg::WGM, wn = wmn / Cfg::WGM;
-  const int64_t m0 = tm * Cfg::BM, n0 = tn * Cfg::BN;
-  const int64_t offCz = p.t.bC[z];
-  const double ar = p.alpha_re, ai = p.alpha_im, br = p.beta_re, bi = p.beta_im;
-  const bool use_beta = (br != 0.0 || bi != 0.0);
-#pragma unroll
-  for (int j = 0; j < Cfg::TN; ++j) {
-    const int64_t col = n0 + (wn * Cfg::TN + j) * 16 + (lane & 15);
-    if (col >= p.N) continue;
-    const int64_t ccol = p.t.colC[col] + offCz;
-#pragma unroll
-    for (int i = 0; i < Cfg::TM; ++i) {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        // D layout: FP32 16x16x4 keeps rows 4*(l/16)+r in lane l; FP64
-        // 16x16x4 interleaves them as rows 4*r + l/16.
-        const int rr = (sizeof(R) == 8) ? (r * 4 + (lane >> 4)) : ((lane >> 4) * 4 + r);
-        const int64_t row = m0 + (wm * Cfg::TM + i) * 16 + rr;
-        if (row >= p.M) continue;
-        const int64_t off = p.t.rowC[row] + ccol;
-        const double cr = (double)acc.r[i][j][r], ci = (double)acc.i[i][j][r];
-        double outr = ar * cr - ai * ci;
-        double outi = ar * ci + ai * cr;
-        if (use_beta) {
-          const S2 old = C[off];
-          outr += br * (double)old.x - bi * (double)old.y;
-          outi += br * (double)old.y + bi * (double)old.x;
-        }
-        S2 o;
-        o.x = outr;
-        o.y = outi;
-        C[off] = o;
-      }
-    }
-  }
-}
-
-// Split-K partials: a result-holding thread stores its registers at
-// ((wave * TM + i) * TN + j) * 4 + r) * 64 + lane, as (re, im) pairs; the
-// same thread of the reducing workgroup reads them back from the same places.
-template <typename R, typename Cfg>
-__device__ __forceinline__ void partial_store(R* __restrict__ part, const TileAcc<R, Cfg>& acc) {
-  if (!holds_result<Cfg>()) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int i = 0; i < Cfg::TM; ++i)
-#pragma unroll
-    for (int j = 0; j < Cfg::TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t e = ((((int64_t)wave * Cfg::TM + i) * Cfg::TN + j) * 4 + r) * 64 + lane;
-        part[2 * e] = acc.r[i][j][r];
-        part[2 * e + 1] = acc.i[i][j][r];
-      }
-}
-
-template <typename R, typename Cfg>
-__device__ __forceinline__ void partial_sum(const R* __restrict__ part, int nchunks, TileAcc<R, Cfg>& acc) {
-  if (!holds_result<Cfg>()) return;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  constexpr int64_t TILE = (int64_t)Cfg::BM * Cfg::BN;
-#pragma unroll
-  for (int i = 0; i < Cfg::TM; ++i)
-#pragma unroll
-    for (int j = 0; j < Cfg::TN; ++j)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int64_t e = ((((int64_t)wave * Cfg::TM + i) * Cfg::TN + j) * 4 + r) * 64 + lane;
-        R sr = 0, si = 0;
-        for (int c = 0; c < nchunks; ++c) {  // fixed order: deterministic
-          sr += part[2 * (c * TILE + e)];
-          si += part[2 * (c * TILE + e) + 1];
-        }
-        acc.r[i][j][r] = sr;
-        acc.i[i][j][r] = si;
-      }
-}
 
 // ---- one contraction per launch -----------------------------------------------
 // Workgroup shapes of the direct kernel: four waves, either all on the same
@@ -361,7 +53,7 @@ __device__ __forceinline__ int64_t xcd_remap(int64_t pid, int64_t total) {
   return (pid % NXCD) * (total / NXCD) + pid / NXCD;
 }
 
-template <typename S2, typename R, int TI, int TJ, int WJ, int WK, int U, bool AFF>
+template <typename S2, typename R, int TI, int TJ, int WJ, int WK, int U, bool AFF, bool PX, bool PY>
 __global__ __launch_bounds__(256, 2) void gemm_direct_kernel(DirectArgs p) {
   static_assert(WJ * WK == 4, "four waves");
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -375,7 +67,7 @@ __global__ __launch_bounds__(256, 2) void gemm_direct_kernel(DirectArgs p) {
   const S2* X = static_cast<const S2*>(p.X) + off(2)[z];
   const S2* Y = static_cast<const S2*>(p.Y) + off(5)[z];
   BlockAcc<R, TI, TJ> acc;
-  direct_accumulate<S2, R, TI, TJ, WK, U, AFF>(X, Y, off(0), off(1), off(3), off(4), i0, p.I, j0, p.J, 0, p.K, wk,
+  direct_accumulate<S2, R, TI, TJ, WK, U, AFF, PX, PY>(X, Y, off(0), off(1), off(3), off(4), i0, p.I, j0, p.J, 0, p.K, wk,
                                                p.conjX != 0, p.conjY != 0, acc);
   if constexpr (WK > 1) {
     __shared__ R red[WK / 2 * TI * TJ * 512];
@@ -417,7 +109,8 @@ __global__ __launch_bounds__(256) void gemm_elements_kernel(GemmTables t, const 
 // The workgroup shape with the least modelled time, in cycles of one CU: per
 // K step the larger of its MFMAs (64 cycles each in FP64, 32 in FP32) and
 // its operand loads (24 cycles of the CU's address unit per wave and block,
-// twice that where 16 lanes read 16 rows instead of neighbours), over the
+// twice that where 16 lanes read 16 rows instead of neighbours, one entry
+// each), over the
 // rounds the 256 CUs need, plus the epilogue of a tile.  On 45 measured shapes
 // (K 4..3840, 24 x 38 to 590000 x 20, both types) the choice is 2% slower than
 // the best of the six in the mean, 26% at worst (complex64 300 x 600 x 300,
@@ -443,6 +136,16 @@ static int choose_direct(double cyc, int64_t I, int64_t J, int64_t K, int64_t ba
   return best;
 }
 
+// every entry pair (2 i, 2 i + 1) of a K table adjacent, and, with an odd
+// length, the last two as well
+bool k_pairs(const std::vector<int64_t>& t) {
+  const size_t n = t.size();
+  if (n < 2) return false;
+  for (size_t k = 0; k + 1 < n; k += 2)
+    if (t[k + 1] != t[k] + 1) return false;
+  return n % 2 == 0 || t[n - 1] == t[n - 2] + 1;
+}
+
 void gemm_form(const std::vector<int64_t> v[9], int64_t M, int64_t N, int64_t K, int64_t batch, int dtype, int prec,
                GemmForm* f) {
   auto stride_of = [](const std::vector<int64_t>& t, int64_t* st) {
@@ -466,12 +169,26 @@ void gemm_form(const std::vector<int64_t> v[9], int64_t M, int64_t N, int64_t K,
     f->cfg = ELEMENTS;
     return;
   }
-  const bool a_adj = gap(0) == 1 || M == 1, b_adj = gap(4) == 1 || N == 1;
+  f->pair_a = k_pairs(v[1]);
+  f->pair_b = k_pairs(v[3]);
+  const bool wide = dtype == TENET_C64;  // pairs of entries per load
+  const bool a_adj = gap(0) == 1 || M == 1 || (wide && f->pair_a);
+  const bool b_adj = gap(4) == 1 || N == 1 || (wide && f->pair_b);
   const double cyc = dtype == TENET_C128 && prec == TENET_PREC_NATIVE ? 64 : 32;
   if (f->j_is_m)
     f->cfg = choose_direct(cyc, N, M, K, batch, b_adj, a_adj);
   else
     f->cfg = choose_direct(cyc, M, N, K, batch, a_adj, b_adj);
+}
+
+template <typename S2, typename R, int TI, int TJ, int WJ, int WK, int U, bool PX, bool PY>
+static int launch_direct_p(const DirectArgs& p, bool affine, unsigned total, hipStream_t s) {
+  if (affine)
+    hipLaunchKernelGGL((gemm_direct_kernel<S2, R, TI, TJ, WJ, WK, U, true, PX, PY>), dim3(total), dim3(256), 0, s, p);
+  else
+    hipLaunchKernelGGL((gemm_direct_kernel<S2, R, TI, TJ, WJ, WK, U, false, PX, PY>), dim3(total), dim3(256), 0, s, p);
+  TENET_HIP_CHECK(hipGetLastError());
+  return TENET_OK;
 }
 
 template <typename S2, typename R, int TI, int TJ, int WJ, int WK, int U>
@@ -483,14 +200,16 @@ static int launch_direct(DirectArgs& p, const GemmLaunch& g, hipStream_t s) {
     set_error("contraction too large for one launch");
     return TENET_ERR_UNSUPPORTED;
   }
-  if (g.form->affine)
-    hipLaunchKernelGGL((gemm_direct_kernel<S2, R, TI, TJ, WJ, WK, U, true>), dim3((unsigned)total), dim3(256), 0, s,
-                       p);
-  else
-    hipLaunchKernelGGL((gemm_direct_kernel<S2, R, TI, TJ, WJ, WK, U, false>), dim3((unsigned)total), dim3(256), 0, s,
-                       p);
-  TENET_HIP_CHECK(hipGetLastError());
-  return TENET_OK;
+  const bool aff = g.form->affine != 0;
+  const unsigned n = (unsigned)total;
+  if constexpr (sizeof(S2) == 8) {
+    const bool px = g.form->j_is_m ? g.form->pair_b : g.form->pair_a;
+    const bool py = g.form->j_is_m ? g.form->pair_a : g.form->pair_b;
+    if (px && py) return launch_direct_p<S2, R, TI, TJ, WJ, WK, 2, true, true>(p, aff, n, s);
+    if (px) return launch_direct_p<S2, R, TI, TJ, WJ, WK, 2, true, false>(p, aff, n, s);
+    if (py) return launch_direct_p<S2, R, TI, TJ, WJ, WK, 2, false, true>(p, aff, n, s);
+  }
+  return launch_direct_p<S2, R, TI, TJ, WJ, WK, U, false, false>(p, aff, n, s);
 }
 
 template <typename S2, typename R, typename IT>
@@ -589,66 +308,163 @@ int launch_gemm_c64(const GemmLaunch& g, int prec, hipStream_t s, void* ws, size
 // Work units (problem, tile, K chunk) are sorted by decreasing cost on the
 // host; persistent workgroups take the next unit from a device counter, so
 // the largest units start first and the tail is short (LPT order).  A tile
-// whose K range is cut into chunks stores each chunk's partial tile; the
-// workgroup that finishes a tile's last chunk (per-tile arrival counter) sums
-// the partials in chunk order and writes C, so results do not depend on the
-// schedule.
+// whose K range is cut into chunks stores each chunk's partial tile, and a
+// second kernel sums them in chunk order and writes C, so results do not
+// depend on the schedule.
+//
+// A unit's workgroup shape: TI x TJ blocks per wave, the four waves in a
+// W x W arrangement over the tile (WK = 1) or all on one tile, dealing its K
+// steps (WK = 4).
+template <int TI_, int TJ_, int W_, int WK_>
+struct UnitCfg {
+  static constexpr int TI = TI_, TJ = TJ_, W = W_, WK = WK_, EDGE = 16 * TI * W;
+  static_assert(TI == TJ && W * W * WK == 4, "square tiles, four waves");
+};
+using Tile64 = UnitCfg<2, 2, 2, 1>;
+using Tile32 = UnitCfg<2, 2, 1, 4>;
+using Tile16 = UnitCfg<1, 1, 1, 4>;
+// LDS values of the K-split fold (WK / 2 * TI * TJ * 512), with the slack that
+// puts the queue word behind them at 17408 / 34816 bytes, the offset the
+// kernel's generated code is checked for
+constexpr int FOLD_VALUES = 4352;
+static_assert(FOLD_VALUES >= 4 / 2 * 2 * 2 * 512, "fold buffer");
+
+// Split-K partials: a result-holding thread stores its registers at
+// ((wave * TI + i) * TJ + j) * 4 + r) * 64 + lane, as (re, im) pairs
+// (grouped_reduce_kernel reads them back).
+template <typename R, typename Cfg>
+__device__ __forceinline__ void partial_store(R* __restrict__ part, int wave,
+                                              const BlockAcc<R, Cfg::TI, Cfg::TJ>& acc) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int i = 0; i < Cfg::TI; ++i)
+#pragma unroll
+    for (int j = 0; j < Cfg::TJ; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int64_t e = ((((int64_t)wave * Cfg::TI + i) * Cfg::TJ + j) * 4 + r) * 64 + lane;
+        part[2 * e] = acc.r[i][j][r];
+        part[2 * e + 1] = acc.i[i][j][r];
+      }
+}
+
 template <typename S2, typename R, typename Cfg>
 __device__ __forceinline__ void grouped_unit(const GroupedProblem& q, const uint64_t* __restrict__ ptrs,
-                                             const GroupedUnit& u, R* __restrict__ partials,
-                                             uint32_t* __restrict__ tile_ctr, GemmSmem<R>& sm, int* bcast) {
-  TileView p;
-  p.A = (const void*)ptrs[3 * u.prob];
-  p.B = (const void*)ptrs[3 * u.prob + 1];
-  p.C = (void*)ptrs[3 * u.prob + 2];
-  p.t = q.t;
-  p.M = q.M;
-  p.N = q.N;
-  p.K = q.K;
-  p.a_mfast = q.a_mfast;
-  p.b_nfast = q.b_nfast;
-  p.conjA = q.conjA;
-  p.conjB = q.conjB;
-  p.alpha_re = 1.0;
-  p.alpha_im = 0.0;
-  p.beta_re = 0.0;
-  p.beta_im = 0.0;
+                                             const GroupedUnit& u, R* __restrict__ partials, R* __restrict__ red) {
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wk = Cfg::WK == 1 ? 0 : wave, wi = Cfg::WK == 1 ? wave % Cfg::W : 0, wj = Cfg::WK == 1 ? wave / Cfg::W : 0;
+  const bool holds = wk == 0;  // this wave ends with results
   const int64_t per_batch = (int64_t)q.tiles_m * q.tiles_n;
   const int64_t z = u.tile / per_batch;
   const int64_t t = u.tile - z * per_batch;
   const int64_t tm = t % q.tiles_m, tn = t / q.tiles_m;
   const int64_t k_lo = (int64_t)u.chunk * q.kc;
   const int64_t k_hi = std::min<int64_t>(q.K, k_lo + q.kc);
-  TileAcc<R, Cfg> acc;
-  if (q.conjA || q.conjB)
-    gemm_accumulate<S2, R, Cfg, true>(p, tm, tn, z, k_lo, k_hi, sm, acc);
-  else
-    gemm_accumulate<S2, R, Cfg, false>(p, tm, tn, z, k_lo, k_hi, sm, acc);
-  if (q.kchunks == 1) {
-    gemm_store<S2, R, Cfg>(p, tm, tn, z, acc);
+  // i and j are A's and B's free indices, or B's and A's when C's entries are
+  // adjacent along m
+  const bool jm = q.j_is_m != 0;
+  const S2* A = reinterpret_cast<const S2*>(ptrs[3 * u.prob]) + q.t.bA[z];
+  const S2* B = reinterpret_cast<const S2*>(ptrs[3 * u.prob + 1]) + q.t.bB[z];
+  S2* C = reinterpret_cast<S2*>(ptrs[3 * u.prob + 2]) + q.t.bC[z];
+  using Off = Offsets<false>;
+  const int64_t I = jm ? q.N : q.M, J = jm ? q.M : q.N;
+  const int64_t i0 = (jm ? tn : tm) * Cfg::EDGE + wi * 16 * Cfg::TI, j0 = (jm ? tm : tn) * Cfg::EDGE + wj * 16 * Cfg::TJ;
+  BlockAcc<R, Cfg::TI, Cfg::TJ> acc;
+  const Off rowX{jm ? q.t.colB : q.t.rowA, 0}, kX{jm ? q.t.kB : q.t.kA, 0};
+  const Off rowY{jm ? q.t.rowA : q.t.colB, 0}, kY{jm ? q.t.kA : q.t.kB, 0};
+  const bool cx = (jm ? q.conjB : q.conjA) != 0, cy = (jm ? q.conjA : q.conjB) != 0;
+  auto accumulate = [&](auto px, auto py) {
+    constexpr int U = decltype(px)::value || decltype(py)::value ? 2 : 1;
+    direct_accumulate<S2, R, Cfg::TI, Cfg::TJ, Cfg::WK, U, false, decltype(px)::value, decltype(py)::value>(
+        jm ? B : A, jm ? A : B, rowX, kX, rowY, kY, i0, I, j0, J, k_lo, k_hi, wk, cx, cy, acc);
+  };
+  using No = std::integral_constant<bool, false>;
+  using Yes = std::integral_constant<bool, true>;
+  if constexpr (sizeof(S2) == 8) {
+    // bit 0: A's K entries come in adjacent pairs, bit 1: B's
+    const int pairs = jm ? ((q.pairs & 1) << 1 | q.pairs >> 1) : q.pairs;
+    switch (pairs) {
+      case 1:
+        accumulate(Yes{}, No{});
+        break;
+      case 2:
+        accumulate(No{}, Yes{});
+        break;
+      case 3:
+        accumulate(Yes{}, Yes{});
+        break;
+      default:
+        accumulate(No{}, No{});
+        break;
+    }
   } else {
-    constexpr int64_t TILE = (int64_t)Cfg::BM * Cfg::BN;
-    R* part = partials + 2 * (q.part_base + u.tile * q.kchunks * TILE);
-    partial_store<R, Cfg>(part + 2 * (int64_t)u.chunk * TILE, acc);
-    __threadfence();  // release this thread's partial stores at device scope
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const uint32_t prev = __hip_atomic_fetch_add(&tile_ctr[q.ctr_base + u.tile], 1u, __ATOMIC_ACQ_REL,
-                                                   __HIP_MEMORY_SCOPE_AGENT);
-      *bcast = (prev + 1 == (uint32_t)q.kchunks) ? 1 : 0;
-    }
-    __syncthreads();
-    // wave-uniform by construction (one LDS word after a barrier); readfirstlane
-    // lets the compiler branch on it with scalar control flow
-    const int last = __builtin_amdgcn_readfirstlane(*bcast);
-    __syncthreads();  // bcast is reused by the next unit
-    if (last) {
-      __threadfence();  // acquire the other chunks' partials
-      partial_sum<R, Cfg>(part, q.kchunks, acc);
-      gemm_store<S2, R, Cfg>(p, tm, tn, z, acc);
-      if (threadIdx.x == 0) tile_ctr[q.ctr_base + u.tile] = 0u;  // ready for the next launch
-    }
+    accumulate(No{}, No{});
   }
+  if constexpr (Cfg::WK > 1) direct_fold<R, Cfg::TI, Cfg::TJ, Cfg::WK>(red, wk, acc);
+  const Off rowC{jm ? q.t.colC : q.t.rowC, 0}, colC{jm ? q.t.rowC : q.t.colC, 0};
+  const Scalars one{1.0, 0.0, 0.0, 0.0};
+  if (q.kchunks == 1) {
+    if (holds) direct_store<S2, R, Cfg::TI, Cfg::TJ, false>(C, rowC, colC, i0, I, j0, J, one, acc);
+  } else {
+    // chunks of K: partials through memory, summed by the kernel behind this
+    // one (inside it, every chunk's device-scope release and acquire wrote back
+    // and invalidated the XCD's L2: twice the chunks cost a 200-problem batch
+    // 718 -> 1648 us)
+    constexpr int64_t TILE = (int64_t)Cfg::EDGE * Cfg::EDGE;
+    R* part = partials + 2 * (q.part_base + u.tile * q.kchunks * TILE);
+    if (holds) partial_store<R, Cfg>(part + 2 * (int64_t)u.chunk * TILE, wave, acc);
+  }
+}
+
+// Sum the chunk partials of one split tile (blockIdx.x) in chunk order and
+// store C.
+template <typename S2, typename R, typename Cfg>
+__device__ __forceinline__ void reduce_tile(const GroupedProblem& q, S2* __restrict__ Call, const GroupedUnit& u,
+                                            const R* __restrict__ partials) {
+  constexpr int64_t TILE = (int64_t)Cfg::EDGE * Cfg::EDGE;
+  const int64_t per_batch = (int64_t)q.tiles_m * q.tiles_n;
+  const int64_t z = u.tile / per_batch;
+  const int64_t t = u.tile - z * per_batch;
+  const int64_t tm = t % q.tiles_m, tn = t / q.tiles_m;
+  const bool jm = q.j_is_m != 0;
+  const R* part = partials + 2 * (q.part_base + u.tile * q.kchunks * TILE);
+  S2* C = Call + q.t.bC[z];
+  for (int e = threadIdx.x; e < (int)TILE; e += 256) {
+    const int lane = e & 63, r = (e >> 6) & 3, blk = e >> 8;
+    const int j = blk % Cfg::TJ, i = (blk / Cfg::TJ) % Cfg::TI, wave = blk / (Cfg::TI * Cfg::TJ);
+    const int wi = wave % Cfg::W, wj = wave / Cfg::W;
+    const int rr = sizeof(R) == 8 ? r * 4 + (lane >> 4) : (lane >> 4) * 4 + r;
+    const int64_t gi = (jm ? tn : tm) * Cfg::EDGE + (wi * Cfg::TI + i) * 16 + rr;
+    const int64_t gj = (jm ? tm : tn) * Cfg::EDGE + (wj * Cfg::TJ + j) * 16 + (lane & 15);
+    const int64_t m = jm ? gj : gi, n = jm ? gi : gj;
+    if (m >= q.M || n >= q.N) continue;
+    R sr = 0, si = 0;
+#pragma unroll 8
+    for (int c = 0; c < q.kchunks; ++c) {  // fixed order: deterministic
+      sr += part[2 * (c * TILE + e)];
+      si += part[2 * (c * TILE + e) + 1];
+    }
+    S2 o;
+    o.x = sr;
+    o.y = si;
+    C[q.t.rowC[m] + q.t.colC[n]] = o;
+  }
+}
+
+template <typename S2, typename R>
+__global__ __launch_bounds__(256) void grouped_reduce_kernel(const GroupedProblem* __restrict__ probs,
+                                                             const GroupedUnit* __restrict__ tiles,
+                                                             const uint64_t* __restrict__ ptrs,
+                                                             const R* __restrict__ partials) {
+  const GroupedUnit u = tiles[blockIdx.x];
+  const GroupedProblem& q = probs[u.prob];
+  S2* C = reinterpret_cast<S2*>(ptrs[3 * u.prob + 2]);
+  if (q.shape == GROUPED_TILE_16)
+    reduce_tile<S2, R, Tile16>(q, C, u, partials);
+  else if (q.shape == GROUPED_TILE_32)
+    reduce_tile<S2, R, Tile32>(q, C, u, partials);
+  else
+    reduce_tile<S2, R, Tile64>(q, C, u, partials);
 }
 
 // A GROUPED_SMALLK unit: output elements [tile * SMALLK_ELEMS, +SMALLK_ELEMS)
@@ -723,12 +539,9 @@ template <typename S2, typename R>
 __device__ __forceinline__ void grouped_gemm_body(const GroupedProblem* __restrict__ probs,
                                                   const GroupedUnit* __restrict__ units, int64_t nunits,
                                                   const uint64_t* __restrict__ ptrs, R* __restrict__ partials,
-                                                  uint32_t* __restrict__ counters) {
-  __shared__ GemmSmem<R> sm;
+                                                  uint32_t* __restrict__ queue) {
+  __shared__ R red[FOLD_VALUES];
   __shared__ uint32_t next;
-  __shared__ int bcast;
-  uint32_t* queue = counters;          // counters[0]: next unit to take
-  uint32_t* tile_ctr = counters + 64;  // per split tile arrival counts
   // Every branch below depends only on values that are uniform across the
   // workgroup and are made scalar with readfirstlane, so the loop compiles to
   // scalar control flow: each iteration takes exactly one unit from the queue
@@ -745,7 +558,13 @@ __device__ __forceinline__ void grouped_gemm_body(const GroupedProblem* __restri
     __syncthreads();
     const int64_t ui = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)next);
     __syncthreads();
-    if (ui >= nunits) break;
+    if (ui >= nunits) {
+      // every workgroup fetches exactly one number past the units, so the
+      // largest comes after all other fetches: its taker readies the queue for
+      // the next launch
+      if (ui == nunits + (int64_t)gridDim.x - 1 && tid == 0) *queue = 0u;
+      break;
+    }
     const GroupedUnit u = units[ui];
     const GroupedProblem& q = probs[u.prob];
     switch (q.shape) {
@@ -753,33 +572,31 @@ __device__ __forceinline__ void grouped_gemm_body(const GroupedProblem* __restri
         grouped_smallk_unit<S2, R>(q, ptrs, u);
         break;
       case GROUPED_TILE_16:
-        grouped_unit<S2, R, Tile16>(q, ptrs, u, partials, tile_ctr, sm, &bcast);
+        grouped_unit<S2, R, Tile16>(q, ptrs, u, partials, red);
         break;
       case GROUPED_TILE_32:
-        grouped_unit<S2, R, Tile32>(q, ptrs, u, partials, tile_ctr, sm, &bcast);
+        grouped_unit<S2, R, Tile32>(q, ptrs, u, partials, red);
         break;
       default:
-        grouped_unit<S2, R, Tile64>(q, ptrs, u, partials, tile_ctr, sm, &bcast);
+        grouped_unit<S2, R, Tile64>(q, ptrs, u, partials, red);
         break;
     }
   }
 }
 
-// complex64: two resident workgroups per CU fit without spills; complex128
-// keeps one (its FP64 accumulators double the register need)
-__global__ __launch_bounds__(256, 2) void grouped_gemm_c64_kernel(const GroupedProblem* __restrict__ probs,
+__global__ __launch_bounds__(256, 3) void grouped_gemm_c64_kernel(const GroupedProblem* __restrict__ probs,
                                                                   const GroupedUnit* __restrict__ units,
                                                                   int64_t nunits, const uint64_t* __restrict__ ptrs,
                                                                   float* __restrict__ partials,
-                                                                  uint32_t* __restrict__ counters) {
-  grouped_gemm_body<float2, float>(probs, units, nunits, ptrs, partials, counters);
+                                                                  uint32_t* __restrict__ queue) {
+  grouped_gemm_body<float2, float>(probs, units, nunits, ptrs, partials, queue);
 }
-__global__ __launch_bounds__(256) void grouped_gemm_c128_kernel(const GroupedProblem* __restrict__ probs,
+__global__ __launch_bounds__(256, 2) void grouped_gemm_c128_kernel(const GroupedProblem* __restrict__ probs,
                                                                 const GroupedUnit* __restrict__ units, int64_t nunits,
                                                                 const uint64_t* __restrict__ ptrs,
                                                                 double* __restrict__ partials,
-                                                                uint32_t* __restrict__ counters) {
-  grouped_gemm_body<double2, double>(probs, units, nunits, ptrs, partials, counters);
+                                                                uint32_t* __restrict__ queue) {
+  grouped_gemm_body<double2, double>(probs, units, nunits, ptrs, partials, queue);
 }
 
 int grouped_occupancy(int dtype) {
@@ -795,20 +612,23 @@ int grouped_occupancy(int dtype) {
 
 int launch_grouped_gemm(const GroupedLaunch& g, hipStream_t s) {
   if (g.nunits <= 0) return TENET_OK;
-  // the queue head is cleared by a kernel (graph-safe); tile counters are
-  // left at zero by the reducing workgroups and cleared at plan creation
-  {
-    const int st = launch_fill_zero(g.counters, sizeof(uint32_t), s);
-    if (st != TENET_OK) return st;
-  }
   const int64_t grid = std::max<int64_t>(1, std::min<int64_t>(g.nunits, g.grid));
   if (g.dtype == TENET_C128)
     hipLaunchKernelGGL(grouped_gemm_c128_kernel, dim3((unsigned)grid), dim3(256), 0, s, g.probs,
-                       g.units, g.nunits, g.ptrs, (double*)g.partials, g.counters);
+                       g.units, g.nunits, g.ptrs, (double*)g.partials, g.queue);
   else
     hipLaunchKernelGGL(grouped_gemm_c64_kernel, dim3((unsigned)grid), dim3(256), 0, s, g.probs,
-                       g.units, g.nunits, g.ptrs, (float*)g.partials, g.counters);
+                       g.units, g.nunits, g.ptrs, (float*)g.partials, g.queue);
   TENET_HIP_CHECK(hipGetLastError());
+  if (g.nsplit > 0) {
+    if (g.dtype == TENET_C128)
+      hipLaunchKernelGGL((grouped_reduce_kernel<double2, double>), dim3((unsigned)g.nsplit), dim3(256), 0, s, g.probs,
+                         g.split, g.ptrs, (const double*)g.partials);
+    else
+      hipLaunchKernelGGL((grouped_reduce_kernel<float2, float>), dim3((unsigned)g.nsplit), dim3(256), 0, s, g.probs,
+                         g.split, g.ptrs, (const float*)g.partials);
+    TENET_HIP_CHECK(hipGetLastError());
+  }
   return TENET_OK;
 }
 

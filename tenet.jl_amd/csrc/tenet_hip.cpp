@@ -778,7 +778,6 @@ static void radix_table(const std::vector<LabelInfo*>& ls, int which, std::vecto
 // kB, colB, bB, rowC, colC, bC) and the GEMM shape, on the host.
 struct HostPlan {
   int64_t M = 0, N = 0, K = 0, batch = 0;
-  int a_mfast = 0, b_nfast = 0;
   int64_t spanA = 0, spanB = 0, spanC = 0;
   std::vector<int64_t> v[9];
 };
@@ -920,7 +919,14 @@ static int analyse_plan(const tenet_tdesc* a, const tenet_tdesc* b, const tenet_
   };
   std::stable_sort(fa.begin(), fa.end(), by(0));
   std::stable_sort(fb.begin(), fb.end(), by(1));
-  std::stable_sort(kk.begin(), kk.end(), by(0));
+  // K runs along the operand that has its adjacent entries there (the longer
+  // run if both do), so that its gathers touch the fewest cache lines
+  int64_t run[2] = {1, 1};
+  for (auto* x : kk) {
+    if (x->sa == 1) run[0] = std::max(run[0], x->extent);
+    if (x->sb == 1) run[1] = std::max(run[1], x->extent);
+  }
+  std::stable_sort(kk.begin(), kk.end(), by(run[1] > run[0] ? 1 : 0));
   std::stable_sort(bt.begin(), bt.end(), by(2));
 
   radix_table(fa, 0, hp.v[0]);  // rowA
@@ -936,8 +942,6 @@ static int analyse_plan(const tenet_tdesc* a, const tenet_tdesc* b, const tenet_
   hp.N = (int64_t)hp.v[4].size();
   hp.K = (int64_t)hp.v[1].size();
   hp.batch = (int64_t)hp.v[2].size();
-  hp.a_mfast = (!fa.empty() && fa[0]->sa == 1) ? 1 : 0;
-  hp.b_nfast = (!fb.empty() && fb[0]->sb == 1) ? 1 : 0;
   auto span = [](const tenet_tdesc* d) {
     int64_t s = 0;
     for (int i = 0; i < d->rank; ++i) {
@@ -969,16 +973,16 @@ static void set_tables(GemmTables& t, int64_t* T, const size_t* off) {
 // rounds of 256 CUs (1024^3, N/T 126 : 145, C/N 136 : 145; 4096^3 7640 : 8090);
 // a last round mostly empty costs the library more than the tiles' rate gains
 // (3072 x 768 x 3840, 2.25 rounds, 1300 : 1140; 1536^3 538 : 500).  complex64:
-// A contiguous along K from 400^3 on (13.5 : 15.7; 700^3 26 : 40; but
-// 300 x 300 x 600 19.6 : 11.7), otherwise only very large ones (2048^3
-// 538 : 612; 1024^3 157 : 92, 250 x 1250 x 462 42 : 20).
+// a band of sizes, with A contiguous along K around 700^3 (26 : 39; 512^3
+// 17.4 : 16.7, 1024^3 90 : 84, 2048^3 637 : 560), otherwise around 2048^3
+// (538 : 605; 1024^3 157 : 84, 250 x 1250 x 462 42 : 19, 4096^3 4890 : 4440).
 static bool lib_pays(int dtype, rocblas_operation opA, int64_t M, int64_t N, int64_t K, int64_t batch) {
   const double fl = 8.0 * M * N * K * batch;
   if (dtype == TENET_C128) {
     const double rounds = (double)((M + 63) / 64) * ((N + 63) / 64) * batch / 256.0;
     return fl >= 5e9 && rounds >= 0.92 * std::ceil(rounds);
   }
-  return fl >= (opA == rocblas_operation_none ? 3e10 : 5e8);
+  return opA == rocblas_operation_none ? fl >= 3e10 && fl < 3e11 : fl >= 1.5e9 && fl < 6e9;
 }
 
 static int build_plan(tenet_ctx ctx, int dtype, int prec, const tenet_tdesc* a, const tenet_tdesc* b,
@@ -1947,10 +1951,12 @@ struct tenet_gplan_s {
   tenet_ctx ctx = nullptr;
   int dtype = 0, prec = 0;
   int64_t count = 0, nunits = 0, grid = 0;
-  void* dev = nullptr;  // one allocation: tables, problems, units, counters, partials, pointer staging
+  void* dev = nullptr;  // one allocation: tables, problems, units, queue, partials, pointer staging
   GroupedProblem* probs = nullptr;
   GroupedUnit* units = nullptr;
-  uint32_t* counters = nullptr;
+  uint32_t* queue = nullptr;
+  GroupedUnit *split = nullptr, *split_rest = nullptr;  // tiles cut into K chunks
+  int64_t nsplit_rest = 0;
   void* partials = nullptr;
   // operand pointers of tenet_grouped_exec: a ring of device tables filled
   // from pinned host slots, each slot reused once the event recorded after
@@ -1998,18 +2004,46 @@ static bool plain_gemm(const HostPlan& hp, bool conjA, bool conjB, rocblas_opera
 
 static const int TILE_EDGE[3] = {64, 32, 16};
 
-// Relative cost of one (tile, 16-wide K step) per tile shape.  Measured by
-// tenet_autotune_tiles; until then a model: the three shapes run 64, 16 and
-// 4 MFMA blocks per K step on four waves, with a fixed per-step overhead.
-static void tile_costs(tenet_ctx ctx, int dtype, double c[3]) {
-  const int d = dtype == TENET_C128 ? 0 : 1;
-  if (ctx->tile_cost[d][0] > 0) {
-    for (int i = 0; i < 3; ++i) c[i] = ctx->tile_cost[d][i];
-    return;
-  }
-  c[0] = 1.0;
-  c[1] = 0.40;
-  c[2] = 0.25;
+// Cycles of a unit outside its K steps (queue, first loads, epilogue), and the
+// smallest unit worth cutting off a longer one.  Batches of 40..1024 unlike
+// problems time within 2% for 1000..6000 and 8192..32768.
+constexpr double UNIT_CYCLES = 3000.0, MIN_UNIT_CYCLES = 16384.0;
+
+// Cycles of a CU's address unit per wave load of 16 rows x 4 contracted
+// entries, from the cache lines it touches (rows: the runs of adjacent row
+// entries; k: those of the contracted entries; pair: two k steps per load).
+static double gather_cycles(const std::vector<int64_t>& rows, const std::vector<int64_t>& k, bool pair) {
+  auto run = [](const std::vector<int64_t>& t) {
+    if (t.size() < 2) return 1.0;
+    size_t breaks = 0;
+    for (size_t i = 1; i < t.size(); ++i) breaks += t[i] != t[i - 1] + 1;
+    return (double)t.size() / (double)(breaks + 1);
+  };
+  const double rr = rows.size() < 2 ? 16.0 : std::min(16.0, run(rows));
+  const double kr = k.size() < 2 ? 4.0 : std::min(4.0, run(k));
+  const double lines = std::max(4.0, 64.0 / std::max(rr, kr));
+  return (16.0 + 2.0 * lines) * (pair && rr < kr ? 0.5 : 1.0);
+}
+
+// Modelled cycles of one (tile, 16-wide K step) per tile shape: the larger of
+// the MFMA time on each SIMD (64, 16 and 4 blocks x 4 products over the four
+// waves) and the operand loads' address time.  The 32 x 32 shape, whose waves
+// deal K, measured 0.8 of that (five batches of each type, 4% in the mean).
+static void tile_step_cycles(int dtype, double clx, double cly, double c[3]) {
+  const double mf = dtype == TENET_C128 ? 64 : 32;
+  c[0] = std::max(64 * mf, 32 * (clx + cly));
+  c[1] = 0.8 * std::max(16 * mf, 8 * (clx + cly));
+  c[2] = std::max(4 * mf, 4 * (clx + cly));
+}
+
+// The model above with each shape's measured efficiency (tenet_autotune_tiles).
+static void tile_costs(tenet_ctx ctx, int dtype, double clx, double cly, double c[3]) {
+  tile_step_cycles(dtype, clx, cly, c);
+  const double* t = ctx->tile_cost[dtype == TENET_C128 ? 0 : 1];
+  if (t[0] <= 0) return;
+  double ref[3];  // the model's costs of the measured problem
+  tile_step_cycles(dtype, 24, 24, ref);
+  for (int v = 0; v < 3; ++v) c[v] *= t[v] * ref[0] / (t[0] * ref[v]);
 }
 
 static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count, const tenet_tdesc* descs,
@@ -2024,8 +2058,6 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
   g->spanA.resize((size_t)count);
   g->spanB.resize((size_t)count);
   g->spanC.resize((size_t)count);
-  double c[3];
-  tile_costs(ctx, dtype, c);
   size_t table_elems = 0;
   double total_cost = 0.0;
   std::vector<double> tile_step_cost((size_t)count);
@@ -2038,8 +2070,6 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
     q.N = hp.N;
     q.K = hp.K;
     q.batch = hp.batch;
-    q.a_mfast = hp.a_mfast;
-    q.b_nfast = hp.b_nfast;
     q.conjA = conj ? (conj[2 * i] != 0) : 0;
     q.conjB = conj ? (conj[2 * i + 1] != 0) : 0;
     g->spanA[(size_t)i] = hp.spanA;
@@ -2062,19 +2092,30 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
       const int64_t sn = hp.N > 1 ? stride_of(hp.v[7]) : INT64_MAX;
       const int64_t sz = hp.batch > 1 ? stride_of(hp.v[8]) : INT64_MAX;
       q.order = (sm <= sn && sm <= sz) ? 0 : (sn <= sz ? 1 : 2);
-      tile_step_cost[(size_t)i] = c[0];
-      if (total > 0) total_cost += c[0] * (double)q.tiles_m;
+      // 16 elements per thread, two loads per term
+      tile_step_cost[(size_t)i] = 3072.0 * (double)std::max<int64_t>(hp.K, 1);
+      if (total > 0) total_cost += (tile_step_cost[(size_t)i] + UNIT_CYCLES) * (double)q.tiles_m;
       continue;
     }
     q.order = 0;
+    {
+      auto gap = [](const std::vector<int64_t>& v) { return v.size() > 1 ? std::llabs(v[1] - v[0]) : INT64_MAX; };
+      q.j_is_m = gap(hp.v[6]) <= gap(hp.v[7]) ? 1 : 0;
+      q.pairs = (k_pairs(hp.v[1]) ? 1 : 0) | (k_pairs(hp.v[3]) ? 2 : 0);
+    }
     // tile shape with the least modelled time for this problem
     const int64_t ksteps = std::max<int64_t>(1, (hp.K + 15) / 16);
     int best = 0;
-    double best_t = 0.0;
+    double best_t = 0.0, c[3];
+    const bool lanes_m = q.j_is_m != 0;
+    const double ca = gather_cycles(hp.v[0], hp.v[1], dtype == TENET_C64 && (q.pairs & 1));
+    const double cb = gather_cycles(hp.v[4], hp.v[3], dtype == TENET_C64 && (q.pairs & 2));
+    tile_costs(ctx, dtype, lanes_m ? cb : ca, lanes_m ? ca : cb, c);
     for (int v = 0; v < 3; ++v) {
       if (force_shape >= 0 && v != force_shape) continue;
       const int64_t e = TILE_EDGE[v];
-      const double t = c[v] * (double)((hp.M + e - 1) / e) * (double)((hp.N + e - 1) / e) * hp.batch * ksteps;
+      const double t =
+          (c[v] * ksteps + UNIT_CYCLES) * (double)((hp.M + e - 1) / e) * (double)((hp.N + e - 1) / e) * hp.batch;
       if (force_shape >= 0 || t < best_t || best_t == 0.0) {
         best = v;
         best_t = t;
@@ -2103,6 +2144,11 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
     for (auto& kv : groups) {
       const auto& key = kv.first;
       const double fl = 8.0 * std::get<2>(key) * std::get<3>(key) * std::get<4>(key) * (double)kv.second.size();
+      // a batch of eight or more fills the chip in one library launch; fewer
+      // go there only where the library would take one of them alone
+      if (kv.second.size() < 8 && !lib_pays(dtype, (rocblas_operation)std::get<0>(key), std::get<2>(key),
+                                            std::get<3>(key), std::get<4>(key), (int64_t)kv.second.size()))
+        continue;
       if (fl < LIB_MIN_FLOPS || std::get<2>(key) < 16 || std::get<3>(key) < 16 || std::get<4>(key) < 16) continue;
       tenet_gplan_s::LibGroup lg;
       lg.opA = (rocblas_operation)std::get<0>(key);
@@ -2136,15 +2182,14 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
   // K chunking: no unit above ~1/4 of one workgroup's fair share (with four
   // or more tiles per workgroup the LPT queue balances them whole; chunks
   // cost partial sums through memory)
-  const double unit_cap = std::max(total_cost / ((double)g->grid * 4.0), 16.0 * c[0]);
-  int64_t part_elems = 0, ctr_elems = 0, nunits = 0;
+  const double unit_cap = std::max(total_cost / ((double)g->grid * 4.0), MIN_UNIT_CYCLES);
+  int64_t part_elems = 0, nunits = 0;
   for (int64_t i = 0; i < count; ++i) {
     GroupedProblem& q = probs[(size_t)i];
     if (q.shape == GROUPED_SMALLK) {
       q.kchunks = 1;
       q.kc = q.K;
       q.part_base = -1;
-      q.ctr_base = -1;
       nunits += q.tiles_m;
       continue;
     }
@@ -2159,13 +2204,10 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
     q.kc = kcs * 16;
     const int64_t tiles = q.tiles_m * q.tiles_n * q.batch;
     q.part_base = -1;
-    q.ctr_base = -1;
     if (ch > 1) {
       const int64_t e = TILE_EDGE[q.shape];
       q.part_base = part_elems;
       part_elems += tiles * ch * e * e;
-      q.ctr_base = ctr_elems;
-      ctr_elems += tiles;
       g->split_tiles += tiles;
     }
     nunits += tiles * ch;
@@ -2179,11 +2221,12 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
   order.reserve((size_t)count);
   for (int64_t i = 0; i < count; ++i) {
     const GroupedProblem& q = probs[(size_t)i];
-    order.push_back({tile_step_cost[(size_t)i] * (double)((q.K + 15) / 16) / q.kchunks, i});
+    const double steps = q.shape == GROUPED_SMALLK ? 1.0 : (double)((q.K + 15) / 16) / q.kchunks;
+    order.push_back({tile_step_cost[(size_t)i] * steps, i});
   }
   std::stable_sort(order.begin(), order.end(),
                    [](const std::pair<double, int64_t>& x, const std::pair<double, int64_t>& y) { return x.first > y.first; });
-  std::vector<GroupedUnit> units_rest;
+  std::vector<GroupedUnit> units_rest, split, split_rest;
   for (auto& o : order) {
     const GroupedProblem& q = probs[(size_t)o.second];
     const int64_t tiles = q.shape == GROUPED_SMALLK ? q.tiles_m : q.tiles_m * q.tiles_n * q.batch;
@@ -2192,6 +2235,10 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
         units.push_back({(int32_t)o.second, ch, t});
         if (!in_lib[(size_t)o.second]) units_rest.push_back({(int32_t)o.second, ch, t});
       }
+    for (int64_t t = 0; q.kchunks > 1 && t < tiles; ++t) {
+      split.push_back({(int32_t)o.second, 0, t});
+      if (!in_lib[(size_t)o.second]) split_rest.push_back({(int32_t)o.second, 0, t});
+    }
   }
   g->nunits_rest = (int64_t)units_rest.size();
   // one device allocation
@@ -2200,20 +2247,26 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
   const size_t b_prob = align_up((size_t)count * sizeof(GroupedProblem), 256);
   const size_t b_unit = align_up(std::max<size_t>(units.size(), 1) * sizeof(GroupedUnit), 256);
   const size_t b_unit_rest = g->nlib ? align_up(std::max<size_t>(units_rest.size(), 1) * sizeof(GroupedUnit), 256) : 0;
-  const size_t b_ctr = align_up((size_t)(64 + ctr_elems) * 4, 256);
+  const size_t b_queue = 256;
+  const size_t b_split = align_up(split.size() * sizeof(GroupedUnit), 256);
+  const size_t b_split_rest = align_up(split_rest.size() * sizeof(GroupedUnit), 256);
   const size_t b_part = align_up((size_t)std::max<int64_t>(part_elems, 1) * 2 * rs, 256);
   const size_t b_ptr = align_up((size_t)g->slot_elems * 8, 256) * tenet_gplan_s::RING;
   // from the context's caching pool: plans are built per batch shape, and a
   // device allocation per plan would cost more than the plan's analysis
-  TRY(tenet_malloc(ctx, b_tab + b_prob + b_unit + b_ctr + b_part + b_ptr + b_unit_rest, &g->dev));
+  TRY(tenet_malloc(ctx, b_tab + b_prob + b_unit + b_queue + b_part + b_ptr + b_unit_rest + b_split + b_split_rest,
+                   &g->dev));
   char* base = (char*)g->dev;
   int64_t* tables = (int64_t*)base;
   g->probs = (GroupedProblem*)(base + b_tab);
   g->units = (GroupedUnit*)(base + b_tab + b_prob);
-  g->counters = (uint32_t*)(base + b_tab + b_prob + b_unit);
-  g->partials = (void*)(base + b_tab + b_prob + b_unit + b_ctr);
-  g->ptrs_dev = (uint64_t*)(base + b_tab + b_prob + b_unit + b_ctr + b_part);
-  g->units_rest = g->nlib ? (GroupedUnit*)(base + b_tab + b_prob + b_unit + b_ctr + b_part + b_ptr) : g->units;
+  g->queue = (uint32_t*)(base + b_tab + b_prob + b_unit);
+  g->partials = (void*)(base + b_tab + b_prob + b_unit + b_queue);
+  g->ptrs_dev = (uint64_t*)(base + b_tab + b_prob + b_unit + b_queue + b_part);
+  g->units_rest = g->nlib ? (GroupedUnit*)(base + b_tab + b_prob + b_unit + b_queue + b_part + b_ptr) : g->units;
+  g->split = (GroupedUnit*)(base + b_tab + b_prob + b_unit + b_queue + b_part + b_ptr + b_unit_rest);
+  g->split_rest = (GroupedUnit*)((char*)g->split + b_split);
+  g->nsplit_rest = (int64_t)split_rest.size();
   if (!g->nlib) {
     g->nunits_rest = g->nunits;
     g->flops_rest = g->flops;
@@ -2239,7 +2292,12 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
   if (g->nlib && !units_rest.empty())
     TENET_HIP_CHECK(hipMemcpy(g->units_rest, units_rest.data(), units_rest.size() * sizeof(GroupedUnit),
                               hipMemcpyHostToDevice));
-  TENET_HIP_CHECK(hipMemset(g->counters, 0, b_ctr));
+  if (!split.empty())
+    TENET_HIP_CHECK(hipMemcpy(g->split, split.data(), split.size() * sizeof(GroupedUnit), hipMemcpyHostToDevice));
+  if (!split_rest.empty())
+    TENET_HIP_CHECK(hipMemcpy(g->split_rest, split_rest.data(), split_rest.size() * sizeof(GroupedUnit),
+                              hipMemcpyHostToDevice));
+  TENET_HIP_CHECK(hipMemset(g->queue, 0, b_queue));
   return TENET_OK;
 }
 
@@ -2286,7 +2344,9 @@ static int grouped_launch(tenet_gplan g, hipStream_t s, const uint64_t* ptrs, bo
   if (L.nunits == 0) return TENET_OK;
   L.ptrs = ptrs;
   L.partials = g->partials;
-  L.counters = g->counters;
+  L.queue = g->queue;
+  L.split = rest ? g->split_rest : g->split;
+  L.nsplit = rest ? g->nsplit_rest : g->split_tiles;
   L.grid = g->grid;
   L.dtype = g->dtype;
   L.prec = g->prec;
