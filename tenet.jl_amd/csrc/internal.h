@@ -227,22 +227,33 @@ int launch_absorb(const void* U, int64_t m, const void* Vh, int64_t ldvh, int64_
 // scale by 1/max|x| and accumulate log(max) into acc[2]; optionally mantissa out
 int launch_rescale_log(void* x, int64_t count, double* acc, int dtype, hipStream_t s);
 // site-parallel amplitudes (k_misc.hip): device tables as for
-// launch_amplitudes, plus chi_max / d bounds and workspace rows (two
-// 2 chi_max double rows per request, one log-scale per request).
+// launch_amplitudes for up to AMP_SLICE requests at a time, the chi_max / n_max / d
+// bounds and workspace (per request two vector rows of 2 chi_max doubles and
+// a log-scale; per site position the requests' tiles and maxima).
+constexpr int64_t AMP_SLICE = 2048;
+struct AmpTile {
+  uint64_t slice;  // address of A[:, x, :]
+  int32_t cl, cr;
+  int32_t rows, pad;  // 0 past the site's last tile
+  int32_t req[16];    // its requests (the last one repeated)
+};
 struct AmpSiteArgs {
   const int64_t* n;
   const uint64_t* sites;
   const uint64_t* chis;
   const uint64_t* bits;
-  int64_t d, chi_max, n_max;
+  int64_t d, chi_max, n_max, nreq;
   double* vbuf;
   double* logs;
   double* out;
+  unsigned long long* vmax;  // n_max x nreq
+  AmpTile* tiles;            // n_max x nreq
+  int32_t* valid;            // nreq
 };
-// one site position of every request (a no-op for requests with fewer sites);
-// e0 / e1: optional event pair stamped by the dispatch
-int launch_amp_site(const AmpSiteArgs& a, int64_t nreq, int64_t site, int dtype, hipStream_t s, hipEvent_t e0,
-                    hipEvent_t e1);
+// the requests' checks and every site position's tiles
+int launch_amp_groups(const AmpSiteArgs& a, int dtype, hipStream_t s);
+// one site position of every request; e0 / e1: optional event pair stamped by the dispatch
+int launch_amp_site(const AmpSiteArgs& a, int64_t site, int dtype, hipStream_t s, hipEvent_t e0, hipEvent_t e1);
 int launch_amplitudes(int64_t nreq, const int64_t* n_dev, const uint64_t* site_ptrs, const uint64_t* chis,
                       const uint64_t* bits, int64_t d, double* out, int dtype, int max_chi, hipStream_t s);
 int launch_write_scalar_from(const void* env, double* out, int dtype, hipStream_t s);

@@ -501,143 +501,356 @@ __global__ __launch_bounds__(AMP_THREADS) void amplitude_kernel(const int64_t* _
 }
 
 // ---- site-parallel amplitudes ------------------------------------------------
-// One launch per site position: workgroup (column block, request) computes
-// AS_COLS entries of v' = (v / m) A[:, x_i, :] for its request, where v is the
-// request's previous vector (read whole from the workspace into LDS) and m
-// its largest |component| (every workgroup of the request computes the same
-// m, so the rescale is deterministic); the workgroup of column block 0 adds
-// log(m) to the request's log-scale.  A request's vectors alternate between
-// two workspace rows; at its last site (chi_r = 1) block 0 writes
-// (re, im, log-scale) to out.  The chain is sequential over sites, so a
-// request's sites are spread over launches instead of one workgroup, and a
-// 512 x 512 slice is read by 32 workgroups at once.
-constexpr int AS_THREADS = 256;
-constexpr int AS_COLS = 16;  // columns per workgroup: 4 per wave
+// One launch per site position.  The requests that read the same slice
+// A[:, x, :] at a site (same tensor, same basis value) form tiles of up to 16
+// rows, and a workgroup computes 16 columns of v' = (v / m) A[:, x, :] for one
+// tile on the FP64 matrix cores, its eight waves dealing the contracted
+// index: a slice leaves the caches once per 16 requests instead of once per
+// request (128 amplitudes of a chi 400 complex64 state: 36.5 us per site
+// position when every request read its own slice, L2-bound).  Tiles of up to
+// 8 rows use the 4 x 4 x 4 instruction, so that a lone request does not pay
+// for 16 rows.  Both instructions add their products in the order of the
+// contracted index, one rounding each (checked bitwise against sequential
+// fma), so a request's value does not depend on the tile it falls into.
+// 96 sites, chi 400, complex64: 128 requests 3.62 -> 1.14 ms, 512 10.4 ->
+// 2.36, one 1.36 -> 0.72; what is left per site is a chain of dependent
+// reads (tile, maximum, vector) between two launches.
+//
+// m is the vector's largest |component|, gathered by the launch of the site
+// before with an atomic maximum; a request's log-scale collects log(m); its
+// vectors alternate between two workspace rows; at its last site (chi_r = 1)
+// (re, im, log-scale) go to out.
+constexpr int AT_WAVES = 8;
+constexpr int AT_ROWS = 16, AT_COLS = 16;
 
-template <typename S2>
-__global__ __launch_bounds__(AS_THREADS) void amp_site_kernel(AmpSiteArgs a, int64_t site) {
-  __shared__ double vr[AMP_MAX_CHI], vi[AMP_MAX_CHI];
-  __shared__ double wm[AS_THREADS / 64];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int64_t req = blockIdx.y;
+// One wave per request: reject requests with more sites than the launches
+// cover or a bond or basis value out of range (NaN, and no tile takes them),
+// and clear the request's maxima.
+__global__ __launch_bounds__(64) void amp_check_kernel(AmpSiteArgs a) {
+  const int64_t req = blockIdx.x;
+  const int lane = threadIdx.x;
   const int64_t n = a.n[req];
-  if (n > a.n_max) {
-    // more sites than the launches cover: report NaN once
-    if (site == 0 && blockIdx.x == 0 && threadIdx.x == 0) {
+  const int64_t* chi = reinterpret_cast<const int64_t*>(a.chis[req]);
+  const uint8_t* x = reinterpret_cast<const uint8_t*>(a.bits[req]);
+  bool bad = n > a.n_max;
+  if (!bad)
+    for (int64_t i = lane; i < n; i += 64) {
+      const int64_t cl = chi[i], cr = chi[i + 1];
+      bad = bad || cl < 1 || cr < 1 || cl > a.chi_max || cr > a.chi_max || (int64_t)x[i] >= a.d ||
+            (i == 0 && cl != 1) || (i == n - 1 && cr != 1);
+    }
+  const bool any = __any(bad);
+  for (int64_t i = lane; i < a.n_max; i += 64) a.vmax[i * a.nreq + req] = 0ull;
+  if (lane == 0) {
+    a.valid[req] = any ? 0 : 1;
+    if (any) {
       a.out[3 * req + 0] = __builtin_nan("");
       a.out[3 * req + 1] = __builtin_nan("");
       a.out[3 * req + 2] = 0.0;
     }
-    return;
   }
-  if (site >= n) return;
-  const int64_t* chi = reinterpret_cast<const int64_t*>(a.chis[req]);
-  const uint8_t* x = reinterpret_cast<const uint8_t*>(a.bits[req]);
-  const int64_t cl = chi[site], cr = chi[site + 1];
-  const int64_t cb0 = (int64_t)blockIdx.x * AS_COLS;
-  if (cb0 >= cr && !(cr < 1 && blockIdx.x == 0)) return;
-  double* out = a.out + 3 * req;
-  if (cl < 1 || cr < 1 || cl > a.chi_max || cr > a.chi_max || (int64_t)x[site] >= a.d || (site == 0 && cl != 1) ||
-      (site == n - 1 && cr != 1)) {
-    // uniform across the request's workgroups: report NaN instead of reading
-    // out of bounds, and mark the request so that its later sites skip it
-    if (blockIdx.x == 0 && tid == 0) {
-      out[0] = __builtin_nan("");
-      out[1] = __builtin_nan("");
-      out[2] = 0.0;
-      a.logs[req] = __builtin_nan("");
+}
+
+// One workgroup per site position: the requests in the order of (tensor,
+// basis value, bonds), cut into tiles of up to 16 that share all of them.
+constexpr int AG_THREADS = 256;
+
+__global__ __launch_bounds__(AG_THREADS) void amp_group_kernel(AmpSiteArgs a, int npow, int elem) {
+  extern __shared__ unsigned long long ag_key[];  // npow keys, then npow request numbers, then npow scan words
+  int* idx = reinterpret_cast<int*>(ag_key + npow);
+  int* head = idx + npow;
+  const int64_t site = blockIdx.x;
+  const int tid = threadIdx.x, nreq = (int)a.nreq;
+  for (int p = tid; p < npow; p += AG_THREADS) {
+    unsigned long long k = ~0ull;
+    if (p < nreq && a.valid[p] && site < a.n[p]) {
+      const uint64_t A = reinterpret_cast<const uint64_t*>(a.sites[p])[site];
+      const int64_t cl = reinterpret_cast<const int64_t*>(a.chis[p])[site];
+      const uint8_t x = reinterpret_cast<const uint8_t*>(a.bits[p])[site];
+      k = A + (uint64_t)x * (uint64_t)cl * (uint64_t)elem;  // the slice's address
     }
-    return;
-  }
-  if (site > 0 && __builtin_isnan(a.logs[req])) return;  // marked at an earlier site
-  double* vin = a.vbuf + ((size_t)req * 2 + ((site + 1) & 1)) * 2 * a.chi_max;
-  double* vout = a.vbuf + ((size_t)req * 2 + (site & 1)) * 2 * a.chi_max;
-  // previous vector into LDS and its largest component
-  double m = 1.0;
-  if (site == 0) {
-    if (tid == 0) {
-      vr[0] = 1.0;
-      vi[0] = 0.0;
-    }
-  } else {
-    double mx = 0.0;
-    for (int64_t l = tid; l < cl; l += AS_THREADS) {
-      const double re = vin[2 * l], im = vin[2 * l + 1];
-      vr[l] = re;
-      vi[l] = im;
-      mx = fmax(mx, fmax(fabs(re), fabs(im)));
-    }
-    mx = wave_max(mx);
-    if (lane == 0) wm[wave] = mx;
-    __syncthreads();
-    m = fmax(fmax(wm[0], wm[1]), fmax(wm[2], wm[3]));
-    if (!(m > 0.0)) m = 1.0;
+    ag_key[p] = k;
+    idx[p] = p;
   }
   __syncthreads();
-  const double sc = 1.0 / m;
-  if (blockIdx.x == 0 && tid == 0) a.logs[req] = (site == 0 ? 0.0 : a.logs[req] + log(m));
-  const S2* A = reinterpret_cast<const S2*>(reinterpret_cast<const uint64_t*>(a.sites[req])[site]) +
-                (int64_t)x[site] * cl;
-  const int64_t ld = cl * a.d;
-  const int64_t c0 = cb0 + 4 * wave;
-  double acc[8];
+  for (int size = 2; size <= npow; size <<= 1)
+    for (int st = size >> 1; st > 0; st >>= 1) {
+      for (int q = tid; q < npow / 2; q += AG_THREADS) {
+        const int lo = 2 * q - (q & (st - 1)), hi = lo + st;
+        const unsigned long long x = ag_key[lo], y = ag_key[hi];
+        const int xi = idx[lo], yi = idx[hi];
+        const bool up = (lo & size) == 0, gt = x > y || (x == y && xi > yi);
+        if (gt == up) {
+          ag_key[lo] = y;
+          ag_key[hi] = x;
+          idx[lo] = yi;
+          idx[hi] = xi;
+        }
+      }
+      __syncthreads();
+    }
+  // head[p]: where p's group (equal slice and bonds) begins
+  auto bond = [&](int r, int which) { return reinterpret_cast<const int64_t*>(a.chis[r])[site + which]; };
+  for (int p = tid; p < npow; p += AG_THREADS) {
+    bool first = p == 0 || ag_key[p] != ag_key[p - 1];
+    if (!first && ag_key[p] != ~0ull)
+      first = bond(idx[p], 0) != bond(idx[p - 1], 0) || bond(idx[p], 1) != bond(idx[p - 1], 1);
+    head[p] = first ? p : 0;
+  }
+  __syncthreads();
+  for (int st = 1; st < npow; st <<= 1) {  // running maximum
+    int v[8];
+    int u = 0;
+    for (int p = tid; p < npow; p += AG_THREADS, ++u) v[u] = p >= st ? max(head[p], head[p - st]) : head[p];
+    __syncthreads();
+    u = 0;
+    for (int p = tid; p < npow; p += AG_THREADS, ++u) head[p] = v[u];
+    __syncthreads();
+  }
+  __shared__ int count;
+  if (tid == 0) count = 0;
+  __syncthreads();
+  AmpTile* tiles = a.tiles + site * a.nreq;
+  for (int p = tid; p < nreq; p += AG_THREADS) {
+    if (ag_key[p] == ~0ull || (p - head[p]) % AT_ROWS != 0) continue;
+    int c = 1;
+    while (c < AT_ROWS && p + c < nreq && head[p + c] == head[p]) ++c;
+    AmpTile* t = tiles + atomicAdd(&count, 1);  // the tiles' order is of no consequence
+    t->slice = ag_key[p];
+    t->cl = (int32_t)bond(idx[p], 0);
+    t->cr = (int32_t)bond(idx[p], 1);
+    t->rows = c;
+    for (int i = 0; i < AT_ROWS; ++i) t->req[i] = idx[p + min(i, c - 1)];
+  }
+  __syncthreads();
+  for (int p = count + tid; p < nreq; p += AG_THREADS) tiles[p].rows = 0;
+}
+
+__device__ __forceinline__ void at_load2(const double2* p, double2 (&y)[2]) {
+  y[0] = p[0];
+  y[1] = p[1];
+}
+__device__ __forceinline__ void at_load2(const float2* p, float2 (&y)[2]) {
+  typedef float f4 __attribute__((ext_vector_type(4), aligned(8)));  // two entries in one load
+  const f4 v = *reinterpret_cast<const f4*>(p);
+  y[0] = make_float2(v[0], v[1]);
+  y[1] = make_float2(v[2], v[3]);
+}
+
+typedef double at_d4 __attribute__((ext_vector_type(4)));
+
+// Accumulate one wave's share of a tile.  Each pair of steps covers eight
+// contracted indices, lane group g = lane / 16 taking 2 g and 2 g + 1.
+// NG = 0: 16 rows by 16 x 16 x 4 (row l % 16 of the operand, rows 4 r + g of
+// the result); NG = 1, 2: that many groups of 4 rows by 4 x 4 x 4 (row l % 4
+// of the operand in each of the four blocks of 4 columns, row g of the
+// result).
+template <typename S2, int NG>
+__device__ __forceinline__ void at_accumulate(const S2* __restrict__ A, int64_t ld, int cl, int col,
+                                              const double* const (&vrow)[2], const double (&sc)[2], int wave,
+                                              double (&cr)[4], double (&ci)[4]) {
+  constexpr int NX = NG == 0 ? 1 : NG;
+  const int g = (threadIdx.x & 63) >> 4;
+  at_d4 dr = {0, 0, 0, 0}, di = {0, 0, 0, 0};
 #pragma unroll
-  for (int j = 0; j < 8; ++j) acc[j] = 0.0;
-#pragma unroll 2
-  for (int64_t l = lane; l < cl; l += 64) {
-    const double pr = vr[l] * sc, pi = vi[l] * sc;
+  for (int q = 0; q < 4; ++q) cr[q] = ci[q] = 0.0;
+  const S2* Ac = A + (int64_t)col * ld;
+  const int nsteps = (cl + 7) / 8;
+  struct Step {
+    S2 y[2];
+    double2 x[NX][2];
+  };
+  const bool odd = (cl & 1) != 0;
+  auto load = [&](int s, Step& t) {
+    const int k = 8 * s + 2 * g;
+    const int kk = min(k, cl - 2);  // past the end: the last two entries, sorted out below
+    at_load2(Ac + kk, t.y);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (c0 + j < cr) {
-        const S2 v = A[l + (c0 + j) * ld];
-        const double ar = (double)v.x, ai = (double)v.y;
-        acc[2 * j] += pr * ar - pi * ai;
-        acc[2 * j + 1] += pr * ai + pi * ar;
+    for (int q = 0; q < NX; ++q) {
+      t.x[q][0] = reinterpret_cast<const double2*>(vrow[q])[kk];
+      t.x[q][1] = reinterpret_cast<const double2*>(vrow[q])[kk + 1];
+    }
+    if (8 * s + 8 > cl) {  // the range ends in this step
+      const bool last = odd && k == cl - 1, in0 = k < cl, in1 = k + 1 < cl;
+      const S2 y0 = last ? t.y[1] : t.y[0];
+      t.y[0] = in0 ? y0 : S2{0, 0};
+      t.y[1] = in1 ? t.y[1] : S2{0, 0};
+#pragma unroll
+      for (int q = 0; q < NX; ++q) {
+        const double2 x0 = last ? t.x[q][1] : t.x[q][0];
+        t.x[q][0] = in0 ? x0 : make_double2(0.0, 0.0);
+        t.x[q][1] = in1 ? t.x[q][1] : make_double2(0.0, 0.0);
       }
     }
-  }
+  };
+  auto mul = [&](const Step& t) {
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
+    for (int u = 0; u < 2; ++u) {
+      const double yr = (double)t.y[u].x, yi = (double)t.y[u].y;
+      if constexpr (NG == 0) {
+        const double xr = t.x[0][u].x * sc[0], xi = t.x[0][u].y * sc[0];
+        dr = __builtin_amdgcn_mfma_f64_16x16x4f64(xr, yr, dr, 0, 0, 0);
+        di = __builtin_amdgcn_mfma_f64_16x16x4f64(xr, yi, di, 0, 0, 0);
+        dr = __builtin_amdgcn_mfma_f64_16x16x4f64(-xi, yi, dr, 0, 0, 0);
+        di = __builtin_amdgcn_mfma_f64_16x16x4f64(xi, yr, di, 0, 0, 0);
+      } else {
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc[j] += __shfl_xor(acc[j], off, 64);
-  }
-  if (lane < 4 && c0 + lane < cr) {
-    double re = acc[0], im = acc[1];
-#pragma unroll
-    for (int j = 1; j < 4; ++j)
-      if (lane == j) {
-        re = acc[2 * j];
-        im = acc[2 * j + 1];
+        for (int q = 0; q < NG; ++q) {
+          const double xr = t.x[q][u].x * sc[q], xi = t.x[q][u].y * sc[q];
+          cr[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(xr, yr, cr[q], 0, 0, 0);
+          ci[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(xr, yi, ci[q], 0, 0, 0);
+          cr[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(-xi, yi, cr[q], 0, 0, 0);
+          ci[q] = __builtin_amdgcn_mfma_f64_4x4x4f64(xi, yr, ci[q], 0, 0, 0);
+        }
       }
-    vout[2 * (c0 + lane)] = re;
-    vout[2 * (c0 + lane) + 1] = im;
-    if (site == n - 1 && c0 + lane == 0) {
-      // the last site has chi_r = 1: its single entry is the amplitude
-      out[0] = re;
-      out[1] = im;
-      out[2] = a.logs[req];
+    }
+  };
+  // one step ahead (further ahead, the registers of the three row forms left
+  // one workgroup per CU: 512 requests at chi 400, 23 -> 39 us per site)
+  Step s0, s1;
+  int s = wave;
+  if (s < nsteps) load(s, s0);
+  for (; s < nsteps; s += 2 * AT_WAVES) {
+    const bool two = s + AT_WAVES < nsteps;
+    if (two) load(s + AT_WAVES, s1);
+    mul(s0);
+    if (s + 2 * AT_WAVES < nsteps) load(s + 2 * AT_WAVES, s0);
+    if (two) mul(s1);
+  }
+  if constexpr (NG == 0) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      cr[r] = dr[r];
+      ci[r] = di[r];
     }
   }
 }
 
-int launch_amp_site(const AmpSiteArgs& a, int64_t nreq, int64_t site, int dtype, hipStream_t s, hipEvent_t e0,
-                    hipEvent_t e1) {
-  if (nreq <= 0) return TENET_OK;
+template <typename S2>
+__global__ __launch_bounds__(64 * AT_WAVES, 4) void amp_tile_kernel(AmpSiteArgs a, int64_t site) {
+  __shared__ double2 part[AT_WAVES][AT_ROWS][AT_COLS];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l16 = lane & 15, g = lane >> 4;
+  const int c0 = (int)blockIdx.x * AT_COLS;
+  for (int64_t ti = blockIdx.y; ti < a.nreq; ti += gridDim.y) {
+    const AmpTile& t = a.tiles[site * a.nreq + ti];
+    const int rows = t.rows, tcl = t.cl, tcr = t.cr;
+    if (rows == 0) break;
+    if (c0 >= tcr) continue;  // uniform across the workgroup
+    // the vector's maximum at the site before (a NaN, above every number, or
+    // an all-zero vector gives 1)
+    auto maximum = [&](int r) {
+      if (site == 0) return 1.0;
+      const double m = __longlong_as_double((long long)a.vmax[(site - 1) * a.nreq + r]);
+      return m > 0.0 ? m : 1.0;
+    };
+    const S2* A = reinterpret_cast<const S2*>(t.slice);
+    const int64_t ld = (int64_t)tcl * a.d;
+    const int col = min(c0 + l16, tcr - 1);
+    auto vin = [&](int r) { return a.vbuf + ((size_t)r * 2 + ((site + 1) & 1)) * 2 * a.chi_max; };
+    double cr[4], ci[4];
+    int ng = 4;  // rows come in result registers of 4 rows each
+    if (tcl == 1) {
+      // one term per column (the first site, where v = 1, or a bond of 1)
+      const S2 y = A[(int64_t)col * ld];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int r = t.req[4 * q + g];
+        const double* v = vin(r);
+        const double sc = 1.0 / maximum(r);
+        const double xr = site == 0 ? 1.0 : v[0] * sc, xi = site == 0 ? 0.0 : v[1] * sc;
+        cr[q] = wave == 0 ? fma(-xi, (double)y.y, xr * (double)y.x) : 0.0;
+        ci[q] = wave == 0 ? fma(xi, (double)y.x, xr * (double)y.y) : 0.0;
+      }
+    } else if (rows > 8) {
+      const int r = t.req[l16];
+      const double* const vr[2] = {vin(r), nullptr};
+      const double sc[2] = {1.0 / maximum(r), 0.0};
+      at_accumulate<S2, 0>(A, ld, tcl, col, vr, sc, wave, cr, ci);
+    } else {
+      const int r0 = t.req[lane & 3], r1 = t.req[4 + (lane & 3)];
+      const double* const vr[2] = {vin(r0), vin(r1)};
+      const double sc[2] = {1.0 / maximum(r0), 1.0 / maximum(r1)};
+      if (rows > 4) {
+        ng = 2;
+        at_accumulate<S2, 2>(A, ld, tcl, col, vr, sc, wave, cr, ci);
+      } else {
+        ng = 1;
+        at_accumulate<S2, 1>(A, ld, tcl, col, vr, sc, wave, cr, ci);
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      if (q < ng) part[wave][4 * q + g][l16] = make_double2(cr[q], ci[q]);
+    __syncthreads();
+    for (int e = tid; e < AT_ROWS * AT_COLS; e += 64 * AT_WAVES) {
+      const int row = e / AT_COLS, c = e % AT_COLS;
+      double re = 0.0, im = 0.0;
+      const bool mine = row < rows && c0 + c < tcr;
+      if (mine) {
+#pragma unroll
+        for (int w = 0; w < AT_WAVES; ++w) {
+          const double2 p = part[w][row][c];
+          re += p.x;
+          im += p.y;
+        }
+      }
+      double mx = fmax(fabs(re), fabs(im));
+#pragma unroll
+      for (int off = 8; off > 0; off >>= 1) mx = fmax(mx, __shfl_xor(mx, off, 16));
+      if (mine) {
+        const int r = t.req[row];
+        double* vout = a.vbuf + ((size_t)r * 2 + (site & 1)) * 2 * a.chi_max;
+        vout[2 * (c0 + c)] = re;
+        vout[2 * (c0 + c) + 1] = im;
+        // nonnegative doubles order like their bits
+        if (c == 0) atomicMax(&a.vmax[site * a.nreq + r], (unsigned long long)__double_as_longlong(mx));
+        if (c0 + c == 0) {
+          const double lg = site == 0 ? 0.0 : a.logs[r] + log(maximum(r));
+          a.logs[r] = lg;
+          if (site == a.n[r] - 1) {  // chi_r = 1: the single entry is the amplitude
+            a.out[3 * r + 0] = re;
+            a.out[3 * r + 1] = im;
+            a.out[3 * r + 2] = lg;
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+}
+
+int launch_amp_groups(const AmpSiteArgs& a, int dtype, hipStream_t s) {
   if (a.chi_max > AMP_MAX_CHI) {
     set_error("amplitudes: bond dimension above 2048");
     return TENET_ERR_UNSUPPORTED;
   }
-  const dim3 grid((unsigned)((a.chi_max + AS_COLS - 1) / AS_COLS), (unsigned)nreq);
+  int npow = 2;
+  while (npow < a.nreq) npow <<= 1;
+  hipLaunchKernelGGL(amp_check_kernel, dim3((unsigned)a.nreq), dim3(64), 0, s, a);
+  TENET_HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(amp_group_kernel, dim3((unsigned)a.n_max), dim3(AG_THREADS), (size_t)npow * 16, s, a, npow,
+                     dtype == TENET_C128 ? 16 : 8);
+  TENET_HIP_CHECK(hipGetLastError());
+  return TENET_OK;
+}
+
+int launch_amp_site(const AmpSiteArgs& a, int64_t site, int dtype, hipStream_t s, hipEvent_t e0, hipEvent_t e1) {
+  // enough tile rows for requests of one state with two basis values; with
+  // more distinct slices the workgroups take further tiles in turn
+  const unsigned gy = (unsigned)((a.nreq + 7) / 8 + 1);
+  const dim3 grid((unsigned)((a.chi_max + AT_COLS - 1) / AT_COLS), gy), block(64 * AT_WAVES);
   if (dtype == TENET_C128) {
     if (e0)
-      hipExtLaunchKernelGGL(amp_site_kernel<double2>, grid, dim3(AS_THREADS), 0, s, e0, e1, 0, a, site);
+      hipExtLaunchKernelGGL(amp_tile_kernel<double2>, grid, block, 0, s, e0, e1, 0, a, site);
     else
-      hipLaunchKernelGGL(amp_site_kernel<double2>, grid, dim3(AS_THREADS), 0, s, a, site);
+      hipLaunchKernelGGL(amp_tile_kernel<double2>, grid, block, 0, s, a, site);
   } else {
     if (e0)
-      hipExtLaunchKernelGGL(amp_site_kernel<float2>, grid, dim3(AS_THREADS), 0, s, e0, e1, 0, a, site);
+      hipExtLaunchKernelGGL(amp_tile_kernel<float2>, grid, block, 0, s, e0, e1, 0, a, site);
     else
-      hipLaunchKernelGGL(amp_site_kernel<float2>, grid, dim3(AS_THREADS), 0, s, a, site);
+      hipLaunchKernelGGL(amp_tile_kernel<float2>, grid, block, 0, s, a, site);
   }
   TENET_HIP_CHECK(hipGetLastError());
   return TENET_OK;

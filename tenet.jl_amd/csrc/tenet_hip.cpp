@@ -1806,24 +1806,37 @@ extern "C" int tenet_amplitudes_sites(tenet_ctx ctx, tenet_stream stream, int dt
   CHECK_ARG(n_dev && site_ptrs_dev && chis_dev && bits_dev && out, "null pointer");
   CHECK_ARG(nreq <= 65535, "more than 65535 requests in one call");
   hipStream_t s = pick(ctx, stream);
+  // slices of requests, one after the other: 2048 of them fill the chip at
+  // every site position, and the order tables stay small
+  const int64_t nr = std::min(nreq, AMP_SLICE), nt = n_max * nr;
   void* w = nullptr;
-  const size_t vb = align_up((size_t)nreq * 4 * chi_max * sizeof(double), 256);
-  TRY(ws_get(ctx, s, vb + align_up((size_t)nreq * sizeof(double), 256), &w));
+  const size_t need = align_up((size_t)nr * 4 * chi_max * sizeof(double), 256) + align_up((size_t)nr * 8, 256) +
+                      align_up((size_t)nt * 8, 256) + align_up((size_t)nt * sizeof(AmpTile), 256) +
+                      align_up((size_t)nr * 4, 256);
+  TRY(ws_get(ctx, s, need, &w));
+  Bump bm(w);
   AmpSiteArgs a{};
-  a.n = n_dev;
-  a.sites = site_ptrs_dev;
-  a.chis = chis_dev;
-  a.bits = bits_dev;
   a.d = d;
   a.chi_max = chi_max;
   a.n_max = n_max;
-  a.vbuf = static_cast<double*>(w);
-  a.logs = reinterpret_cast<double*>(static_cast<char*>(w) + vb);
-  a.out = out;
-  for (int64_t i = 0; i < n_max; ++i) {
-    StatScope st(ctx, s, TENET_KSTAT_AMPLITUDE, 0.0, 0.0, true);
-    TRY(launch_amp_site(a, nreq, i, dtype, s, st.start_event(), st.stop_event()));
-    st.launched();
+  a.vbuf = (double*)bm.take((size_t)nr * 4 * chi_max * sizeof(double));
+  a.logs = (double*)bm.take((size_t)nr * 8);
+  a.vmax = (unsigned long long*)bm.take((size_t)nt * 8);
+  a.tiles = (AmpTile*)bm.take((size_t)nt * sizeof(AmpTile));
+  a.valid = (int32_t*)bm.take((size_t)nr * 4);
+  for (int64_t r0 = 0; r0 < nreq; r0 += nr) {
+    a.n = n_dev + r0;
+    a.sites = site_ptrs_dev + r0;
+    a.chis = chis_dev + r0;
+    a.bits = bits_dev + r0;
+    a.out = out + 3 * r0;
+    a.nreq = std::min(nr, nreq - r0);
+    TRY(launch_amp_groups(a, dtype, s));
+    for (int64_t i = 0; i < n_max; ++i) {
+      StatScope st(ctx, s, TENET_KSTAT_AMPLITUDE, 0.0, 0.0, true);
+      TRY(launch_amp_site(a, i, dtype, s, st.start_event(), st.stop_event()));
+      st.launched();
+    }
   }
   return TENET_OK;
 }
