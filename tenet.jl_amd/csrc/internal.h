@@ -224,8 +224,9 @@ int launch_fill_zero(void* dst, size_t bytes, hipStream_t s);
 int launch_absorb(const void* U, int64_t m, const void* Vh, int64_t ldvh, int64_t n, const double* S,
                   const int64_t* k_dev, int absorb, void* Aout, void* Bout, int64_t kmax, int dtype,
                   hipStream_t s);
-// scale by 1/max|x| and accumulate log(max) into acc[2]; optionally mantissa out
-int launch_rescale_log(void* x, int64_t count, double* acc, int dtype, hipStream_t s);
+// scale by 1/max|x| and accumulate log(max) into acc[2]; slot: a zeroed device
+// word for this call
+int launch_rescale_log(void* x, int64_t count, double* acc, unsigned long long* slot, int dtype, hipStream_t s);
 // site-parallel amplitudes (k_misc.hip): device tables as for
 // launch_amplitudes for up to AMP_SLICE requests at a time, the chi_max / n_max / d
 // bounds and workspace (per request two vector rows of 2 chi_max doubles and

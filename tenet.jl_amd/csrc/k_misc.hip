@@ -118,11 +118,61 @@ __global__ __launch_bounds__(1024) void rescale_log_kernel(S2* __restrict__ x, i
   }
 }
 
-int launch_rescale_log(void* x, int64_t count, double* acc, int dtype, hipStream_t s) {
-  if (dtype == TENET_C128)
-    hipLaunchKernelGGL(rescale_log_kernel<double2>, dim3(1), dim3(1024), 0, s, (double2*)x, count, acc);
-  else
-    hipLaunchKernelGGL(rescale_log_kernel<float2>, dim3(1), dim3(1024), 0, s, (float2*)x, count, acc);
+// The same over many workgroups, for arrays one workgroup would stream alone
+// (90000 complex64 entries: 46 us): the largest component into *slot (zero
+// before), then the scaling.
+template <typename S2>
+__global__ __launch_bounds__(256) void env_max_kernel(const S2* __restrict__ x, int64_t count,
+                                                      unsigned long long* slot) {
+  __shared__ double red[4];
+  const int tid = threadIdx.x;
+  double mx = 0.0;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + tid; i < count; i += (int64_t)gridDim.x * 256) {
+    const S2 v = x[i];
+    mx = fmax(mx, fmax(fabs((double)v.x), fabs((double)v.y)));
+  }
+  mx = wave_max(mx);
+  if ((tid & 63) == 0) red[tid >> 6] = mx;
+  __syncthreads();
+  // nonnegative doubles order like their bits
+  if (tid == 0)
+    atomicMax(slot, (unsigned long long)__double_as_longlong(fmax(fmax(red[0], red[1]), fmax(red[2], red[3]))));
+}
+template <typename S2>
+__global__ __launch_bounds__(256) void env_scale_kernel(S2* __restrict__ x, int64_t count,
+                                                        const unsigned long long* __restrict__ slot, double* acc) {
+  const double m = __longlong_as_double((long long)*slot);
+  if (!(m > 0.0)) return;
+  const double inv = 1.0 / m;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < count; i += (int64_t)gridDim.x * 256) {
+    S2 v = x[i];
+    v.x = (double)v.x * inv;
+    v.y = (double)v.y * inv;
+    x[i] = v;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) acc[2] += log(m);
+}
+
+// slot: a zeroed word for this call, used above RESCALE_ONE entries
+int launch_rescale_log(void* x, int64_t count, double* acc, unsigned long long* slot, int dtype, hipStream_t s) {
+  // one workgroup takes 4 entries per thread in ~4 us, two launches ~6 us at any size here
+  constexpr int64_t RESCALE_ONE = 4096;
+  if (count <= RESCALE_ONE) {
+    if (dtype == TENET_C128)
+      hipLaunchKernelGGL(rescale_log_kernel<double2>, dim3(1), dim3(1024), 0, s, (double2*)x, count, acc);
+    else
+      hipLaunchKernelGGL(rescale_log_kernel<float2>, dim3(1), dim3(1024), 0, s, (float2*)x, count, acc);
+    TENET_HIP_CHECK(hipGetLastError());
+    return TENET_OK;
+  }
+  const dim3 grid((unsigned)std::min<int64_t>((count + 1023) / 1024, 1024));
+  if (dtype == TENET_C128) {
+    hipLaunchKernelGGL(env_max_kernel<double2>, grid, dim3(256), 0, s, (const double2*)x, count, slot);
+    hipLaunchKernelGGL(env_scale_kernel<double2>, grid, dim3(256), 0, s, (double2*)x, count, slot, acc);
+  } else {
+    hipLaunchKernelGGL(env_max_kernel<float2>, grid, dim3(256), 0, s, (const float2*)x, count, slot);
+    hipLaunchKernelGGL(env_scale_kernel<float2>, grid, dim3(256), 0, s, (float2*)x, count, slot, acc);
+  }
   TENET_HIP_CHECK(hipGetLastError());
   return TENET_OK;
 }

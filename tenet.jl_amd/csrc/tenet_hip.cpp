@@ -1752,10 +1752,14 @@ extern "C" int tenet_overlap(tenet_ctx ctx, tenet_stream stream, int dtype, int 
   for (int64_t i = 0; i <= n; ++i) max_env = std::max(max_env, chi_a[i] * chi_b[i]);
   for (int64_t i = 0; i < n; ++i) max_t = std::max(max_t, chi_b[i] * d * chi_a[i + 1]);
   void* w = nullptr;
-  TRY(ws_get(ctx, s, 2 * align_up((size_t)max_env * es, 256) + align_up((size_t)max_t * es, 256) + 256, &w));
+  TRY(ws_get(ctx, s,
+             2 * align_up((size_t)max_env * es, 256) + align_up((size_t)max_t * es, 256) + align_up((size_t)n * 8, 256) + 256,
+             &w));
   Bump bm(w);
   void* env[2] = {bm.take((size_t)max_env * es), bm.take((size_t)max_env * es)};
   void* T = bm.take((size_t)max_t * es);
+  auto* slots = (unsigned long long*)bm.take((size_t)n * 8);  // one per site's rescale
+  TRY(launch_fill_zero(slots, (size_t)n * 8, s));
   TRY(launch_fill_zero(out, 3 * sizeof(double), s));
   int cur = 0;
   // site 0: env(ra, rb) = sum_s A(1, s, ra) conj(B(1, s, rb))
@@ -1764,7 +1768,7 @@ extern "C" int tenet_overlap(tenet_ctx ctx, tenet_stream stream, int dtype, int 
     const tenet_tdesc dB = mkdesc({1, d, chi_b[1]}, {100, 3, 5});
     const tenet_tdesc dE = mkdesc({1, chi_a[1], chi_b[1]}, {100, 4, 5});
     TRY(einsum_internal(ctx, s, dtype, prec, dA, a_sites[0], dB, b_sites[0], dE, env[cur], 0, 1));
-    TRY(launch_rescale_log(env[cur], chi_a[1] * chi_b[1], out, dtype, s));
+    TRY(launch_rescale_log(env[cur], chi_a[1] * chi_b[1], out, slots, dtype, s));
   }
   for (int64_t i = 1; i < n; ++i) {
     const int64_t la = chi_a[i], lb = chi_b[i], ra = chi_a[i + 1], rb = chi_b[i + 1];
@@ -1778,7 +1782,7 @@ extern "C" int tenet_overlap(tenet_ctx ctx, tenet_stream stream, int dtype, int 
     const tenet_tdesc dE2 = mkdesc({ra, rb}, {4, 5});
     TRY(einsum_internal(ctx, s, dtype, prec, dT, T, dB, b_sites[i], dE2, env[cur ^ 1], 0, 1));
     cur ^= 1;
-    TRY(launch_rescale_log(env[cur], ra * rb, out, dtype, s));
+    TRY(launch_rescale_log(env[cur], ra * rb, out, slots + i, dtype, s));
   }
   return launch_write_scalar_from(env[cur], out, dtype, s);
 }
@@ -1853,11 +1857,15 @@ static int env_sweep(tenet_ctx ctx, hipStream_t s, int dtype, int prec, int64_t 
   for (int64_t j = 0; j <= w; ++j) max_env = std::max(max_env, chi[start + j] * chi[start + j]);
   for (int64_t j = 0; j < w; ++j) max_site = std::max(max_site, chi[start + j] * d * chi[start + j + 1]);
   void* wsp = nullptr;
-  TRY(ws_get(ctx, s, 2 * align_up((size_t)max_env * es, 256) + 2 * align_up((size_t)max_site * es, 256) + 256, &wsp));
+  TRY(ws_get(ctx, s, 2 * align_up((size_t)max_env * es, 256) + 2 * align_up((size_t)max_site * es, 256) +
+                      align_up((size_t)w * 8, 256) + 256,
+             &wsp));
   Bump bm(wsp);
   void* env[2] = {bm.take((size_t)max_env * es), bm.take((size_t)max_env * es)};
   void* PA = bm.take((size_t)max_site * es);
   void* T = bm.take((size_t)max_site * es);
+  auto* slots = (unsigned long long*)bm.take((size_t)w * 8);  // one per site's rescale
+  TRY(launch_fill_zero(slots, (size_t)w * 8, s));
   TRY(launch_fill_zero(out, 3 * sizeof(double), s));
   int cur = 0;
   const int64_t c0 = chi[start];
@@ -1883,7 +1891,7 @@ static int env_sweep(tenet_ctx ctx, hipStream_t s, int dtype, int prec, int64_t 
     const tenet_tdesc dE2 = mkdesc({r, r}, {5, 4});
     TRY(einsum_internal(ctx, s, dtype, prec, dA, sites[i], dT, T, dE2, env[cur ^ 1], 1, 0));
     cur ^= 1;
-    TRY(launch_rescale_log(env[cur], r * r, out, dtype, s));
+    TRY(launch_rescale_log(env[cur], r * r, out, slots + j, dtype, s));
     if (env_each && env_each[j + 1])
       TENET_HIP_CHECK(hipMemcpyAsync(env_each[j + 1], env[cur], (size_t)r * r * es, hipMemcpyDeviceToDevice, s));
     if (log_each)
