@@ -15,6 +15,7 @@
 #include "../../include/tenet_hip.h"
 #include "internal.h"
 
+#include <algorithm>
 #include <utility>
 
 namespace tenet {
@@ -558,7 +559,8 @@ __global__ __launch_bounds__(QP3_THREADS) void qr_panel_v3_kernel(double* __rest
 // column j, which the then idle wave j + 1 assembles one step later
 // (T(a, j) = -tau_j sum_{c=a}^{j-1} T(a, c) w_c, T(j, j) = tau_j: zlarft's
 // forward columnwise rule).  One barrier per column; the outputs are those of
-// qr_panel_v3_kernel.
+// qr_panel_v3_kernel.  src: the panel's columns (panel rows, leading dimension
+// lds), in W or in LDS.
 template <int RL>
 __device__ __forceinline__ void qp4_reflector(double (&ar)[RL], double (&ai)[RL], int jj, int lane,
                                               double2 (*Vs)[64 * RL], double2* taus, double* __restrict__ tau,
@@ -625,8 +627,8 @@ __device__ __forceinline__ void qp4_tcol(int jj, int lane, const double2* taus, 
 }
 
 template <int RL>
-__device__ __forceinline__ void qp4_panel(double* __restrict__ W, double* __restrict__ tau, double* __restrict__ Tout,
-                                          int m, int j0, int jb) {
+__device__ __forceinline__ void qp4_panel(double* W, double* __restrict__ tau, double* __restrict__ Tout,
+                                          int m, int j0, int jb, const double2* src, int lds) {
   __shared__ double2 Vs[2][64 * RL];  // reflector j in Vs[j & 1], panel rows
   __shared__ double2 taus[QB];
   __shared__ double2 Ws[2][QB];    // w_c = v_c^H v_j by the parity of j
@@ -640,7 +642,7 @@ __device__ __forceinline__ void qp4_panel(double* __restrict__ W, double* __rest
   for (int r = 0; r < RL; ++r) {  // branch-free: lanes outside the panel read element 0 and drop it
     const int row = lane + 64 * r;
     const bool ok = wave < jb && row < mr;
-    const double2 v = Wc[ok ? (size_t)(j0 + wave) * m + j0 + row : 0];
+    const double2 v = src[ok ? (size_t)wave * lds + row : 0];
     ar[r] = ok ? v.x : 0.0;
     ai[r] = ok ? v.y : 0.0;
   }
@@ -721,7 +723,7 @@ __device__ __forceinline__ void qp4_panel(double* __restrict__ W, double* __rest
 template <int RL>
 __global__ __launch_bounds__(64 * QB) void qr_panel_v4_kernel(double* __restrict__ W, double* __restrict__ tau,
                                                              double* __restrict__ Tout, int m, int j0, int jb) {
-  qp4_panel<RL>(W, tau, Tout, m, j0, jb);
+  qp4_panel<RL>(W, tau, Tout, m, j0, jb, reinterpret_cast<const double2*>(W) + (size_t)j0 * m + j0, m);
 }
 
 // Panel p of every problem of a batch (one workgroup per problem; problems
@@ -731,68 +733,18 @@ __global__ __launch_bounds__(64 * QB) void qr_panel_v4_batched_kernel(const QrBa
   const QrBatchProb& q = probs[blockIdx.x];
   const int k = min(q.m, q.n), j0 = p * QB;
   if (j0 >= k) return;
-  qp4_panel<RL>(q.W, q.tau, q.T + (size_t)p * QB * QB * 2, q.m, j0, min(QB, k - j0));
-}
-
-// Q (m x k) = [I; 0] in FP64
-__global__ void qr_eye_kernel(double* __restrict__ Q, int m, int k) {
-  const size_t total = (size_t)m * k;
-  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x) {
-    const int r = (int)(e % m), c = (int)(e / m);
-    double2 v;
-    v.x = (r == c) ? 1.0 : 0.0;
-    v.y = 0.0;
-    reinterpret_cast<double2*>(Q)[e] = v;
-  }
-}
-
-// Copy Q (FP64, m x k) and R (upper triangle of W) to the outputs
-template <typename S2>
-__global__ void qr_store_kernel(const double* __restrict__ W, const double* __restrict__ Q, int m, int n, void* Qout,
-                                int64_t ldq, void* Rout, int64_t ldr, int flags) {
-  const int k = min(m, n);
-  const size_t nq = (size_t)m * k, nr = (size_t)k * n;
-  const bool qadj = (flags & TENET_QR_Q_ADJ) != 0, radj = (flags & TENET_QR_R_ADJ) != 0;
-  S2* Qo = static_cast<S2*>(Qout);
-  S2* Ro = static_cast<S2*>(Rout);
-  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < nq + nr; e += (size_t)gridDim.x * blockDim.x) {
-    if (e < nq) {
-      const int r = (int)(e % m), c = (int)(e / m);
-      const double2 v = reinterpret_cast<const double2*>(Q)[e];
-      S2 o;
-      o.x = v.x;
-      o.y = qadj ? -v.y : v.y;
-      if (qadj)
-        Qo[(size_t)r * ldq + c] = o;
-      else
-        Qo[(size_t)c * ldq + r] = o;
-    } else {
-      const size_t f = e - nq;
-      const int r = (int)(f % k), c = (int)(f / k);
-      double2 v;
-      v.x = 0.0;
-      v.y = 0.0;
-      if (r <= c) v = reinterpret_cast<const double2*>(W)[(size_t)c * m + r];
-      S2 o;
-      o.x = v.x;
-      o.y = radj ? -v.y : v.y;
-      if (radj)
-        Ro[(size_t)r * ldr + c] = o;
-      else
-        Ro[(size_t)c * ldr + r] = o;
-    }
-  }
+  qp4_panel<RL>(q.W, q.tau, q.T + (size_t)p * QB * QB * 2, q.m, j0, min(QB, k - j0),
+                reinterpret_cast<const double2*>(q.W) + (size_t)j0 * q.m + j0, q.m);
 }
 
 bool qr_blocked_fits(int64_t m) { return m <= QP_MAX_ROWS; }
 
-// Row-chunked application of one block reflector, M <- (I - V T' V^H) M on
-// rows [j0, m) and columns [col_begin, col_end): two launches, each with a
-// workgroup per (16-column block, 64-row chunk), so a 512-row update runs on
-// 8x the workgroups of the one-pass kernel above.
+// Row-chunked application of one block reflector on a batch of matrices,
+// M <- (I - V T^H V^H) M on rows [j0, m) and columns [col_begin, col_end), a
+// workgroup per (16-column block, 64-row chunk):
 //   phase Y: Ypart[chunk][block] = V[chunk]^H M[chunk, block]   (16 x 16)
-//   phase X: Z = T' sum_chunks Ypart (each workgroup, fixed order);
-//            M[chunk, block] -= V[chunk] Z
+//   phase Z: Z = T^H sum_chunks Ypart, once per column block
+//   phase X: M[chunk, block] -= V[chunk] Z
 constexpr int QA_RC = 64;
 
 __device__ __forceinline__ void qa_load_v(const double2* __restrict__ Wc, int m, int j0, int jb, int rb, int rows,
@@ -896,95 +848,6 @@ __device__ __forceinline__ void qa_y_body(const double* __restrict__ W, const do
     out[2 * e] = yred[0][e][0] + yred[1][e][0] + yred[2][e][0] + yred[3][e][0];
     out[2 * e + 1] = yred[0][e][1] + yred[1][e][1] + yred[2][e][1] + yred[3][e][1];
   }
-}
-
-__global__ __launch_bounds__(QR_THREADS) void qr_apply_y_kernel(const double* __restrict__ W,
-                                                                 const double* __restrict__ M, double* __restrict__ Yp,
-                                                                 int m, int ldm, int j0, int jb, int col_begin,
-                                                                 int col_end) {
-  qa_y_body(W, M, Yp, m, ldm, j0, jb, col_begin, col_end, blockIdx.x, blockIdx.y, gridDim.x);
-}
-
-__device__ __forceinline__ void qa_x_body(const double* __restrict__ W, const double* __restrict__ T,
-                                          const double* __restrict__ Yp, double* __restrict__ M, int m, int ldm,
-                                          int j0, int jb, int col_begin, int col_end, int nchunks, int adj, int blk,
-                                          int chunk, int nblk) {
-  __shared__ double vr[QA_RC][QB + 1], vi[QA_RC][QB + 1];
-  __shared__ double yr[QB][QB + 1], yi[QB][QB + 1];
-  __shared__ double zr[QB][QB + 1], zi[QB][QB + 1];
-  const int tid = threadIdx.x;
-  const int cb0 = col_begin + blk * QB;
-  const int nc = min(QB, col_end - cb0);
-  const int rb = j0 + chunk * QA_RC;
-  const int rows = min(QA_RC, m - rb);
-  if (nc <= 0 || rows <= 0) return;
-  const double2* Wc = reinterpret_cast<const double2*>(W);
-  double2* Mc = reinterpret_cast<double2*>(M);
-  qa_load_v(Wc, m, j0, jb, rb, rows, vr, vi);
-  {
-    // Y = sum over chunks (fixed order), one entry per thread
-    const int a = tid / QB, c = tid % QB;
-    double sr = 0.0, si = 0.0;
-    for (int ch = 0; ch < nchunks; ++ch) {
-      const double* in = Yp + ((size_t)ch * nblk + blk) * QB * QB * 2;
-      sr += in[2 * (a * QB + c)];
-      si += in[2 * (a * QB + c) + 1];
-    }
-    yr[a][c] = sr;
-    yi[a][c] = si;
-  }
-  __syncthreads();
-  {
-    // Z = T' Y
-    const int a = tid / QB, c = tid % QB;
-    double sr = 0.0, si = 0.0;
-    for (int b = 0; b < jb; ++b) {
-      double tr, ti;
-      if (adj) {
-        tr = T[2 * (a * QB + b)];
-        ti = -T[2 * (a * QB + b) + 1];
-      } else {
-        tr = T[2 * (b * QB + a)];
-        ti = T[2 * (b * QB + a) + 1];
-      }
-      sr += tr * yr[b][c] - ti * yi[b][c];
-      si += tr * yi[b][c] + ti * yr[b][c];
-    }
-    zr[a][c] = (a < jb) ? sr : 0.0;
-    zi[a][c] = (a < jb) ? si : 0.0;
-  }
-  __syncthreads();
-  // M[chunk rows] -= V Z: thread owns row tid % 64 and 4 columns
-  const int rsub = tid % QA_RC, cq = 4 * (tid / QA_RC);
-  if (rsub < rows) {
-    double sr[4] = {0, 0, 0, 0}, si[4] = {0, 0, 0, 0};
-#pragma unroll
-    for (int b = 0; b < QB; ++b) {
-      const double pr = vr[rsub][b], pi = vi[rsub][b];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        sr[j] += pr * zr[b][cq + j] - pi * zi[b][cq + j];
-        si[j] += pr * zi[b][cq + j] + pi * zr[b][cq + j];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      if (cq + j < nc) {
-        double2 x = Mc[(size_t)(cb0 + cq + j) * ldm + rb + rsub];
-        x.x -= sr[j];
-        x.y -= si[j];
-        Mc[(size_t)(cb0 + cq + j) * ldm + rb + rsub] = x;
-      }
-    }
-  }
-}
-
-__global__ __launch_bounds__(QR_THREADS) void qr_apply_x_kernel(const double* __restrict__ W,
-                                                                 const double* __restrict__ T,
-                                                                 const double* __restrict__ Yp, double* __restrict__ M,
-                                                                 int m, int ldm, int j0, int jb, int col_begin,
-                                                                 int col_end, int nchunks, int adj) {
-  qa_x_body(W, T, Yp, M, m, ldm, j0, jb, col_begin, col_end, nchunks, adj, blockIdx.x, blockIdx.y, gridDim.x);
 }
 
 // Batched form: Z = T^H sum_chunks Ypart formed once per (problem, column
@@ -1443,21 +1306,6 @@ __global__ __launch_bounds__(QR_THREADS, 2) void qr_wfused_batched_kernel(const 
   }
 }
 
-// M <- (I - V T' V^H) M (adj = 1: T' = T^H, forward application during the
-// factorisation; adj = 0: T' = T, backward accumulation of Q)
-static int qr_apply_chunked(const double* W, const double* T, double* M, int m, int ldm, int j0, int jb, int c_begin,
-                            int c_end, int adj, double* Yp, hipStream_t s) {
-  if (c_end <= c_begin || m <= j0) return TENET_OK;
-  const unsigned nblk = (unsigned)((c_end - c_begin + QB - 1) / QB);
-  const unsigned nch = (unsigned)((m - j0 + QA_RC - 1) / QA_RC);
-  hipLaunchKernelGGL(qr_apply_y_kernel, dim3(nblk, nch), dim3(QR_THREADS), 0, s, W, M, Yp, m, ldm, j0, jb, c_begin,
-                     c_end);
-  TENET_HIP_CHECK(hipGetLastError());
-  hipLaunchKernelGGL(qr_apply_x_kernel, dim3(nblk, nch), dim3(QR_THREADS), 0, s, W, T, Yp, M, m, ldm, j0, jb, c_begin,
-                     c_end, (int)nch, adj);
-  TENET_HIP_CHECK(hipGetLastError());
-  return TENET_OK;
-}
 
 // Householder QR of every problem of a batch in place (R on and above the
 // diagonal of W, the reflectors below; tau and the panels' T factors kept):
@@ -1523,9 +1371,7 @@ int launch_qr_batched(const QrBatchProb* probs, int64_t nprob, int max_m, int ma
 size_t qr_blocked_ws_bytes(int64_t m, int64_t n) {
   const int64_t k = std::min(m, n);
   const int64_t np = (k + QB - 1) / QB;
-  const int64_t ych = (m + QA_RC - 1) / QA_RC, yblk = (std::max(n, k) + QB - 1) / QB;
-  return (size_t)m * n * 16 + (size_t)m * k * 16 + (size_t)k * 16 + (size_t)np * QB * QB * 16 +
-         (size_t)ych * yblk * QB * QB * 16 + 2048;
+  return (size_t)m * n * 16 + (size_t)k * 16 + (size_t)np * QB * QB * 16 + 2048;
 }
 
 // ---------------------------------------------------------------------------
@@ -1881,55 +1727,378 @@ int launch_qr_small(const void* A, int64_t lda, int64_t m, int64_t n, void* Qout
 
 // W (m x n, FP64 complex, already packed) -> Q, R outputs.  Workspace after W:
 // Q scratch (m x k), tau (k), T blocks.
-int launch_qr_blocked(double* W, int64_t m, int64_t n, void* Qout, int64_t ldq, void* Rout, int64_t ldr, int dtype,
-                      int flags, hipStream_t s) {
-  const int64_t k = std::min(m, n);
-  const int64_t np = (k + QB - 1) / QB;
-  double* Q = W + (size_t)m * n * 2;
-  double* tau = Q + (size_t)m * k * 2;
-  double* Tb = tau + (size_t)k * 2;
-  double* Yp = Tb + (size_t)np * QB * QB * 2;  // chunk partials of V^H M
-  for (int64_t p = 0; p < np; ++p) {
-    const int j0 = (int)(p * QB), jb = (int)std::min<int64_t>(QB, k - j0);
-    double* Tp = Tb + (size_t)p * QB * QB * 2;
-    const int mr = (int)m - j0;
-    if (mr <= 64)
-      hipLaunchKernelGGL(qr_panel_v4_kernel<1>, dim3(1), dim3(64 * QB), 0, s, W, tau, Tp, (int)m, j0, jb);
-    else if (mr <= 128)
-      hipLaunchKernelGGL(qr_panel_v4_kernel<2>, dim3(1), dim3(64 * QB), 0, s, W, tau, Tp, (int)m, j0, jb);
-    else if (mr <= 256)
-      hipLaunchKernelGGL(qr_panel_v4_kernel<4>, dim3(1), dim3(64 * QB), 0, s, W, tau, Tp, (int)m, j0, jb);
-    else if (mr <= 512)
-      hipLaunchKernelGGL(qr_panel_v4_kernel<8>, dim3(1), dim3(64 * QB), 0, s, W, tau, Tp, (int)m, j0, jb);
-    else
-      hipLaunchKernelGGL(qr_panel_v3_kernel<4>, dim3(1), dim3(QP3_THREADS), 0, s, W, tau, Tb + (size_t)p * QB * QB * 2,
-                         (int)m, j0, jb);
-    TENET_HIP_CHECK(hipGetLastError());
-    const int cb = j0 + jb;
-    if (cb < n) {
-      const int st = qr_apply_chunked(W, Tb + (size_t)p * QB * QB * 2, W, (int)m, (int)m, j0, jb, cb, (int)n, 1, Yp, s);
-      if (st != TENET_OK) return st;
+// ---- one matrix: a launch per panel, and one for Q ----------------------------
+// The 16 x 16 x 4 FP64 MFMA leaves row 4 r + l / 16, column l % 16 of its result
+// in register r of lane l, which is the layout its B operand wants for the
+// contracted index 4 r + l / 16.  So a 16-column block C of the matrix sits in
+// the accumulators of a workgroup's 16 waves (row block b in wave b mod 16)
+// and serves as the operand of Y = V^H C as it is; Z = T' Y (16 x 16, summed
+// over the waves through LDS) serves the same way in C -= V Z.  One pass of V
+// from memory per product, C never leaves the registers.  A panel of 16
+// columns is one launch (29 us at 256 rows, 36 at 320, 39 at 512, of which the
+// 16 dependent columns take 20..25) and Q one more, where a launch for Y and
+// one for C per panel and product took 15 us each: 320 x 160 505 -> 384 us,
+// 256 x 256 733 -> 474, 512 x 256 891 -> 784, 100 x 70 204 -> 113.
+constexpr int QS_WAVES = 16;
+
+struct QsShared {
+  double2 part[QS_WAVES][QB][QB];  // [wave][a][c]
+  double2 y[QB][QB];
+  double2 z[QB][QB];
+  double2 t[QB][QB];  // T' as t[a][b]
+};
+
+// V(row, a) of the panel at j0 (jb columns): unit lower trapezoid
+__device__ __forceinline__ double2 qs_v(const double2* W, int m, int j0, int jb, int row, int a) {
+  const bool in = a < jb && row > j0 + a && row < m;
+  const double2 v = W[in ? (size_t)(j0 + a) * m + row : 0];
+  double2 o;
+  o.x = in ? v.x : (a < jb && row == j0 + a ? 1.0 : 0.0);
+  o.y = in ? v.y : 0.0;
+  return o;
+}
+
+// T' = T^H (adj) or T into LDS
+__device__ __forceinline__ void qs_load_t(const double* __restrict__ T, bool adj, QsShared& sm) {
+  const int tid = threadIdx.x;
+  if (tid < QB * QB) {
+    const int a = tid / QB, b = tid % QB;
+    const double2 v = reinterpret_cast<const double2*>(T)[adj ? a * QB + b : b * QB + a];
+    sm.t[a][b] = make_double2(v.x, adj ? -v.y : v.y);
+  }
+}
+
+// Y += V^H C for the 16 rows from r0 (PRE: all of V's entries loaded ahead of
+// the products; a wave holding four row blocks has no registers for that)
+template <bool PRE>
+__device__ __forceinline__ void qs_dot(const double2* W, int m, int j0, int jb, int r0, const qr_d4v& cr,
+                                       const qr_d4v& ci, qr_d4v& yr, qr_d4v& yi) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  double2 v[4];
+  if constexpr (PRE) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = qs_v(W, m, j0, jb, r0 + 4 * q + g, l16);
+  }
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if constexpr (!PRE) {
+      v[q] = qs_v(W, m, j0, jb, r0 + 4 * q + g, l16);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    yr = qr_mfma(v[q].x, cr[q], yr);
+    yi = qr_mfma(v[q].x, ci[q], yi);
+    yr = qr_mfma(v[q].y, ci[q], yr);
+    yi = qr_mfma(-v[q].y, cr[q], yi);
+  }
+}
+
+// Z = T' (sum of the waves' Y) into LDS
+__device__ __forceinline__ void qs_z(QsShared& sm, const qr_d4v& yr, const qr_d4v& yi) {
+  const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+#pragma unroll
+  for (int q = 0; q < 4; ++q) sm.part[wave][4 * q + g][l16] = make_double2(yr[q], yi[q]);
+  __syncthreads();
+  const int a = tid / QB, c = tid % QB;
+  if (tid < QB * QB) {
+    double sr = 0.0, si = 0.0;
+#pragma unroll
+    for (int w = 0; w < QS_WAVES; ++w) {
+      const double2 p = sm.part[w][a][c];
+      sr += p.x;
+      si += p.y;
+    }
+    sm.y[a][c] = make_double2(sr, si);
+  }
+  __syncthreads();
+  if (tid < QB * QB) {
+    double sr = 0.0, si = 0.0;
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      const double2 t = sm.t[a][b], y = sm.y[b][c];
+      sr = fma(t.x, y.x, fma(-t.y, y.y, sr));
+      si = fma(t.x, y.y, fma(t.y, y.x, si));
+    }
+    sm.z[a][c] = make_double2(sr, si);
+  }
+  __syncthreads();
+}
+
+// C -= V Z for the 16 rows from r0; V Z is summed on its own and subtracted
+// once: one rounding at C's scale
+template <bool PRE>
+__device__ __forceinline__ void qs_sub(const double2* W, int m, int j0, int jb, int r0, const double2 (&z)[4],
+                                       qr_d4v& cr, qr_d4v& ci) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  double2 v[4];
+  if constexpr (PRE) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) v[q] = qs_v(W, m, j0, jb, r0 + l16, 4 * q + g);
+  }
+  qr_d4v tr = {0, 0, 0, 0}, ti = {0, 0, 0, 0};
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    if constexpr (!PRE) {
+      v[q] = qs_v(W, m, j0, jb, r0 + l16, 4 * q + g);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    tr = qr_mfma(v[q].x, z[q].x, tr);
+    ti = qr_mfma(v[q].x, z[q].y, ti);
+    tr = qr_mfma(-v[q].y, z[q].y, tr);
+    ti = qr_mfma(v[q].y, z[q].x, ti);
+  }
+  cr -= tr;
+  ci -= ti;
+}
+
+// C <- (I - V T' V^H) C; cr / ci: row blocks rb0 + wave + 16 i of the 16
+// columns, blocks above the panel untouched.  Ends with a barrier (the shared
+// buffers may be reused).
+template <int NB>
+__device__ __forceinline__ void qs_apply(const double2* W, int m, int j0, int jb, const double* __restrict__ T,
+                                         bool adj, int rb0, QsShared& sm, qr_d4v (&cr)[NB], qr_d4v (&ci)[NB]) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  qs_load_t(T, adj, sm);
+  qr_d4v yr = {0, 0, 0, 0}, yi = {0, 0, 0, 0};
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int r0 = 16 * (rb0 + wave + QS_WAVES * i);
+    if (r0 < m && r0 + 15 >= j0) qs_dot<(NB < 4)>(W, m, j0, jb, r0, cr[i], ci[i], yr, yi);  // uniform across the wave
+  }
+  qs_z(sm, yr, yi);
+  double2 z[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) z[q] = sm.z[4 * q + g][l16];
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    const int r0 = 16 * (rb0 + wave + QS_WAVES * i);
+    if (r0 < m && r0 + 15 >= j0) qs_sub<(NB < 4)>(W, m, j0, jb, r0, z, cr[i], ci[i]);
+  }
+  __syncthreads();
+}
+
+// Apply reflector block [j0, j0 + jb) to the 16 columns from c0 (rows from
+// j0).  With cols set, rows from j1 on of the first keep columns go there
+// (cols[c * ldc + row - j1]) instead of back to W.
+template <int NB>
+__device__ __forceinline__ void qs_update_columns(double2* W, int m, int n, int j0, int jb, const double* T, int c0,
+                                                  QsShared& sm, double2* cols, int ldc, int keep, int j1) {
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rb0 = j0 / 16, col = c0 + l16;
+  qr_d4v cr[NB], ci[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int row = 16 * (rb0 + wave + QS_WAVES * i) + 4 * q + g;
+      const bool in = row < m && col < n;
+      const double2 v = W[in ? (size_t)col * m + row : 0];
+      cr[i][q] = in ? v.x : 0.0;
+      ci[i][q] = in ? v.y : 0.0;
+    }
+  qs_apply<NB>(W, m, j0, jb, T, true, rb0, sm, cr, ci);
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int row = 16 * (rb0 + wave + QS_WAVES * i) + 4 * q + g;
+      if (row < m && col < n) {
+        const double2 v = make_double2(cr[i][q], ci[i][q]);
+        if (cols && row >= j1 && l16 < keep)
+          cols[l16 * ldc + row - j1] = v;
+        else
+          W[(size_t)col * m + row] = v;
+      }
+    }
+}
+
+// Panel p done: workgroup 0 brings the next panel's columns up to date and
+// factors them, the others update the columns right of it.  The chain of
+// panels is the critical path (16 dependent columns each); the rest of the
+// trailing update hides behind it.  The updated panel goes to the
+// factorisation through LDS (in the buffers of the update, done by then).
+template <int RL>
+__global__ __launch_bounds__(64 * QB) void qr_step_kernel(double* W, double* tau, double* Tb, int m, int n, int k,
+                                                          int p) {
+  constexpr int NB = (4 * RL + 1 + QS_WAVES - 1) / QS_WAVES;  // row blocks per wave for 64 RL + 16 rows
+  constexpr int LDC = 64 * RL + 1;
+  constexpr size_t BYTES = std::max(sizeof(QsShared), (size_t)QB * LDC * sizeof(double2));
+  __shared__ __align__(16) char buf[BYTES];
+  QsShared& sm = *reinterpret_cast<QsShared*>(buf);
+  double2* cols = reinterpret_cast<double2*>(buf);
+  const int j0 = p * QB, j1 = j0 + QB;  // a next panel exists: this one is full
+  const double* T = Tb + (size_t)p * QB * QB * 2;
+  const bool next = blockIdx.x == 0;
+  const int jb1 = min(QB, k - j1);
+  qs_update_columns<NB>(reinterpret_cast<double2*>(W), m, n, j0, QB, T, j1 + (int)blockIdx.x * QB, sm,
+                        next ? cols : nullptr, LDC, jb1, j1);
+  if (next) {
+    __syncthreads();
+    qp4_panel<RL>(W, tau, Tb + (size_t)(p + 1) * QB * QB * 2, m, j1, jb1, cols, LDC);
+  }
+}
+
+// The update alone: panels taller than the step kernel's, and the columns
+// right of the last panel.  Any number of row blocks per wave, each read
+// again for its update.
+__global__ __launch_bounds__(64 * QB) void qr_update_kernel(double* Wd, const double* Tb, int m, int n, int p, int jb,
+                                                            int c0) {
+  __shared__ QsShared sm;
+  double2* W = reinterpret_cast<double2*>(Wd);
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j0 = p * QB, col = c0 + (int)blockIdx.x * QB + l16;
+  qs_load_t(Tb + (size_t)p * QB * QB * 2, true, sm);
+  auto load = [&](int r0, qr_d4v& cr, qr_d4v& ci) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int row = r0 + 4 * q + g;
+      const bool in = row < m && col < n;
+      const double2 v = W[in ? (size_t)col * m + row : 0];
+      cr[q] = in ? v.x : 0.0;
+      ci[q] = in ? v.y : 0.0;
+    }
+  };
+  qr_d4v yr = {0, 0, 0, 0}, yi = {0, 0, 0, 0}, cr, ci;
+  for (int r0 = j0 + 16 * wave; r0 < m; r0 += 16 * QS_WAVES) {
+    load(r0, cr, ci);
+    qs_dot<true>(W, m, j0, jb, r0, cr, ci, yr, yi);
+  }
+  qs_z(sm, yr, yi);
+  double2 z[4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) z[q] = sm.z[4 * q + g][l16];
+  for (int r0 = j0 + 16 * wave; r0 < m; r0 += 16 * QS_WAVES) {
+    load(r0, cr, ci);
+    qs_sub<true>(W, m, j0, jb, r0, z, cr, ci);
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int row = r0 + 4 * q + g;
+      if (row < m && col < n) W[(size_t)col * m + row] = make_double2(cr[q], ci[q]);
     }
   }
+}
+
+// Q = H_1 ... H_k [I; 0]: the 16-column blocks are independent, and block j
+// only meets the panels j, j - 1, ..., 0, so one workgroup takes a block
+// through all of them in registers.  Workgroups from nq on write R.
+template <typename S2, int NB>
+__global__ __launch_bounds__(64 * QB) void qr_form_kernel(const double* Wd, const double* __restrict__ Tb, int m, int n,
+                                                          int k, int nq, void* Qout, int64_t ldq, void* Rout,
+                                                          int64_t ldr, int flags) {
+  __shared__ QsShared sm;
+  const double2* W = reinterpret_cast<const double2*>(Wd);
+  if ((int)blockIdx.x >= nq) {
+    const bool radj = (flags & TENET_QR_R_ADJ) != 0;
+    S2* Ro = static_cast<S2*>(Rout);
+    const size_t nr = (size_t)k * n, step = (size_t)(gridDim.x - nq) * blockDim.x;
+    for (size_t f = (size_t)(blockIdx.x - nq) * blockDim.x + threadIdx.x; f < nr; f += step) {
+      const int r = (int)(f % k), c = (int)(f / k);
+      double2 v = make_double2(0.0, 0.0);
+      if (r <= c) v = W[(size_t)c * m + r];
+      S2 o;
+      o.x = v.x;
+      o.y = radj ? -v.y : v.y;
+      Ro[radj ? (size_t)r * ldr + c : (size_t)c * ldr + r] = o;
+    }
+    return;
+  }
+  // the blocks with the most panels first
+  const int jblk = nq - 1 - (int)blockIdx.x;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int col = jblk * QB + l16;
+  qr_d4v cr[NB], ci[NB];
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      cr[i][q] = 16 * (wave + QS_WAVES * i) + 4 * q + g == col ? 1.0 : 0.0;
+      ci[i][q] = 0.0;
+    }
+  for (int p = jblk; p >= 0; --p)
+    qs_apply<NB>(W, m, p * QB, min(QB, k - p * QB), Tb + (size_t)p * QB * QB * 2, false, 0, sm, cr, ci);
+  const bool qadj = (flags & TENET_QR_Q_ADJ) != 0;
+  S2* Qo = static_cast<S2*>(Qout);
+#pragma unroll
+  for (int i = 0; i < NB; ++i)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int row = 16 * (wave + QS_WAVES * i) + 4 * q + g;
+      if (row < m && col < k) {
+        S2 o;
+        o.x = cr[i][q];
+        o.y = qadj ? -ci[i][q] : ci[i][q];
+        Qo[qadj ? (size_t)row * ldq + col : (size_t)col * ldq + row] = o;
+      }
+    }
+}
+
+template <typename S2>
+static void launch_qr_form(const double* W, const double* Tb, int m, int n, int k, int np, void* Q, int64_t ldq,
+                           void* R, int64_t ldr, int flags, hipStream_t s) {
+  const unsigned nr = (unsigned)std::max<int64_t>(1, std::min<int64_t>(((int64_t)k * n + 4095) / 4096, 64));
+  const dim3 grid((unsigned)np + nr), block(64 * QB);
+  if (m <= 256)
+    hipLaunchKernelGGL((qr_form_kernel<S2, 1>), grid, block, 0, s, W, Tb, m, n, k, np, Q, ldq, R, ldr, flags);
+  else if (m <= 512)
+    hipLaunchKernelGGL((qr_form_kernel<S2, 2>), grid, block, 0, s, W, Tb, m, n, k, np, Q, ldq, R, ldr, flags);
+  else
+    hipLaunchKernelGGL((qr_form_kernel<S2, 4>), grid, block, 0, s, W, Tb, m, n, k, np, Q, ldq, R, ldr, flags);
+}
+
+int launch_qr_blocked(double* W, int64_t m64, int64_t n64, void* Qout, int64_t ldq, void* Rout, int64_t ldr, int dtype,
+                      int flags, hipStream_t s) {
+  const int m = (int)m64, n = (int)n64, k = std::min(m, n), np = (k + QB - 1) / QB;
+  double* tau = W + (size_t)m * n * 2;
+  double* Tb = tau + (size_t)k * 2;
+  // the first panel, then one launch per further panel
   {
-    const size_t total = (size_t)m * k;
-    const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>((total + 255) / 256, 4096));
-    hipLaunchKernelGGL(qr_eye_kernel, dim3(g), dim3(256), 0, s, Q, (int)m, (int)k);
+    const int jb = std::min(QB, k);
+    if (m <= 64)
+      hipLaunchKernelGGL(qr_panel_v4_kernel<1>, dim3(1), dim3(64 * QB), 0, s, W, tau, Tb, m, 0, jb);
+    else if (m <= 128)
+      hipLaunchKernelGGL(qr_panel_v4_kernel<2>, dim3(1), dim3(64 * QB), 0, s, W, tau, Tb, m, 0, jb);
+    else if (m <= 256)
+      hipLaunchKernelGGL(qr_panel_v4_kernel<4>, dim3(1), dim3(64 * QB), 0, s, W, tau, Tb, m, 0, jb);
+    else if (m <= 512)
+      hipLaunchKernelGGL(qr_panel_v4_kernel<8>, dim3(1), dim3(64 * QB), 0, s, W, tau, Tb, m, 0, jb);
+    else
+      hipLaunchKernelGGL(qr_panel_v3_kernel<4>, dim3(1), dim3(QP3_THREADS), 0, s, W, tau, Tb, m, 0, jb);
     TENET_HIP_CHECK(hipGetLastError());
   }
-  for (int64_t p = np - 1; p >= 0; --p) {
-    const int j0 = (int)(p * QB), jb = (int)std::min<int64_t>(QB, k - j0);
-    const int st = qr_apply_chunked(W, Tb + (size_t)p * QB * QB * 2, Q, (int)m, (int)m, j0, jb, j0, (int)k, 0, Yp, s);
-    if (st != TENET_OK) return st;
+  for (int p = 0; p + 1 < np; ++p) {
+    const int j1 = (p + 1) * QB, mr = m - j1;
+    const dim3 grid((unsigned)((n - j1 + QB - 1) / QB)), block(64 * QB);
+    if (mr <= 64)
+      hipLaunchKernelGGL(qr_step_kernel<1>, grid, block, 0, s, W, tau, Tb, m, n, k, p);
+    else if (mr <= 128)
+      hipLaunchKernelGGL(qr_step_kernel<2>, grid, block, 0, s, W, tau, Tb, m, n, k, p);
+    else if (mr <= 256)
+      hipLaunchKernelGGL(qr_step_kernel<4>, grid, block, 0, s, W, tau, Tb, m, n, k, p);
+    else if (mr <= 512)
+      hipLaunchKernelGGL(qr_step_kernel<8>, grid, block, 0, s, W, tau, Tb, m, n, k, p);
+    else {
+      // more than 512 rows: the panel's rows do not fit the 16-wave kernel
+      hipLaunchKernelGGL(qr_update_kernel, grid, block, 0, s, W, Tb, m, n, p, QB, j1);
+      TENET_HIP_CHECK(hipGetLastError());
+      hipLaunchKernelGGL(qr_panel_v3_kernel<4>, dim3(1), dim3(QP3_THREADS), 0, s, W, tau,
+                         Tb + (size_t)(p + 1) * QB * QB * 2, m, j1, std::min(QB, k - j1));
+    }
+    TENET_HIP_CHECK(hipGetLastError());
   }
-  const size_t total = (size_t)m * k + (size_t)k * n;
-  const unsigned g = (unsigned)std::max<size_t>(1, std::min<size_t>((total + 255) / 256, 4096));
+  const int jl = (np - 1) * QB, jbl = k - jl;
+  if (k < n) {  // columns right of the last panel (m < n: at most 16 rows are left)
+    const dim3 grid((unsigned)((n - k + QB - 1) / QB)), block(64 * QB);
+    hipLaunchKernelGGL(qr_update_kernel, grid, block, 0, s, W, Tb, m, n, np - 1, jbl, k);
+    TENET_HIP_CHECK(hipGetLastError());
+  }
   if (dtype == TENET_C128)
-    hipLaunchKernelGGL(qr_store_kernel<double2>, dim3(g), dim3(256), 0, s, W, Q, (int)m, (int)n, Qout, ldq, Rout, ldr,
-                       flags);
+    launch_qr_form<double2>(W, Tb, m, n, k, np, Qout, ldq, Rout, ldr, flags, s);
   else
-    hipLaunchKernelGGL(qr_store_kernel<float2>, dim3(g), dim3(256), 0, s, W, Q, (int)m, (int)n, Qout, ldq, Rout, ldr,
-                       flags);
+    launch_qr_form<float2>(W, Tb, m, n, k, np, Qout, ldq, Rout, ldr, flags, s);
   TENET_HIP_CHECK(hipGetLastError());
   return TENET_OK;
 }
