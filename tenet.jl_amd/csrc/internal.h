@@ -159,11 +159,12 @@ int launch_qr_blocked(double* W, int64_t m, int64_t n, void* Qout, int64_t ldq, 
 // ---- K3: one-sided block Jacobi SVD -----------------------------------------
 struct SvdProblem {
   double* X;      // nr x ncp work matrix (complex, column-major)
+  double* X2;     // second X buffer of rounds that split a pair's rows (NULL: none do)
   double* V;      // ncp x ncp accumulated rotations
   double* Gpart;  // npairs * q partial Gram blocks (2b x 2b complex)
   double* sigma;  // ncp
   int32_t* perm;  // ncp
-  int32_t* flag;  // [0] rotated in this sweep, [1] converged, [2] sweeps; flag + 4: the sweep's max squared relative off-diagonal (double)
+  int32_t* flag;  // [0] rotated in this sweep, [1] converged, [2] sweeps, [3] an off-diagonal of this sweep above sqrt(tol) / 2 relative
   double* fro2;   // ||A||_F^2 (absolute rotation floor eps^2 * ||A||_F^2)
   int32_t nr, ncols, ncp, b, nblk, q;
   int32_t m, n, transposed;
@@ -190,12 +191,13 @@ struct SvdProblem {
   int32_t pad1;
 };
 // Problems are passed either as a device array (grouped) or inline (one).
-// units (grouped rounds): when set, a one-dimensional grid whose workgroup i
-// takes (problem, pair) = units[i] instead of (blockIdx.y, blockIdx.x)
+// units (grouped rounds): when set, workgroup i takes units[i] = {problem (-1:
+// nothing), pair, chunk | chunks << 16, bit 0: X is read from X2, bit 1: X is
+// written to X2}
 struct SvdBatch {
   const SvdProblem* arr;
   SvdProblem one;
-  const int2* units;
+  const int4* units;
 };
 int launch_svd_init(const SvdBatch& b, int64_t nprob, int64_t max_elems, int max_ncp, int dtype, hipStream_t s);
 // ev0 / ev1 (optional): stamped at the kernel's start and end by the dispatch

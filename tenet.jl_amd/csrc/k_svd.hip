@@ -11,10 +11,12 @@
 // applied to the pair's columns of X and V.  At convergence X = U diag(s),
 // A = X V^H.  All rotations, Gram sums and norms are FP64.
 //
-// Each pair may be split over q workgroups by rows (phase 0: partial Gram
-// per row chunk; phase 1: every workgroup of the pair sums the q partials in
-// a fixed order, solves the same 2b x 2b problem, and rotates its own row
-// chunk).  With q = 1 the two phases fuse (phase 2).
+// A round is one launch (phase 2): a pair is one workgroup, or q workgroups that
+// each form its Gram, solve the same 2b x 2b problem and rotate their share of
+// the rows.  One tall matrix (above 768 rows, or a single pair) takes two
+// launches: partial Grams per row chunk (phase 0), then every workgroup of the
+// pair sums the q partials in a fixed order, solves and rotates its own row
+// chunk (phase 1).
 #include <hip/hip_ext.h>
 
 #include "../../include/tenet_hip.h"
@@ -30,6 +32,8 @@ constexpr int SR_THREADS = 512;
 constexpr int B2MAX = 32;  // 2b
 constexpr int RS = 64;     // staged rows per LDS pass
 constexpr int SORT_MAX = 4096;
+constexpr int GT = 8;      // rows of a wave's Gram tile
+constexpr int GT_LD = 34;  // its leading dimension: 16 lanes' 16-byte writes and reads meet in no LDS bank
 
 __device__ __forceinline__ int circle_pos(int i, int r, int nb) {
   return i == 0 ? 0 : 1 + ((i - 1 + r) % (nb - 1));
@@ -45,17 +49,16 @@ struct SvSmem {
       double xr[RS][B2MAX + 1];
       double xi[RS][B2MAX + 1];
     };
+    double2 tile[SR_THREADS / 64][GT][GT_LD];  // per wave: rows of the pair on their way into MFMA operands
     struct {  // second Gram buffer of the inner solve
       double hr[B2MAX][B2MAX + 1];
       double hi[B2MAX][B2MAX + 1];
     };
   };
-  double rc[B2MAX / 2], rsr[B2MAX / 2], rsi[B2MAX / 2];
-  int rp[B2MAX / 2], rq[B2MAX / 2], ract[B2MAX / 2];
-  double rmax[B2MAX / 2];  // per rotation slot: max |g_pq|^2 / (g_pp g_qq) seen
-  double rcs[SR_THREADS / 64][B2MAX / 2][4];  // per wave, per slot: c, Re s, Im s, (pad)
-  int rpq[SR_THREADS / 64][B2MAX / 2];         // per wave, per slot: rotation active
-  int any_outer;
+  // rotations by slot: [0..1] c, Re s, Im s (and d') by step parity, [2..3] the new diagonal
+  double rcs[4][B2MAX / 2][4];
+  int rpq[2][B2MAX / 2];  // rotation active
+  int any_outer, any_big, need;
 };
 
 __device__ __forceinline__ int pair_col(int l, int I, int J, int b) { return l < b ? I * b + l : J * b + (l - b); }
@@ -202,8 +205,8 @@ __device__ void gram_over_rows(SvSmem& sm, const double* X, int64_t ld, int r0, 
 //   G'[p'][q']             = one entry of J_k1^H B J_k2, B the 2x2 block
 //                            {p_k1, q_k1} x {p_k2, q_k2} of G before step s,
 // all known from G_s and step s's rotations.  Wave 7 (one lane per slot)
-// writes step s's diagonal blocks (closed form) and forms step s + 1's
-// rotations while waves 0-1 update the off-diagonal 2 x 2 blocks (one thread
+// writes the (p, q) entries of step s's slots (closed form; G's diagonal
+// passes through the rotation slots) and forms step s + 1's rotations while waves 0-1 update the off-diagonal 2 x 2 blocks (one thread
 // per block: both output rows) and waves 2-6 rotate W with step s's
 // rotations; the rotations (c, s and the new diagonal) pass through LDS
 // slots double-buffered by step parity.
@@ -228,19 +231,11 @@ typedef double GramRow[B2MAX + 1];
 
 // 1/sqrt(x) for x > 0: hardware estimate and two Newton steps in correction
 // form y <- y + y (1 - x y^2) / 2 (each squares the relative error; the
-// estimate is good to ~2^-23, so two steps reach double precision).
+// estimate is good to ~2^-24, so two steps reach double precision).
 __device__ __forceinline__ double rsqrt_nr(double x) {
   double y = __builtin_amdgcn_rsq(x);
   y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
   y = fma(0.5 * y, fma(-x * y, y, 1.0), y);
-  return y;
-}
-
-// 1/x for x > 0: hardware estimate and two Newton steps y <- y + y (1 - x y)
-__device__ __forceinline__ double rcp_nr(double x) {
-  double y = __builtin_amdgcn_rcp(x);
-  y = fma(y, fma(-x, y, 1.0), y);
-  y = fma(y, fma(-x, y, 1.0), y);
   return y;
 }
 
@@ -264,15 +259,18 @@ __device__ __forceinline__ double from_next_lane(double x) {
 struct Rot {
   double c, sr, si;  // J = [[c, s], [-conj(s), c]]
   double an, dn;     // new diagonal
-  double rel2;       // |g|^2 / (a d), for the convergence test
   int act;
+  int big;  // |g|^2 > big2 a d: the sweep has not converged (compared, not divided: a
+            // reciprocal here would lengthen every step of the inner solve)
 };
 
-__device__ __forceinline__ Rot form_rotation(double ra, double rd, double rxr, double rxi, double tol2, double abs2) {
+__device__ __forceinline__ Rot form_rotation(double ra, double rd, double rxr, double rxi, double tol2, double abs2,
+                                             double big2) {
   Rot o;
   const double g2 = rxr * rxr + rxi * rxi;
   const double ad = fmax(ra, 0.0) * fmax(rd, 0.0);
   o.act = (g2 > tol2 * ad && g2 > abs2) ? 1 : 0;
+  o.big = (g2 > big2 * ad && ad > 0.0) ? 1 : 0;
   o.c = 1.0;
   o.sr = 0.0;
   o.si = 0.0;
@@ -284,36 +282,40 @@ __device__ __forceinline__ Rot form_rotation(double ra, double rd, double rxr, d
     const double v = fma(0.5 * fabs(dl), ir, 0.5);  // c^2
     const double y = rsqrt_nr(v);                   // 1 / c
     o.c = v * y;
-    const double sn = 0.5 * ir * y;
-    const double tg = (0.5 * g2) * (ir * (y * y));
-    const bool pos = dl >= 0.0;
-    o.sr = pos ? sn * rxr : -(sn * rxr);
-    o.si = pos ? sn * rxi : -(sn * rxi);
-    o.an = pos ? ra - tg : ra + tg;
-    o.dn = pos ? rd + tg : rd - tg;
+    const double sn = copysign(0.5 * ir * y, dl);
+    const double tg = copysign((0.5 * g2) * (ir * (y * y)), dl);
+    o.sr = sn * rxr;
+    o.si = sn * rxi;
+    o.an = ra - tg;
+    o.dn = rd + tg;
   }
-  o.rel2 = ad > 0.0 ? g2 * rcp_nr(ad) : 0.0;
   return o;
 }
 
-// row h of B' = J_k^H B J_l for the 2x2 block B = [B0; B1] and the rotations
-// J = [[c, e], [-conj(e), c]]: row h of T = J_k^H B is a B0 + b B1 with
-// (a, b) = (c_k, -e_k) for h = 0 and (conj(e_k), c_k) for h = 1, and row h of
-// B' is (c_l T0 - conj(e_l) T1, e_l T0 + c_l T1).
-__device__ __forceinline__ void block_row(bool h1, double ck, double ekr, double eki, double cl, double elr,
-                                          double eli, const double (&b)[8], double& n0r, double& n0i, double& n1r,
-                                          double& n1i) {
-  const double a_r = h1 ? ekr : ck, a_i = h1 ? -eki : 0.0;
-  const double b_r = h1 ? ck : -ekr, b_i = h1 ? 0.0 : -eki;
+// row H of B' = J_k^H B J_l for the 2x2 block B = [B0; B1] and the rotations
+// J = [[c, e], [-conj(e), c]]: row 0 of T = J_k^H B is c_k B0 - e_k B1, row 1
+// conj(e_k) B0 + c_k B1, and a row of B' is (c_l T0 - conj(e_l) T1,
+// e_l T0 + c_l T1).
+template <int H>
+__device__ __forceinline__ void block_row(double ck, double ekr, double eki, double cl, double elr, double eli,
+                                          const double (&b)[8], double& n0r, double& n0i, double& n1r, double& n1i) {
   // b = {B00 re, im, B01 re, im, B10 re, im, B11 re, im}
-  const double t0r = (a_r * b[0] - a_i * b[1]) + (b_r * b[4] - b_i * b[5]);
-  const double t0i = (a_r * b[1] + a_i * b[0]) + (b_r * b[5] + b_i * b[4]);
-  const double t1r = (a_r * b[2] - a_i * b[3]) + (b_r * b[6] - b_i * b[7]);
-  const double t1i = (a_r * b[3] + a_i * b[2]) + (b_r * b[7] + b_i * b[6]);
-  n0r = cl * t0r - (elr * t1r + eli * t1i);
-  n0i = cl * t0i - (elr * t1i - eli * t1r);
-  n1r = (elr * t0r - eli * t0i) + cl * t1r;
-  n1i = (elr * t0i + eli * t0r) + cl * t1i;
+  double t[4];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    const double xr = b[2 * j], xi = b[2 * j + 1], yr = b[4 + 2 * j], yi = b[5 + 2 * j];
+    if (H == 0) {
+      t[2 * j] = fma(ck, xr, fma(eki, yi, -(ekr * yr)));
+      t[2 * j + 1] = fma(ck, xi, -fma(ekr, yi, eki * yr));
+    } else {
+      t[2 * j] = fma(ck, yr, fma(ekr, xr, eki * xi));
+      t[2 * j + 1] = fma(ck, yi, fma(ekr, xi, -(eki * xr)));
+    }
+  }
+  n0r = fma(cl, t[0], -fma(elr, t[2], eli * t[3]));
+  n0i = fma(cl, t[1], fma(eli, t[2], -(elr * t[3])));
+  n1r = fma(cl, t[2], fma(elr, t[0], -(eli * t[1])));
+  n1i = fma(cl, t[3], fma(elr, t[1], eli * t[0]));
 }
 
 // G entry (r, c), r != c, from the upper triangle (an entry below it is the
@@ -360,8 +362,7 @@ __device__ __forceinline__ void jacobi_inner(SvSmem& sm, int n2, double tol, dou
     sm.wr[i][c] = (i == c && i < n2) ? 1.0 : 0.0;
     sm.wi[i][c] = 0.0;
   }
-  if (tid == 0) sm.any_outer = 0;
-  const double tol2 = tol * tol, abs2 = abs_tol * abs_tol;
+  const double tol2 = tol * tol, abs2 = abs_tol * abs_tol, big2 = 0.25 * tol;
   const bool gwave = wave < 2, wwave = tid >= IW_FIRST && tid < IW_FIRST + IW_THREADS, rwave = wave == IROT_WAVE;
   // G: the npair (npair - 1) / 2 blocks bk < bl in row-major order, one thread each
   int bk = 0, bl = 1;
@@ -392,15 +393,14 @@ __device__ __forceinline__ void jacobi_inner(SvSmem& sm, int n2, double tol, dou
   const int k = rwave ? min(ln, npair - 1) : 0;
   Rot rt;
   double rgr = 0.0, rgi = 0.0;  // G[p_k][q_k] the current rotation was formed from
-  double rmax2 = 0.0;
-  int any = 0;
+  int any = 0, big = 0;
   __syncthreads();
   if (rwave) {
     int p, q;
     circle_pair(k, 0, n2, p, q);
     rgr = sm.gr[p][q];
     rgi = sm.gi[p][q];
-    rt = form_rotation(sm.gr[p][p], sm.gr[q][q], rgr, rgi, tol2, abs2);
+    rt = form_rotation(sm.gr[p][p], sm.gr[q][q], rgr, rgi, tol2, abs2, big2);
     if (rown) {
       sm.rcs[0][k][0] = rt.c;
       sm.rcs[0][k][1] = rt.sr;
@@ -408,7 +408,7 @@ __device__ __forceinline__ void jacobi_inner(SvSmem& sm, int n2, double tol, dou
       sm.rcs[2][k][0] = rt.an;
       sm.rcs[2][k][1] = rt.dn;
       sm.rpq[0][k] = rt.act;
-      rmax2 = fmax(rmax2, rt.rel2);
+      big |= rt.big;
       any |= rt.act;
     }
   }
@@ -431,14 +431,13 @@ __device__ __forceinline__ void jacobi_inner(SvSmem& sm, int n2, double tol, dou
         g_get(cr, ci, q0, q1, b[6], b[7]);
         const double ck = sm.rcs[par][bk][0], ekr = sm.rcs[par][bk][1], eki = sm.rcs[par][bk][2];
         const double cl = sm.rcs[par][bl][0], elr = sm.rcs[par][bl][1], eli = sm.rcs[par][bl][2];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          double n0r, n0i, n1r, n1i;
-          block_row(h != 0, ck, ekr, eki, cl, elr, eli, b, n0r, n0i, n1r, n1i);
-          const int ph = h ? q0 : p0;
-          g_put(nr, ni, ph, p1, n0r, n0i);
-          g_put(nr, ni, ph, q1, n1r, n1i);
-        }
+        double n0r, n0i, n1r, n1i;
+        block_row<0>(ck, ekr, eki, cl, elr, eli, b, n0r, n0i, n1r, n1i);
+        g_put(nr, ni, p0, p1, n0r, n0i);
+        g_put(nr, ni, p0, q1, n1r, n1i);
+        block_row<1>(ck, ekr, eki, cl, elr, eli, b, n0r, n0i, n1r, n1i);
+        g_put(nr, ni, q0, p1, n0r, n0i);
+        g_put(nr, ni, q0, q1, n1r, n1i);
       }
     } else if (wwave) {
       // W <- W J on this thread's elements
@@ -457,14 +456,10 @@ __device__ __forceinline__ void jacobi_inner(SvSmem& sm, int n2, double tol, dou
         sm.wi[row][wq] = (er * pi + ei * pr) + cw * qi;
       }
     } else if (rwave) {
-      // this step's diagonal blocks, then the next step's rotations
+      // the slots' off-diagonal entries of this step, then the next step's rotations
       if (rown) {
         int p, q;
         circle_pair(k, step, n2, p, q);
-        nr[p][p] = rt.an;
-        ni[p][p] = 0.0;
-        nr[q][q] = rt.dn;
-        ni[q][q] = 0.0;
         nr[p][q] = rt.act ? 0.0 : rgr;
         ni[p][q] = rt.act ? 0.0 : rgi;
       }
@@ -483,11 +478,14 @@ __device__ __forceinline__ void jacobi_inner(SvSmem& sm, int n2, double tol, dou
         const double c1 = sm.rcs[par][k1][0], s1r = sm.rcs[par][k1][1], s1i = sm.rcs[par][k1][2];
         const double c2 = sm.rcs[par][k2][0], s2r = sm.rcs[par][k2][1], s2i = sm.rcs[par][k2][2];
         const double an = sm.rcs[2 + par][k1][h1], dn = sm.rcs[2 + par][k2][h2];
-        double n0r, n0i, n1r, n1i;
-        block_row(h1 != 0, c1, s1r, s1i, c2, s2r, s2i, b, n0r, n0i, n1r, n1i);
+        double x0r, x0i, x1r, x1i, y0r, y0i, y1r, y1i;
+        block_row<0>(c1, s1r, s1i, c2, s2r, s2i, b, x0r, x0i, x1r, x1i);
+        block_row<1>(c1, s1r, s1i, c2, s2r, s2i, b, y0r, y0i, y1r, y1i);
+        const double n0r = h1 ? y0r : x0r, n0i = h1 ? y0i : x0i;
+        const double n1r = h1 ? y1r : x1r, n1i = h1 ? y1i : x1i;
         rgr = h2 ? n1r : n0r;
         rgi = h2 ? n1i : n0i;
-        rt = form_rotation(an, dn, rgr, rgi, tol2, abs2);
+        rt = form_rotation(an, dn, rgr, rgi, tol2, abs2, big2);
         if (rown) {
           sm.rcs[par ^ 1][k][0] = rt.c;
           sm.rcs[par ^ 1][k][1] = rt.sr;
@@ -495,220 +493,289 @@ __device__ __forceinline__ void jacobi_inner(SvSmem& sm, int n2, double tol, dou
           sm.rcs[2 + (par ^ 1)][k][0] = rt.an;
           sm.rcs[2 + (par ^ 1)][k][1] = rt.dn;
           sm.rpq[par ^ 1][k] = rt.act;
-          rmax2 = fmax(rmax2, rt.rel2);
+          big |= rt.big;
           any |= rt.act;
         }
       }
     }
     __syncthreads();
   }
-  if (rown) sm.rmax[k] = rmax2;
   if (rown && any) sm.any_outer = 1;
+  if (rown && big) sm.any_big = 1;
   __syncthreads();
 }
 
-// Cross-block inner solve for 2b = 32 (every cross round: a matrix with more
-// than one block pair has b = 16) with the rotations formed one step ahead.
-// In the cross order p_k = k at every step and q_k(s + 1) = q_{k+1}(s)
-// (slots mod 16), so the Gram entries rotation k of step s + 1 needs are
-//   G'[k][k]       = the new diagonal a'_k of rotation k of step s,
-//   G'[q][q]       = the new diagonal d'_{k+1} of rotation k + 1 of step s,
-//   G'[k][q_{k+1}] = row p_k, column q_{k+1} of J_k^H B J_{k+1}, B the 2x2
-//                    block {k, q_k} x {k+1, q_{k+1}} of G before step s,
+// Inner solve for 2b = 32 (every round of a matrix of more than 30 columns), in
+// levels H = h0, 2 h0, .. 16: at level H the 32 columns are 16 / H groups of
+// 2H, and its H steps rotate every column of a group's first half with every
+// one of its second half.  h0 = 16 is the cross-block solve of two 16-column
+// blocks; h0 = 1 visits all 496 pairs once, within the blocks before across
+// them.  Slot k (0..15), j = k mod H, pairs at step s
+//   p_k = 2 (k - j) + j  and  q_k(s) = 2 (k - j) + H + (j + s) mod H,
+// so p_k stays and q_k(s + 1) = q_n(s), n = k - j + (j + 1) mod H the group's
+// next slot.  The entries rotation k of step s + 1 needs are therefore
+//   G'[p][p]   = the new diagonal a'_k of rotation k of step s,
+//   G'[q][q]   = the new diagonal d'_n of rotation n of step s,
+//   G'[p][q_n] = row p, column q_n of J_k^H B J_n, B the 2x2 block
+//                {p_k, q_k} x {p_n, q_n} of G before step s,
 // all known from G_s and step s's rotations.  Wave 7 (lanes 0-15: one slot
 // each) forms them and step s + 1's rotations while 120 threads of waves
 // 0-1 update the G blocks above the diagonal (one 2 x 2 block each, read
 // once; only G's upper triangle is kept, entries below it read as
-// conjugated mirrors) and waves 4-6 rotate W, which
-// they keep in registers, with step s's rotations; the rotations pass
-// through LDS slots double-buffered by step parity, so a step still takes
-// one workgroup barrier.  Wave 7 also writes the diagonal blocks (closed
-// form).
-constexpr int XB = 16;         // b
+// conjugated mirrors) and waves 4-6 rotate W, which they keep in registers,
+// with step s's rotations; the rotations pass through LDS slots
+// double-buffered by step parity, so a step takes one workgroup barrier.
+// Wave 7 also writes the (p, q) entries of the step's slots (closed form); G's
+// diagonal stays in its registers and goes to LDS between levels.
+//
+// The step is wave 7's dependent chain (LDS reads, one row of a block, two
+// reciprocal square roots): ~1000 cycles; the circle order of jacobi_inner,
+// whose slots change partners irregularly, takes 2500.
+constexpr int XB = 16;         // slots
 constexpr int XROT_WAVE = 7;   // rotation wave
 
-__device__ __forceinline__ void jacobi_cross32(SvSmem& sm, double tol, double abs_tol) {
-  const int tid = threadIdx.x, wave = tid >> 6, ln = tid & 63;
-  if (tid == 0) sm.any_outer = 0;
-  const double tol2 = tol * tol, abs2 = abs_tol * abs_tol;
-  // roles (wave-uniform)
-  const bool gwave = wave < 4, wwave = wave >= 4 && wave < XROT_WAVE, rwave = wave == XROT_WAVE;
-  // G: blocks bk < bl in row-major order, one thread each (both output rows:
-  // the 2 x 2 block is read once)
-  int bk = 0, bl = 1;
-  bool gown = false;
-  if (gwave) {
-    const int u = tid;
-    gown = u < XB * (XB - 1) / 2;
-    int rem = gown ? u : 0, k = 0;
-    while (k < XB - 1 && rem >= XB - 1 - k) {
-      rem -= XB - 1 - k;
-      ++k;
+// x of the next slot of the group (lanes of one 16-lane row)
+__device__ __forceinline__ double from_next_slot(double x, int H, int lane) {
+  return H == XB ? from_next_lane(x) : __shfl(x, lane, 64);
+}
+
+//
+// Each role runs its own copy of the loops below (so that its registers are its
+// own), chosen by a scalar branch on the wave's number; every copy passes the
+// same 1 + H barriers a level.
+template <typename Init, typename Step, typename Done>
+__device__ __forceinline__ void level_loops(int h0, Init init, Step step, Done done) {
+  int par = 0;  // the G buffer and rotation slots of the coming step
+#pragma unroll 1
+  for (int H = h0; H <= XB; H <<= 1) {
+    init(H, par);
+    __syncthreads();
+#pragma unroll 1
+    for (int st = 0; st < H; ++st) {
+      step(H, st, par);
+      par ^= 1;
+      __syncthreads();
     }
-    bk = k;
-    bl = k + 1 + rem;
+    done(H);
   }
-  // rotation wave: lane k < 16 owns slot k
-  const int k = ln & (XB - 1), kn = (k + 1) & (XB - 1);
-  // W lives in the registers of waves 4-6: lane k of 16-lane row group wg
-  // (0..11) holds, for rows wg, wg + 12 and wg + 24 (< 32), P = W[row][k]
-  // (slot k's p column is k at every step) and Q = W[row][q_k(step)] with
-  // q_k(s) = 16 + (k + s) mod 16; since q_k(s + 1) = q_{k+1}(s), Q moves
-  // one lane down between steps (a DPP row rotation), and W goes to LDS once
-  // at the end.
-  const int wg = wwave ? ((tid - 4 * 64) >> 4) : 0;
-  double Pr[3], Pi[3], Qr[3], Qi[3];
-#pragma unroll
-  for (int u = 0; u < 3; ++u) {
-    const int row = wg + 12 * u;
-    Pr[u] = row == k ? 1.0 : 0.0;
-    Pi[u] = 0.0;
-    Qr[u] = row == XB + k ? 1.0 : 0.0;
-    Qi[u] = 0.0;
-  }
-  const bool rown = rwave && ln < XB;
-  Rot rt;
-  double gr = 0.0, gi = 0.0;  // G[k][q_k] the current rotation was formed from
-  double rmax2 = 0.0;
-  int any = 0;
-  if (rwave) {
-    const int q = XB + k;
-    gr = sm.gr[k][q];
-    gi = sm.gi[k][q];
-    rt = form_rotation(sm.gr[k][k], sm.gr[q][q], gr, gi, tol2, abs2);
-    if (rown) {
-      sm.rcs[0][k][0] = rt.c;
-      sm.rcs[0][k][1] = rt.sr;
-      sm.rcs[0][k][2] = rt.si;
-      sm.rpq[0][k] = rt.act;
-      rmax2 = fmax(rmax2, rt.rel2);
-      any |= rt.act;
-    }
-  }
-  __syncthreads();
-#pragma unroll 2
-  for (int step = 0; step < XB; ++step) {
-    const int par = step & 1;
-    const GramRow* cr = par ? sm.hr : sm.gr;
-    const GramRow* ci = par ? sm.hi : sm.gi;
-    GramRow* nr = par ? sm.gr : sm.hr;
-    GramRow* ni = par ? sm.gi : sm.hi;
-    if (gwave) {
-      // only the upper triangle of G is kept up to date: an entry below the
-      // diagonal is read as the conjugate of its mirror
-      const int p0 = bk, q0 = XB + ((bk + step) & (XB - 1));
-      const int p1 = bl, q1 = XB + ((bl + step) & (XB - 1));
-      const int qa = min(q0, q1), qb = max(q0, q1);
-      const double qs = q0 <= q1 ? 1.0 : -1.0;
-      double b[8];
-      b[0] = cr[p0][p1];
-      b[1] = ci[p0][p1];
-      b[2] = cr[p0][q1];
-      b[3] = ci[p0][q1];
-      b[4] = cr[p1][q0];
-      b[5] = -ci[p1][q0];
-      b[6] = cr[qa][qb];
-      b[7] = qs * ci[qa][qb];
-      const double ck = sm.rcs[par][bk][0], ekr = sm.rcs[par][bk][1], eki = sm.rcs[par][bk][2];
-      const double cl = sm.rcs[par][bl][0], elr = sm.rcs[par][bl][1], eli = sm.rcs[par][bl][2];
-      if (gown) {
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          double n0r, n0i, n1r, n1i;
-          block_row(h != 0, ck, ekr, eki, cl, elr, eli, b, n0r, n0i, n1r, n1i);
-          if (h == 0) {
+}
+
+__device__ __forceinline__ void jacobi_levels(SvSmem& sm, int h0, double tol, double abs_tol) {
+  const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = tid & 63;
+  const int k = ln & (XB - 1);
+  if (wave < 2) {
+    // G: blocks bk < bl, one thread each (both output rows: the 2 x 2 block is
+    // read once), sixteen threads at one distance d around the circle of slots
+    // (d = 1..7, then half of d = 8): a wave's reads of G then meet in few LDS
+    // banks (32 cycles for the eight reads of a step, 58 in row-major order)
+    const bool own = tid < XB * (XB - 1) / 2;
+    const int i = tid % XB, i2 = (i + 1 + tid / XB) % XB;
+    const int bk = own ? min(i, i2) : 0, bl = own ? max(i, i2) : 1;
+    int jk, jl, p0, p1, h0k, h0l;  // the blocks' columns p and the first of their groups' second halves
+    level_loops(
+        h0,
+        [&](int H, int) {
+          jk = bk & (H - 1);
+          jl = bl & (H - 1);
+          p0 = 2 * bk - jk;
+          p1 = 2 * bl - jl;
+          h0k = p0 - jk + H;
+          h0l = p1 - jl + H;
+        },
+        [&](int H, int step, int par) {
+          const GramRow* cr = par ? sm.hr : sm.gr;
+          const GramRow* ci = par ? sm.hi : sm.gi;
+          GramRow* nr = par ? sm.gr : sm.hr;
+          GramRow* ni = par ? sm.gi : sm.hi;
+          // only the upper triangle of G is kept up to date: an entry below the
+          // diagonal is read as the conjugate of its mirror
+          const int q0 = h0k + ((jk + step) & (H - 1)), q1 = h0l + ((jl + step) & (H - 1));
+          const int qa = min(q0, q1), qb = max(q0, q1), ra = min(q0, p1), rb = max(q0, p1);
+          double b[8];
+          b[0] = cr[p0][p1];
+          b[1] = ci[p0][p1];
+          b[2] = cr[p0][q1];
+          b[3] = ci[p0][q1];
+          b[4] = cr[ra][rb];
+          b[5] = ci[ra][rb];
+          b[6] = cr[qa][qb];
+          b[7] = ci[qa][qb];
+          const double ck = sm.rcs[par][bk][0], ekr = sm.rcs[par][bk][1], eki = sm.rcs[par][bk][2];
+          const double cl = sm.rcs[par][bl][0], elr = sm.rcs[par][bl][1], eli = sm.rcs[par][bl][2];
+          b[5] = q0 <= p1 ? b[5] : -b[5];
+          b[7] = q0 <= q1 ? b[7] : -b[7];
+          if (own) {
+            double n0r, n0i, n1r, n1i;
+            block_row<0>(ck, ekr, eki, cl, elr, eli, b, n0r, n0i, n1r, n1i);
             nr[p0][p1] = n0r;
             ni[p0][p1] = n0i;
             nr[p0][q1] = n1r;
             ni[p0][q1] = n1i;
-          } else {
-            nr[p1][q0] = n0r;
-            ni[p1][q0] = -n0i;
+            block_row<1>(ck, ekr, eki, cl, elr, eli, b, n0r, n0i, n1r, n1i);
+            nr[ra][rb] = n0r;
+            ni[ra][rb] = q0 <= p1 ? n0i : -n0i;
             nr[qa][qb] = n1r;
-            ni[qa][qb] = qs * n1i;
+            ni[qa][qb] = q0 <= q1 ? n1i : -n1i;
           }
-        }
-      }
-    } else if (wwave) {
-      if (step > 0) {
+        },
+        [](int) {});
+  } else if (wave >= 4 && wave < XROT_WAVE) {
+    // W lives in the registers of waves 4-6: lane k of 16-lane row group wg
+    // (0..11) holds, for rows wg, wg + 12 and wg + 24 (< 32), P = W[row][p_k]
+    // and Q = W[row][q_k(step)]; Q moves one slot down between steps, and W
+    // goes through LDS between levels.
+    const int wg = (tid - 4 * 64) >> 4;
+    double Pr[3], Pi[3], Qr[3], Qi[3];
+    level_loops(
+        h0,
+        [&](int H, int) {
+          const int p = 2 * k - (k & (H - 1));
 #pragma unroll
-        for (int u = 0; u < 3; ++u) {
-          Qr[u] = from_next_lane(Qr[u]);
-          Qi[u] = from_next_lane(Qi[u]);
-        }
-      }
-      if (sm.rpq[par][k]) {
-        const double c = sm.rcs[par][k][0], er = sm.rcs[par][k][1], ei = sm.rcs[par][k][2];
+          for (int u = 0; u < 3; ++u) {
+            const int row = wg + 12 * u, r = min(row, 2 * XB - 1);
+            if (H == h0) {
+              Pr[u] = row == p ? 1.0 : 0.0;
+              Pi[u] = 0.0;
+              Qr[u] = row == p + H ? 1.0 : 0.0;
+              Qi[u] = 0.0;
+            } else {  // written by this wave at the level before
+              Pr[u] = sm.wr[r][p];
+              Pi[u] = sm.wi[r][p];
+              Qr[u] = sm.wr[r][p + H];
+              Qi[u] = sm.wi[r][p + H];
+            }
+          }
+        },
+        [&](int H, int step, int par) {
+          // an inactive rotation is c = 1, s = 0
+          const double c = sm.rcs[par][k][0], er = sm.rcs[par][k][1], ei = sm.rcs[par][k][2];
+          if (step > 0) {
+            const int next = (ln & ~(H - 1)) | ((ln + 1) & (H - 1));
 #pragma unroll
-        for (int u = 0; u < 3; ++u) {
-          const double pr = Pr[u], pi = Pi[u], qr = Qr[u], qi = Qi[u];
-          Pr[u] = c * pr - (er * qr + ei * qi);
-          Pi[u] = c * pi - (er * qi - ei * qr);
-          Qr[u] = (er * pr - ei * pi) + c * qr;
-          Qi[u] = (er * pi + ei * pr) + c * qi;
-        }
-      }
-    } else {
-      // rotation wave: this step's diagonal blocks, then the next step's rotations
-      const int q = XB + ((k + step) & (XB - 1));
-      const int qn = XB + ((kn + step) & (XB - 1));
-      const int ka = min(k, kn), kb2 = max(k, kn), qa = min(q, qn), qb = max(q, qn);
-      const double ks = k <= kn ? 1.0 : -1.0, qs = q <= qn ? 1.0 : -1.0;
-      double b[8];
-      b[0] = cr[ka][kb2];
-      b[1] = ks * ci[ka][kb2];
-      b[2] = cr[k][qn];
-      b[3] = ci[k][qn];
-      b[4] = cr[kn][q];
-      b[5] = -ci[kn][q];
-      b[6] = cr[qa][qb];
-      b[7] = qs * ci[qa][qb];
-      if (rown) {
-        const double ogr = rt.act ? 0.0 : gr, ogi = rt.act ? 0.0 : gi;
-        nr[k][k] = rt.an;
-        ni[k][k] = 0.0;
-        nr[q][q] = rt.dn;
-        ni[q][q] = 0.0;
-        nr[k][q] = ogr;
-        ni[k][q] = ogi;
-      }
-      if (step + 1 < XB) {
-        // slot k + 1's rotation and new diagonal d' (lanes 0-15 hold slots 0-15)
-        const double cn = from_next_lane(rt.c), srn = from_next_lane(rt.sr), sin_ = from_next_lane(rt.si);
-        const double dnn = from_next_lane(rt.dn);
-        double n0r, n0i, n1r, n1i;
-        block_row(false, rt.c, rt.sr, rt.si, cn, srn, sin_, b, n0r, n0i, n1r, n1i);
-        gr = n1r;
-        gi = n1i;
-        rt = form_rotation(rt.an, dnn, gr, gi, tol2, abs2);
-        if (rown) {
-          sm.rcs[par ^ 1][k][0] = rt.c;
-          sm.rcs[par ^ 1][k][1] = rt.sr;
-          sm.rcs[par ^ 1][k][2] = rt.si;
-          sm.rpq[par ^ 1][k] = rt.act;
-          rmax2 = fmax(rmax2, rt.rel2);
-          any |= rt.act;
-        }
-      }
-    }
-    __syncthreads();
+            for (int u = 0; u < 3; ++u) {
+              Qr[u] = from_next_slot(Qr[u], H, next);
+              Qi[u] = from_next_slot(Qi[u], H, next);
+            }
+          }
+#pragma unroll
+          for (int u = 0; u < 3; ++u) {
+            const double pr = Pr[u], pi = Pi[u], qr = Qr[u], qi = Qi[u];
+            Pr[u] = c * pr - (er * qr + ei * qi);
+            Pi[u] = c * pi - (er * qi - ei * qr);
+            Qr[u] = (er * pr - ei * pi) + c * qr;
+            Qi[u] = (er * pi + ei * pr) + c * qi;
+          }
+        },
+        [&](int H) {
+          const int j = k & (H - 1), p = 2 * k - j;
+          const int q = p - j + H + ((j + H - 1) & (H - 1));  // q_k of the last step
+#pragma unroll
+          for (int u = 0; u < 3; ++u) {
+            const int row = wg + 12 * u;
+            if (row < 2 * XB) {
+              sm.wr[row][p] = Pr[u];
+              sm.wi[row][p] = Pi[u];
+              sm.wr[row][q] = Qr[u];
+              sm.wi[row][q] = Qi[u];
+            }
+          }
+        });
+  } else if (wave == XROT_WAVE) {
+    // lane k < 16 owns slot k
+    const double tol2 = tol * tol, abs2 = abs_tol * abs_tol, big2 = 0.25 * tol;
+    const bool own = ln < XB;
+    int any = 0, big = 0;
+    Rot rt;
+    double gr, gi;  // G[p_k][q_k] the current rotation was formed from
+    auto put = [&](int par) {
+      if (!own) return;
+      sm.rcs[par][k][0] = rt.c;
+      sm.rcs[par][k][1] = rt.sr;
+      sm.rcs[par][k][2] = rt.si;
+      sm.rcs[par][k][3] = rt.dn;
+      big |= rt.big;
+      any |= rt.act;
+    };
+    level_loops(
+        h0,
+        [&](int H, int par) {
+          const GramRow* cr = par ? sm.hr : sm.gr;
+          const GramRow* ci = par ? sm.hi : sm.gi;
+          const int p = 2 * k - (k & (H - 1)), q = p + H;
+          gr = cr[p][q];
+          gi = ci[p][q];
+          rt = form_rotation(cr[p][p], cr[q][q], gr, gi, tol2, abs2, big2);
+          put(par);
+        },
+        [&](int H, int step, int par) {
+          const GramRow* cr = par ? sm.hr : sm.gr;
+          const GramRow* ci = par ? sm.hi : sm.gi;
+          GramRow* nr = par ? sm.gr : sm.hr;
+          GramRow* ni = par ? sm.gi : sm.hi;
+          const int j = k & (H - 1), jn = (j + 1) & (H - 1), base = 2 * (k - j), kn = k - j + jn;
+          const int p = base + j, pn = base + jn;
+          const int q = base + H + ((j + step) & (H - 1)), qn = base + H + ((j + 1 + step) & (H - 1));
+          const int pa = min(p, pn), pb = max(p, pn), qa = min(q, qn), qb = max(q, qn);
+          // (in a level's last step these feed nothing)
+          double b[8];
+          b[0] = cr[pa][pb];
+          b[1] = ci[pa][pb];
+          b[2] = cr[p][qn];
+          b[3] = ci[p][qn];
+          b[4] = cr[pn][q];
+          b[5] = ci[pn][q];
+          b[6] = cr[qa][qb];
+          b[7] = ci[qa][qb];
+          // the next slot's rotation and new diagonal d'
+          const double cn = sm.rcs[par][kn][0], srn = sm.rcs[par][kn][1], sin_ = sm.rcs[par][kn][2];
+          const double dnn = sm.rcs[par][kn][3];
+          if (own) {
+            nr[p][q] = rt.act ? 0.0 : gr;
+            ni[p][q] = rt.act ? 0.0 : gi;
+          }
+          if (step + 1 < H) {
+            b[1] = p > pn ? -b[1] : b[1];
+            b[5] = -b[5];
+            b[7] = q > qn ? -b[7] : b[7];
+            double n0r, n0i;
+            block_row<0>(rt.c, rt.sr, rt.si, cn, srn, sin_, b, n0r, n0i, gr, gi);
+            rt = form_rotation(rt.an, dnn, gr, gi, tol2, abs2, big2);
+            put(par ^ 1);
+          } else if (own) {
+            nr[p][p] = rt.an;
+            nr[q][q] = rt.dn;
+          }
+        },
+        [](int) {});
+    if (own && any) sm.any_outer = 1;
+    if (own && big) sm.any_big = 1;
+  } else {
+    level_loops(h0, [](int, int) {}, [](int, int, int) {}, [](int) {});
   }
-  if (wwave) {
-    const int q = XB + ((k + XB - 1) & (XB - 1));  // q_k of the last step
-#pragma unroll
-    for (int u = 0; u < 3; ++u) {
-      const int row = wg + 12 * u;
-      if (row < 2 * XB) {
-        sm.wr[row][k] = Pr[u];
-        sm.wi[row][k] = Pi[u];
-        sm.wr[row][q] = Qr[u];
-        sm.wi[row][q] = Qi[u];
-      }
-    }
-  }
-  if (rown) sm.rmax[k] = rmax2;
-  if (rown && any) sm.any_outer = 1;
   __syncthreads();
+}
+
+// The inner solve of a pair visit: a full sweep of its 2b columns (mode 0) or
+// the cross-block rotations only (mode 1: always 2b = 32).  A pair none of
+// whose entries asks for a rotation is left at once (nearly all pairs of the
+// last sweep, where the solve would be half of the round).
+__device__ __forceinline__ void inner_solve(SvSmem& sm, int n2, int mode, double tol, double abs_tol) {
+  const double tol2 = tol * tol, abs2 = abs_tol * abs_tol;
+  if (threadIdx.x == 0) sm.any_outer = sm.any_big = sm.need = 0;
+  __syncthreads();
+  const int h = n2 / 2;
+  for (int e = threadIdx.x; e < (mode == 1 ? h * h : n2 * n2); e += SR_THREADS) {
+    const int i = mode == 1 ? e % h : e % n2, j = mode == 1 ? h + e / h : e / n2;
+    if (i >= j) continue;
+    const double re = sm.gr[i][j], im = sm.gi[i][j], g2 = re * re + im * im;
+    if (g2 > tol2 * (fmax(sm.gr[i][i], 0.0) * fmax(sm.gr[j][j], 0.0)) && g2 > abs2) sm.need = 1;
+  }
+  __syncthreads();
+  if (!sm.need) return;
+  if (n2 == B2MAX)
+    jacobi_levels(sm, mode == 1 ? XB : 1, tol, abs_tol);
+  else
+    jacobi_inner(sm, n2, tol, abs_tol);
 }
 
 // The staged rows [rb, rb + rows) of the pair's columns of M <- M W.  Thread
@@ -768,18 +835,6 @@ __device__ __forceinline__ svd_d4v mfma_f64(double a, double b, svd_d4v c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// All 32 staged columns (zeros beyond 2b and below `rows`), so that the MFMA
-// operands never read stale LDS.
-__device__ __forceinline__ void store_rows_all(SvSmem& sm, const double2 (&v)[STAGE_PER]) {
-#pragma unroll
-  for (int u = 0; u < STAGE_PER; ++u) {
-    const int e = threadIdx.x + u * SR_THREADS;
-    const int r = e % RS, l = e / RS;
-    sm.xr[r][l] = v[u].x;
-    sm.xi[r][l] = v[u].y;
-  }
-}
-
 // Gram G = X^H X of the pair's columns over rows [r0, r1) into sm.gr / sm.gi.
 // With P = Xr^T Xi:  Re G = Xr^T Xr + Xi^T Xi (symmetric), Im G = P - P^T.
 // For a 4-row K step the A operand of X^T and the B operand of X are the same
@@ -789,105 +844,97 @@ __device__ __forceinline__ void store_rows_all(SvSmem& sm, const double2 (&v)[ST
 // S = Xr + Xi and P, since Re G = S^T S - P - P^T; the off-diagonal block
 // three (Gauss): T1 = Xr0^T Xr1, T2 = Xi0^T Xi1 and
 // T3 = (Xr0 + Xi0)^T (Xr1 - Xi1) give Re G(0,1) = T1 + T2 and
-// Im G(0,1) = T1 - T2 - T3.  Each 64-row chunk is cut into four 16-row
-// groups; group g belongs to waves g and g + 4 (the two waves of one SIMD):
-// wave g sums S0^T S0, S1^T S1 and P(0,0), wave g + 4 P(1,1), T1, T2 and T3
-// (seven products per K step on the SIMD).  The groups' partials are added
-// in LDS in a fixed order (1 into 0 and 3 into 2, then 2 into 0:
-// deterministic).
-__device__ void gram_mfma(SvSmem& sm, const double* X, int64_t ld, int r0, int r1, int I, int J, int b) {
+// Im G(0,1) = T1 - T2 - T3.
+//
+// Wave w takes rows 8 w .. 8 w + 7 of each 64: it loads them with eight
+// consecutive rows of a column in eight lanes (an MFMA operand wants sixteen
+// columns in sixteen lanes, which as a load costs 76 cycles instead of 16),
+// turns them round in an LDS tile of its own and forms all seven products, so
+// no barrier falls into the loop; D loads are on their way while one is
+// multiplied (they take 4000 cycles where other XCDs wrote the columns in the
+// round before).  The waves' sums are added in LDS in a fixed order, halving
+// the waves.  A chunk of 64 rows is bound by the products: 1800 cycles of the
+// matrix cores.
+template <int D>
+__device__ __forceinline__ void gram_mfma(SvSmem& sm, const double* X, int64_t ld, int r0, int r1, int I, int J,
+                                          int b) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int grp = wave & 3;
-  const bool hiw = wave >= 4;
   const int kr = lane >> 4, kc = lane & 15;
-  svd_d4v a0 = {0, 0, 0, 0}, a1 = {0, 0, 0, 0}, a2 = {0, 0, 0, 0}, a3 = {0, 0, 0, 0};
-  double2 v[STAGE_PER];
-  load_rows(v, X, ld, r0, min(RS, r1 - r0), I, J, b);
-  for (int rb = r0; rb < r1; rb += RS) {
-    __syncthreads();
-    store_rows_all(sm, v);
-    __syncthreads();
-    if (rb + RS < r1) load_rows(v, X, ld, rb + RS, min(RS, r1 - rb - RS), I, J, b);
+  const int n2 = 2 * b, tr = lane & (GT - 1), tc = lane / GT;
+  const double2* X2 = reinterpret_cast<const double2*>(X);
+  size_t col[4];
 #pragma unroll
-    for (int s = 0; s < RS / 16; ++s) {
-      const int row = grp * (RS / 4) + 4 * s + kr;
-      const double xr0 = sm.xr[row][kc], xi0 = sm.xi[row][kc];
-      const double xr1 = sm.xr[row][16 + kc], xi1 = sm.xi[row][16 + kc];
-      if (!hiw) {
-        const double s0 = xr0 + xi0, s1 = xr1 + xi1;
-        a0 = mfma_f64(s0, s0, a0);
-        a1 = mfma_f64(s1, s1, a1);
-        a2 = mfma_f64(xr0, xi0, a2);
-      } else {
-        a0 = mfma_f64(xr1, xi1, a0);
-        a1 = mfma_f64(xr0, xr1, a1);
-        a2 = mfma_f64(xi0, xi1, a2);
-        a3 = mfma_f64(xr0 + xi0, xr1 - xi1, a3);
+  for (int u = 0; u < 4; ++u) col[u] = (size_t)pair_col(min(tc + GT * u, n2 - 1), I, J, b) * ld;
+  double2(*tile)[GT_LD] = sm.tile[wave];
+  svd_d4v a[7];
+#pragma unroll
+  for (int t = 0; t < 7; ++t) a[t] = svd_d4v{0, 0, 0, 0};
+  double2 v[D][4];
+  const int own = r0 + GT * wave + tr;
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (r0 + d * RS < r1)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) v[d][u] = X2[col[u] + min(own + d * RS, r1 - 1)];
+  for (int r2 = r0; r2 < r1; r2 += D * RS) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int rb = r2 + d * RS, rn = rb + D * RS, row = own + rb - r0;
+      if (rb >= r1) break;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const bool in = row < r1 && tc + GT * u < n2;
+        double2 z = v[d][u];
+        z.x = in ? z.x : 0.0;
+        z.y = in ? z.y : 0.0;
+        tile[tr][tc + GT * u] = z;
+      }
+      if (rn < r1)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[d][u] = X2[col[u] + min(row + D * RS, r1 - 1)];
+#pragma unroll
+      for (int s = 0; s < GT / 4; ++s) {
+        const double2 x0 = tile[4 * s + kr][kc], x1 = tile[4 * s + kr][16 + kc];
+        const double s0 = x0.x + x0.y, s1 = x1.x + x1.y;
+        a[0] = mfma_f64(s0, s0, a[0]);
+        a[1] = mfma_f64(s1, s1, a[1]);
+        a[2] = mfma_f64(x0.x, x0.y, a[2]);
+        a[3] = mfma_f64(x1.x, x1.y, a[3]);
+        a[4] = mfma_f64(x0.x, x1.x, a[4]);
+        a[5] = mfma_f64(x0.y, x1.y, a[5]);
+        a[6] = mfma_f64(s0, x1.x - x1.y, a[6]);
       }
     }
   }
-  // partials through the staging area: slot (pair, wave half) of 4 x 4 x 64
-  double* red = &sm.xr[0][0];
-  const int slot = (grp >> 1) * 2 + (hiw ? 1 : 0);
-  __syncthreads();
-  if (grp & 1) {
+  double* red = reinterpret_cast<double*>(&sm);
+  static_assert(sizeof(SvSmem) >= (SR_THREADS / 128) * 28 * 64 * sizeof(double), "half the waves' sums fit");
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      red[((slot * 4 + 0) * 4 + r) * 64 + lane] = a0[r];
-      red[((slot * 4 + 1) * 4 + r) * 64 + lane] = a1[r];
-      red[((slot * 4 + 2) * 4 + r) * 64 + lane] = a2[r];
-      red[((slot * 4 + 3) * 4 + r) * 64 + lane] = a3[r];
-    }
+  for (int half = SR_THREADS / 128; half > 0; half /= 2) {
+    __syncthreads();
+    if (wave >= half && wave < 2 * half)
+#pragma unroll
+      for (int i = 0; i < 28; ++i) red[((wave - half) * 28 + i) * 64 + lane] = a[i / 4][i % 4];
+    __syncthreads();
+    if (wave < half)
+#pragma unroll
+      for (int i = 0; i < 28; ++i) a[i / 4][i % 4] += red[(wave * 28 + i) * 64 + lane];
   }
-  __syncthreads();
-  if (!(grp & 1)) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      a0[r] += red[((slot * 4 + 0) * 4 + r) * 64 + lane];
-      a1[r] += red[((slot * 4 + 1) * 4 + r) * 64 + lane];
-      a2[r] += red[((slot * 4 + 2) * 4 + r) * 64 + lane];
-      a3[r] += red[((slot * 4 + 3) * 4 + r) * 64 + lane];
-    }
-  }
-  __syncthreads();
-  if (grp == 2) {
-    const int s2 = hiw ? 1 : 0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      red[((s2 * 4 + 0) * 4 + r) * 64 + lane] = a0[r];
-      red[((s2 * 4 + 1) * 4 + r) * 64 + lane] = a1[r];
-      red[((s2 * 4 + 2) * 4 + r) * 64 + lane] = a2[r];
-      red[((s2 * 4 + 3) * 4 + r) * 64 + lane] = a3[r];
-    }
-  }
-  __syncthreads();
-  if (grp == 0) {
-    const int s2 = hiw ? 1 : 0;
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      a0[r] += red[((s2 * 4 + 0) * 4 + r) * 64 + lane];
-      a1[r] += red[((s2 * 4 + 1) * 4 + r) * 64 + lane];
-      a2[r] += red[((s2 * 4 + 2) * 4 + r) * 64 + lane];
-      a3[r] += red[((s2 * 4 + 3) * 4 + r) * 64 + lane];
-    }
+  if (wave == 0) {
     // S^T S of the diagonal blocks and Re G(0,1) (mirrored) into gr, P into
-    // wr (scratch until the inner solve sets W)
+    // wr (scratch until the inner solve sets W); the off-diagonal block of
+    // Im G goes into wr above the diagonal (zeros below), so that
+    // gi = wr - wr^T holds it and its mirror
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int i = 4 * r + kr, j = kc;
-      if (!hiw) {
-        sm.gr[i][j] = a0[r];
-        sm.gr[16 + i][16 + j] = a1[r];
-        sm.wr[i][j] = a2[r];
-      } else {
-        // the off-diagonal block of Im G goes into wr above the diagonal
-        // (zeros below), so that gi = wr - wr^T holds it and its mirror
-        sm.wr[16 + i][16 + j] = a0[r];
-        sm.gr[i][16 + j] = a1[r] + a2[r];
-        sm.gr[16 + j][i] = a1[r] + a2[r];
-        sm.wr[i][16 + j] = a1[r] - a2[r] - a3[r];
-        sm.wr[16 + j][i] = 0.0;
-      }
+      sm.gr[i][j] = a[0][r];
+      sm.gr[16 + i][16 + j] = a[1][r];
+      sm.wr[i][j] = a[2][r];
+      sm.wr[16 + i][16 + j] = a[3][r];
+      sm.gr[i][16 + j] = a[4][r] + a[5][r];
+      sm.gr[16 + j][i] = a[4][r] + a[5][r];
+      sm.wr[i][16 + j] = a[4][r] - a[5][r] - a[6][r];
+      sm.wr[16 + j][i] = 0.0;
     }
   }
   __syncthreads();
@@ -900,71 +947,119 @@ __device__ void gram_mfma(SvSmem& sm, const double* X, int64_t ld, int r0, int r
   __syncthreads();
 }
 
-// Rows [r0, r1) of the pair's columns of M <- M W by MFMA, with no LDS
-// staging: wave w takes the 16-row strips w, w + 8, ... and computes all 32
-// output columns of its strip (two 16-column blocks over K = 32, three real
-// products each, see below).  Its A operands come straight from memory (lane
-// l: row l % 16 of the strip, columns 4s + l / 16: 256 contiguous bytes per
-// column and load), W's from LDS, and the outputs go out from the
-// accumulators (lanes l, l + 16, l + 32, l + 48: four consecutive rows of one
-// column).  A wave reads and writes only its own rows, so the waves run
-// without a barrier.
-__device__ void apply_mfma(SvSmem& sm, double* M, int64_t ld, int r0, int r1, int I, int J, int b) {
-  const int n2 = 2 * b;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int kr = lane >> 4, kc = lane & 15;
-  double2* M2 = reinterpret_cast<double2*>(M);
-  const size_t safe = (size_t)pair_col(0, I, J, b) * ld + r0;  // a valid element (masked loads read it)
-  for (int rs = r0 + 16 * wave; rs < r1; rs += 16 * (SR_THREADS / 64)) {
-    const int row = rs + kc;
-    double2 x[B2MAX / 4];
+// M <- M W by MFMA, with no LDS staging, in strips of 16 rows: one wave takes a
+// strip, X's operands straight from memory (lane l: row l % 16 of the strip,
+// columns 4s + l / 16: 256 contiguous bytes per column and load) and W's from
+// LDS.  The product is formed as W^T X^T, so that an accumulator register too
+// holds sixteen rows of a column in sixteen lanes and is stored as it was
+// loaded (as X W its lanes lie in sixteen columns, and the eight stores of a
+// strip took 76 cycles each of the address unit, together nearly the time of
+// the products).  The strips of X and then, where the rotations are
+// accumulated, those of V are numbered through.
+constexpr int STRIP = 16;
+
+// A strip's first row in the pair's two 16-column blocks.  With b < 16 (one
+// block pair: I = 0, J = 1) the pair's columns are 0 .. 2b - 1, the second block
+// its columns from 16 on.  All members are uniform over the wave.
+struct Strip {
+  const char* src[2];
+  char* dst[2];
+  size_t ld;  // bytes from column to column
+  int rows;     // rows of the strip inside the matrix (16 and more: all)
+};
+
+__device__ __forceinline__ int strip_count(const SvdProblem& P) {
+  return (P.nr + STRIP - 1) / STRIP + (P.accum ? (P.ncp + STRIP - 1) / STRIP : 0);
+}
+
+// strip i of the (rows x n) matrix M going to D
+__device__ __forceinline__ Strip strip_at(const double* M, double* D, int rows, int i, int I, int J, int b) {
+  Strip t;
+  const size_t c0 = (size_t)I * b, c1 = b == 16 ? (size_t)J * 16 : 16;
+  const size_t o0 = (c0 * rows + (size_t)STRIP * i) * sizeof(double2), o1 = (c1 * rows + (size_t)STRIP * i) * sizeof(double2);
+  t.src[0] = reinterpret_cast<const char*>(M) + o0;
+  t.src[1] = reinterpret_cast<const char*>(M) + o1;
+  t.dst[0] = reinterpret_cast<char*>(D) + o0;
+  t.dst[1] = reinterpret_cast<char*>(D) + o1;
+  t.ld = rows * sizeof(double2);
+  t.rows = rows - STRIP * i;
+  return t;
+}
+
+// X's strips may go from one buffer to another; V is rotated in place
+__device__ __forceinline__ Strip strip_of(const SvdProblem& P, const double* Xs, double* Xd, int i, int I, int J) {
+  const int sx = (P.nr + STRIP - 1) / STRIP;
+  return i < sx ? strip_at(Xs, Xd, P.nr, i, I, J, P.b) : strip_at(P.V, P.V, P.ncp, i - sx, I, J, P.b);
+}
+
+// x[s]: row l % 16, column 4s + l / 16 (rows past the matrix: its last row
+// again, never stored; columns past 2b: 0)
+__device__ __forceinline__ void strip_load(double2 (&x)[B2MAX / 4], const Strip& t, int b) {
+  const int lane = threadIdx.x & 63, kr = lane >> 4;
+  const unsigned row = min(lane & 15, t.rows - 1) * (unsigned)sizeof(double2);
 #pragma unroll
-    for (int s = 0; s < B2MAX / 4; ++s) {
-      const int l = 4 * s + kr;
-      const bool ok = row < r1 && l < n2;
-      const double2 v = M2[ok ? (size_t)pair_col(l, I, J, b) * ld + row : safe];
-      x[s].x = ok ? v.x : 0.0;
-      x[s].y = ok ? v.y : 0.0;
+  for (int s = 0; s < B2MAX / 4; ++s) {
+    const bool ok = 4 * s + kr < 2 * b;
+    const size_t off = (ok ? (4 * (s & 3) + kr) * t.ld : 0) + row;
+    const double2 v = *reinterpret_cast<const double2*>((ok ? t.src[s >> 2] : t.src[0]) + off);
+    x[s].x = ok ? v.x : 0.0;
+    x[s].y = ok ? v.y : 0.0;
+  }
+}
+
+// The strip's output columns 16 cb .. 16 cb + 15, cb in [cb0, cb0 + NCB).
+// Three real products per complex one (Gauss):
+//   T1 = Xr Wr, T2 = Xi Wi, T3 = (Xr + Xi)(Wr + Wi);
+//   Re Y = T1 - T2, Im Y = T3 - T1 - T2
+// (W is unitary, so the cancellation in Im Y costs O(eps |X|))
+template <int NCB>
+__device__ __forceinline__ void strip_rotate(const SvSmem& sm, const double2 (&x)[B2MAX / 4], const Strip& t0, int cb0,
+                                             int b) {
+  const int lane = threadIdx.x & 63, kr = lane >> 4, kc = lane & 15;
+  svd_d4v t[NCB][3];
+#pragma unroll
+  for (int cb = 0; cb < NCB; ++cb)
+#pragma unroll
+    for (int u = 0; u < 3; ++u) t[cb][u] = svd_d4v{0, 0, 0, 0};
+#pragma unroll
+  for (int s = 0; s < B2MAX / 4; ++s) {
+    const double xr = x[s].x, xi = x[s].y, xs = xr + xi;
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb) {
+      const int c = 16 * (cb0 + cb) + kc;
+      const double wre = sm.wr[4 * s + kr][c], wim = sm.wi[4 * s + kr][c];
+      t[cb][0] = mfma_f64(wre, xr, t[cb][0]);
+      t[cb][1] = mfma_f64(wim, xi, t[cb][1]);
+      t[cb][2] = mfma_f64(wre + wim, xs, t[cb][2]);
     }
-    // three real products per complex one (Gauss):
-    //   T1 = Xr Wr, T2 = Xi Wi, T3 = (Xr + Xi)(Wr + Wi);
-    //   Re Y = T1 - T2, Im Y = T3 - T1 - T2
-    // (W is unitary, so the cancellation in Im Y costs O(eps |X|))
-    svd_d4v t[2][3];
+  }
+  if (kc >= t0.rows) return;
 #pragma unroll
-    for (int cb = 0; cb < 2; ++cb)
+  for (int cb = 0; cb < NCB; ++cb) {
+    char* dst = cb0 + cb ? t0.dst[1] : t0.dst[0];
 #pragma unroll
-      for (int u = 0; u < 3; ++u) t[cb][u] = svd_d4v{0, 0, 0, 0};
-#pragma unroll
-    for (int s = 0; s < B2MAX / 4; ++s) {
-      const double xr = x[s].x, xi = x[s].y, xs = xr + xi;
-#pragma unroll
-      for (int cb = 0; cb < 2; ++cb) {
-        const double wre = sm.wr[4 * s + kr][16 * cb + kc], wim = sm.wi[4 * s + kr][16 * cb + kc];
-        t[cb][0] = mfma_f64(xr, wre, t[cb][0]);
-        t[cb][1] = mfma_f64(xi, wim, t[cb][1]);
-        t[cb][2] = mfma_f64(xs, wre + wim, t[cb][2]);
-      }
-    }
-#pragma unroll
-    for (int cb = 0; cb < 2; ++cb) {
-      const int l = 16 * cb + kc;
-      if (l < n2) {
-        double2* col = M2 + (size_t)pair_col(l, I, J, b) * ld + rs;
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int rr = 4 * r + kr;
-          if (rs + rr < r1) {
-            double2 o;
-            o.x = t[cb][0][r] - t[cb][1][r];
-            o.y = t[cb][2][r] - t[cb][0][r] - t[cb][1][r];
-            col[rr] = o;
-          }
-        }
+    for (int r = 0; r < 4; ++r) {
+      if (16 * (cb0 + cb) + 4 * r + kr < 2 * b) {
+        double2 o;
+        o.x = t[cb][0][r] - t[cb][1][r];
+        o.y = t[cb][2][r] - t[cb][0][r] - t[cb][1][r];
+        *reinterpret_cast<double2*>(dst + ((4 * r + kr) * t0.ld + kc * sizeof(double2))) = o;
       }
     }
   }
-  __syncthreads();
+}
+
+// strip t's rows of the pair's columns from one buffer to the other (an
+// unrotated pair whose X changes buffers)
+__device__ __forceinline__ void strip_copy(const Strip& t, int b) {
+  const int lane = threadIdx.x & 63, kr = lane >> 4;
+  if ((lane & 15) >= t.rows) return;
+#pragma unroll 1
+  for (int s = 0; s < B2MAX / 4; ++s) {
+    const size_t off = (4 * (s & 3) + kr) * t.ld + (lane & 15) * sizeof(double2);
+    if (4 * s + kr < 2 * b)
+      *reinterpret_cast<double2*>(t.dst[s >> 2] + off) = *reinterpret_cast<const double2*>(t.src[s >> 2] + off);
+  }
 }
 
 // Pair (I, J) of item p in round `round` (mode 0: the fixed pairs (2p, 2p+1);
@@ -983,17 +1078,50 @@ __device__ __forceinline__ void round_pair(int p, int round, int mode, int nb, i
   }
 }
 
-// One round with one workgroup per pair over all rows (the grouped batches
-// and small single problems): the Gram and the rotation of X (and of V when
-// accumulated) on FP64 MFMA, the inner solve as in svd_round_kernel.
+// One round in one launch: the Gram and the rotation of X (and of V when
+// accumulated) on FP64 MFMA, the inner solve between them.
+//
+// A pair is one workgroup, in place, or q workgroups: each forms the whole
+// Gram and solves the same inner problem (the same sums in the same order, so
+// the same W), then rotates its own share of the strips.  As the others may
+// still be reading X for their Gram, X then goes to the problem's second
+// buffer; an unrotated pair is copied there.  The q workgroups of a pair lie
+// eight apart in the grid: on one XCD, whose L2 holds the pair's columns for
+// all of them.  With at most four strips per workgroup each strip goes to two
+// waves, one per 16 output columns, loaded before the inner solve, whose
+// barriers part those loads from the stores of the other wave.
+//
+// Why: with few pairs (one matrix, or the rounds that only the largest
+// problems of a batch reach) a workgroup that rotates all rows of X and V is
+// the whole round: 63 us at 512 rows of each, 30 us cut.  Such a round is a
+// chain: launch 3 us, Gram 8 us at 256 rows (loads, then 2450 cycles per 64
+// rows), inner solve 9 us (a sweep's first, fixed-pair round 17), rotation 2 us
+// (one 256 x 256 matrix: 22.5 us a round; with two launches, the partial Grams
+// on the VALU, it was 36).  With two workgroups on each CU (ALONE = false:
+// 496 pairs of 512 rows, 63 us) the rounds run at 6.3 TB/s over X, read twice
+// and written once, from beyond the L2s.
 // mode 0: full inner sweep on the fixed pairs; mode 1: cross-block inner steps.
-__global__ __launch_bounds__(SR_THREADS, 4) void svd_round_mfma_kernel(SvdBatch Bt, int round, int mode) {
+constexpr int NXCD = 8;
+constexpr unsigned NCU = 256;
+
+template <bool ALONE>
+__global__ __launch_bounds__(SR_THREADS, ALONE ? 2 : 4) void svd_round_mfma_kernel(SvdBatch Bt, int round, int mode) {
   __shared__ SvSmem sm;
-  int prob = blockIdx.y, p = blockIdx.x;
+  int prob = 0, p, c, q, flip;
   if (Bt.units) {
-    const int2 u = Bt.units[blockIdx.x];
+    const int4 u = Bt.units[blockIdx.x];
+    if (u.x < 0) return;  // padding of the list
     prob = u.x;
     p = u.y;
+    c = u.z & 0xffff;
+    q = u.z >> 16;
+    flip = u.w;
+  } else {
+    q = Bt.one.q;
+    const int k = blockIdx.x / NXCD;
+    p = blockIdx.x % NXCD + NXCD * (k / q);
+    c = k % q;
+    flip = q > 1 ? 2 : 0;
   }
   const SvdProblem& P = Bt.arr ? Bt.arr[prob] : Bt.one;
   if (P.flag[1]) return;  // converged
@@ -1003,21 +1131,40 @@ __global__ __launch_bounds__(SR_THREADS, 4) void svd_round_mfma_kernel(SvdBatch 
   int I, J;
   round_pair(p, round, mode, nb, I, J);
   const int b = P.b, n2 = 2 * b;
-  gram_mfma(sm, P.X, P.nr, 0, P.nr, I, J, b);
-  const double abs_tol = fmax(4.930380657631324e-32 * (*P.fro2), 1e-300);
-  if (mode == 1)
-    jacobi_cross32(sm, P.tol, abs_tol);
-  else
-    jacobi_inner(sm, n2, P.tol, abs_tol);
-  if (threadIdx.x == 0) {
-    double mx = 0.0;
-    for (int k = 0; k < n2 / 2; ++k) mx = fmax(mx, sm.rmax[k]);
-    atomicMax(reinterpret_cast<unsigned long long*>(P.flag + 4), (unsigned long long)__double_as_longlong(mx));
+  const double* Xs = (flip & 1) ? P.X2 : P.X;
+  double* Xd = (flip & 2) ? P.X2 : P.X;
+  const double abs_tol = fmax(4.930380657631324e-32 * (*P.fro2), 1e-300), tol = P.tol;
+  gram_mfma<ALONE ? 4 : 2>(sm, Xs, P.nr, 0, P.nr, I, J, b);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int S = strip_count(P);
+  const int lo = (int)((int64_t)c * S / q), hi = (int)((int64_t)(c + 1) * S / q);
+  const bool narrow = ALONE && q > 1 && hi - lo <= SR_THREADS / 128;
+  double2 x[B2MAX / 4];
+  if (narrow && lo + (wave >> 1) < hi) strip_load(x, strip_of(P, Xs, Xd, lo + (wave >> 1), I, J), b);
+  inner_solve(sm, n2, mode, tol, abs_tol);
+  if (threadIdx.x == 0 && c == 0) {
+    if (sm.any_outer) P.flag[0] = 1;
+    if (sm.any_big) P.flag[3] = 1;
   }
-  if (!sm.any_outer) return;  // pair already orthogonal: W = I (uniform branch)
-  if (threadIdx.x == 0) P.flag[0] = 1;
-  apply_mfma(sm, P.X, P.nr, 0, P.nr, I, J, b);
-  if (P.accum) apply_mfma(sm, P.V, P.ncp, 0, P.ncp, I, J, b);
+  const bool still = !sm.any_outer;  // pair already orthogonal: W = I (uniform)
+  if (still) {
+    if (Xs == Xd) return;
+    for (int i = lo + wave; i < hi; i += SR_THREADS / 64) {
+      const Strip t = strip_of(P, Xs, Xd, i, I, J);
+      if (t.src[0] != t.dst[0]) strip_copy(t, b);
+    }
+    return;
+  }
+  if (narrow) {
+    const int i = lo + (wave >> 1);
+    if (i < hi) strip_rotate<1>(sm, x, strip_of(P, Xs, Xd, i, I, J), wave & 1, b);
+    return;
+  }
+  for (int i = lo + wave; i < hi; i += SR_THREADS / 64) {
+    const Strip t = strip_of(P, Xs, Xd, i, I, J);
+    strip_load(x, t, b);
+    strip_rotate<2>(sm, x, t, 0, b);
+  }
 }
 
 // Rounds with each pair split over q workgroups by rows (phase 0: partial
@@ -1111,19 +1258,12 @@ __global__ __launch_bounds__(SR_THREADS) void svd_round_kernel(SvdBatch Bt, int 
   // absolute floor (e.g. eps ||A||_F^2) stops the late small-angle rotations
   // that give one-sided Jacobi its accuracy on small singular values.
   const double abs_tol = fmax(4.930380657631324e-32 * (*P.fro2), 1e-300);
-  if (mode == 1)
-    jacobi_cross32(sm, P.tol, abs_tol);
-  else
-    jacobi_inner(sm, n2, P.tol, abs_tol);
-  // largest squared relative off-diagonal of this pair visit -> the sweep's maximum
-  // (non-negative doubles order like their bit patterns)
+  inner_solve(sm, n2, mode, P.tol, abs_tol);
   if (threadIdx.x == 0 && c == 0) {
-    double mx = 0.0;
-    for (int k = 0; k < n2 / 2; ++k) mx = fmax(mx, sm.rmax[k]);
-    atomicMax(reinterpret_cast<unsigned long long*>(P.flag + 4), (unsigned long long)__double_as_longlong(mx));
+    if (sm.any_outer) P.flag[0] = 1;
+    if (sm.any_big) P.flag[3] = 1;
   }
   if (!sm.any_outer) return;  // pair already orthogonal: W = I (uniform branch)
-  if (threadIdx.x == 0 && c == 0) P.flag[0] = 1;
   apply_rows(sm, P.X, P.nr, r0, r1, I, J, b);
   if (!P.accum) return;
   const int rcv = (P.ncp + q - 1) / q;
@@ -1137,17 +1277,15 @@ __global__ void svd_sweep_end_kernel(SvdBatch Bt, int64_t nprob) {
   if (i >= nprob) return;
   const SvdProblem& P = Bt.arr ? Bt.arr[i] : Bt.one;
   if (P.flag[1]) return;
-  // Converged when a sweep rotated nothing, or when its largest relative
-  // off-diagonal was below sqrt(tol) / 2 (squared: tol / 4): one-sided
+  // Converged when a sweep rotated nothing, or when no relative off-diagonal
+  // of it was above sqrt(tol) / 2 (squared: tol / 4): one-sided
   // Jacobi converges quadratically, so after such a sweep every pair's
   // cosine is ~ that squared, below tol, and the verification sweep would
   // rotate nothing.
-  unsigned long long* om = reinterpret_cast<unsigned long long*>(P.flag + 4);
-  const double mx2 = __longlong_as_double((long long)*om);
-  if (P.flag[0] == 0 || mx2 < 0.25 * P.tol) P.flag[1] = 1;
+  if (P.flag[0] == 0 || P.flag[3] == 0) P.flag[1] = 1;
   P.flag[0] = 0;
   P.flag[2] += 1;
-  *om = 0ull;
+  P.flag[3] = 0;
 }
 
 // X (nr x ncp) from A or A^H with zero padding; V = I.
@@ -1191,7 +1329,7 @@ __global__ void svd_init_kernel(SvdBatch Bt) {
     P.flag[0] = 0;
     P.flag[1] = 0;
     P.flag[2] = 0;
-    *reinterpret_cast<unsigned long long*>(P.flag + 4) = 0ull;
+    P.flag[3] = 0;
   }
 }
 
@@ -1684,12 +1822,16 @@ int launch_svd_round(const SvdBatch& b, int64_t nprob, int max_items, int round,
     return TENET_ERR_UNSUPPORTED;
   }
   // with a unit list, max_items is its length
-  const dim3 grid = b.units ? dim3((unsigned)max_items) : dim3((unsigned)max_items, (unsigned)nprob);
+  // one matrix in one launch: its pairs dealt over the XCDs, padded to whole rows of NXCD
+  const int dealt = (max_items + NXCD - 1) / NXCD * NXCD * (phase == 2 && !b.arr ? b.one.q : 1);
+  const dim3 grid = b.units ? dim3((unsigned)max_items)
+                            : (phase == 2 ? dim3((unsigned)dealt) : dim3((unsigned)max_items, (unsigned)nprob));
   if (phase == 2) {
+    const auto kernel = grid.x <= NCU ? svd_round_mfma_kernel<true> : svd_round_mfma_kernel<false>;
     if (ev0)
-      hipExtLaunchKernelGGL(svd_round_mfma_kernel, grid, dim3(SR_THREADS), 0, s, ev0, ev1, 0, b, round, mode);
+      hipExtLaunchKernelGGL(kernel, grid, dim3(SR_THREADS), 0, s, ev0, ev1, 0, b, round, mode);
     else
-      hipLaunchKernelGGL(svd_round_mfma_kernel, grid, dim3(SR_THREADS), 0, s, b, round, mode);
+      hipLaunchKernelGGL(kernel, grid, dim3(SR_THREADS), 0, s, b, round, mode);
   } else if (ev0) {
     hipExtLaunchKernelGGL(svd_round_kernel, grid, dim3(SR_THREADS), 0, s, ev0, ev1, 0, b, round, phase, mode);
   } else {

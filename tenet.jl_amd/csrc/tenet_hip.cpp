@@ -1352,12 +1352,27 @@ extern "C" int tenet_qr_thin(tenet_ctx ctx, tenet_stream stream, int dtype, int6
 // ---------------------------------------------------------------------------
 // SVD (one-sided block Jacobi)
 // ---------------------------------------------------------------------------
+// How a pair's rows are shared out: one workgroup; q workgroups in one launch
+// a round, each forming the whole Gram (X alternates between two buffers); or
+// q workgroups in two launches a round, with the Gram summed over row chunks.
+enum SvdSplit { SVD_WHOLE, SVD_ONE_LAUNCH, SVD_TWO_PHASE };
+
 struct SvdShape {
   int64_t nr, ncols, b, nblk, ncp, q, npairs;
   bool transposed;
+  SvdSplit split;
 };
 
-static SvdShape svd_shape(int64_t m, int64_t n, bool allow_split, bool force_adj = false) {
+// One matrix takes the one-launch rounds up to this many rows: each workgroup
+// of a pair forms the whole Gram (2450 cycles per 64 rows), which has to stay
+// below what a second launch a round costs.  Against the two launches: 256 x 256
+// 6.7 -> 4.1 ms, 700 x 300 8.8 -> 7.1, 760 x 128 3.1 -> 2.7; at 1024 rows the
+// Gram alone would take as long as both.
+constexpr int64_t SVD_ONE_LAUNCH_ROWS = 768;
+constexpr int64_t SVD_STRIP = 16;  // rows a wave rotates at a time
+constexpr int64_t SVD_CUS = 256;
+
+static SvdShape svd_shape(int64_t m, int64_t n, SvdSplit split, bool force_adj = false) {
   SvdShape sh{};
   sh.transposed = force_adj || m < n;
   sh.nr = std::max(m, n);
@@ -1373,7 +1388,14 @@ static SvdShape svd_shape(int64_t m, int64_t n, bool allow_split, bool force_adj
   sh.ncp = sh.nblk * sh.b;
   sh.npairs = sh.nblk / 2;
   sh.q = 1;
-  if (allow_split) sh.q = std::min<int64_t>(16, std::max<int64_t>(1, (sh.nr + 63) / 64));
+  sh.split = split;
+  if (split == SVD_ONE_LAUNCH) {
+    const int64_t strips = (sh.nr + SVD_STRIP - 1) / SVD_STRIP + (sh.ncp + SVD_STRIP - 1) / SVD_STRIP;
+    sh.q = std::max<int64_t>(1, std::min(SVD_CUS / sh.npairs, (strips + 3) / 4));
+    if (sh.nblk == 2 || sh.nr > SVD_ONE_LAUNCH_ROWS) sh.split = SVD_TWO_PHASE;
+  }
+  if (sh.split == SVD_TWO_PHASE) sh.q = std::min<int64_t>(16, std::max<int64_t>(1, (sh.nr + 63) / 64));
+  if (sh.q == 1) sh.split = SVD_WHOLE;
   return sh;
 }
 
@@ -1382,7 +1404,10 @@ static size_t svd_ws_bytes(const SvdShape& sh) {
   size_t t = 0;
   t += align_up((size_t)sh.nr * sh.ncp * 16, 256);
   t += align_up((size_t)sh.ncp * sh.ncp * 16, 256);
-  t += align_up((size_t)sh.npairs * sh.q * n2 * n2 * 16, 256);
+  if (sh.split == SVD_ONE_LAUNCH)
+    t += align_up((size_t)sh.nr * sh.ncp * 16, 256);
+  else
+    t += align_up((size_t)sh.npairs * sh.q * n2 * n2 * 16, 256);
   t += align_up((size_t)sh.ncp * 8, 256);
   t += align_up((size_t)sh.ncp * 4, 256);
   t += 256;  // flags
@@ -1399,13 +1424,16 @@ static double svd_tol(int64_t nr) { return 1e-14 * std::max(1.0, std::sqrt((doub
 
 static int svd_run(tenet_ctx ctx, hipStream_t s, int dtype, int64_t m, int64_t n, const void* A, int64_t lda, void* U,
                    int64_t ldu, double* S, void* Vh, int64_t ldvh, int64_t maxdim, double thr, int64_t* k_dev,
-                   double* disc_dev, void* wsp, bool allow_split, bool force_adj = false) {
-  const SvdShape sh = svd_shape(m, n, allow_split, force_adj);
+                   double* disc_dev, void* wsp, SvdSplit split, bool force_adj = false) {
+  const SvdShape sh = svd_shape(m, n, split, force_adj);
   Bump bm(wsp);
   SvdProblem P{};
   P.X = (double*)bm.take((size_t)sh.nr * sh.ncp * 16);
   P.V = (double*)bm.take((size_t)sh.ncp * sh.ncp * 16);
-  P.Gpart = (double*)bm.take((size_t)sh.npairs * sh.q * (2 * sh.b) * (2 * sh.b) * 16);
+  if (sh.split == SVD_ONE_LAUNCH)
+    P.X2 = (double*)bm.take((size_t)sh.nr * sh.ncp * 16);
+  else
+    P.Gpart = (double*)bm.take((size_t)sh.npairs * sh.q * (2 * sh.b) * (2 * sh.b) * 16);
   P.sigma = (double*)bm.take((size_t)sh.ncp * 8);
   P.perm = (int32_t*)bm.take((size_t)sh.ncp * 4);
   P.flag = (int32_t*)bm.take(256);
@@ -1449,9 +1477,14 @@ static int svd_run(tenet_ctx ctx, hipStream_t s, int dtype, int64_t m, int64_t n
   const double apply_fl = 8.0 * sh.npairs * n2 * n2 * (sh.nr + sh.ncp);
   const double xv_bytes = 16.0 * sh.npairs * n2 * (sh.nr + sh.ncp);
   auto round = [&](int r, int mode) -> int {
-    if (sh.q == 1)
-      return svd_round_timed(ctx, s, gram_fl + apply_fl, 16.0 * sh.npairs * n2 * sh.nr + 2.0 * xv_bytes, B, 1,
-                             (int)sh.npairs, r, 2, mode);
+    if (sh.split != SVD_TWO_PHASE) {
+      TRY(svd_round_timed(ctx, s, gram_fl + apply_fl, 16.0 * sh.npairs * n2 * sh.nr + 2.0 * xv_bytes, B, 1,
+                          (int)sh.npairs, r, 2, mode));
+      // a sweep is nblk rounds, an even number: X is back in its own buffer
+      // when it ends, also where a captured run's later rounds return at once
+      if (sh.split == SVD_ONE_LAUNCH) std::swap(B.one.X, B.one.X2);
+      return TENET_OK;
+    }
     TRY(svd_round_timed(ctx, s, gram_fl, 16.0 * sh.npairs * n2 * sh.nr, B, 1, (int)(sh.npairs * sh.q), r, 0, mode));
     return svd_round_timed(ctx, s, apply_fl, 2.0 * xv_bytes, B, 1, (int)(sh.npairs * sh.q), r, 1, mode);
   };
@@ -1499,13 +1532,13 @@ static bool svd_precond_applies(tenet_ctx ctx, int dtype, int64_t m, int64_t n) 
 static size_t svd_precond_ws_bytes(int64_t m, int64_t n) {
   const int64_t p = std::max(m, n), q = std::min(m, n);
   return 2 * align_up((size_t)p * q * 16, 256) + 3 * align_up((size_t)q * q * 16, 256) +
-         align_up(qr_ws_bytes(p, q), 256) + svd_ws_bytes(svd_shape(q, q, true, true)) + align_up((size_t)q * 8, 256) +
+         align_up(qr_ws_bytes(p, q), 256) + svd_ws_bytes(svd_shape(q, q, SVD_ONE_LAUNCH, true)) + align_up((size_t)q * 8, 256) +
          align_up((size_t)q * 4, 256) + 1024;
 }
 
 // workspace any SVD path of an m x n matrix may need
 static size_t svd_any_ws_bytes(tenet_ctx ctx, int dtype, int64_t m, int64_t n) {
-  size_t b = svd_ws_bytes(svd_shape(m, n, true));
+  size_t b = svd_ws_bytes(svd_shape(m, n, SVD_ONE_LAUNCH));
   if (svd_precond_applies(ctx, dtype, m, n)) b = std::max(b, svd_precond_ws_bytes(m, n));
   return b;
 }
@@ -1526,10 +1559,10 @@ static int svd_any(tenet_ctx ctx, hipStream_t s, int dtype, int64_t m, int64_t n
                    int64_t ldu, double* S, void* Vh, int64_t ldvh, int64_t maxdim, double thr, int64_t* k_dev,
                    double* disc_dev, void* wsp) {
   if (!svd_precond_applies(ctx, dtype, m, n))
-    return svd_run(ctx, s, dtype, m, n, A, lda, U, ldu, S, Vh, ldvh, maxdim, thr, k_dev, disc_dev, wsp, true);
+    return svd_run(ctx, s, dtype, m, n, A, lda, U, ldu, S, Vh, ldvh, maxdim, thr, k_dev, disc_dev, wsp, SVD_ONE_LAUNCH);
   if (!qr_blocked_fits(std::max(m, n))) {
     // the Jacobi works on its own copy of A, so a retry starts from the untouched input
-    const int st0 = svd_run(ctx, s, dtype, m, n, A, lda, U, ldu, S, Vh, ldvh, maxdim, thr, k_dev, disc_dev, wsp, true);
+    const int st0 = svd_run(ctx, s, dtype, m, n, A, lda, U, ldu, S, Vh, ldvh, maxdim, thr, k_dev, disc_dev, wsp, SVD_ONE_LAUNCH);
     if (st0 != TENET_ERR_NOCONV) return st0;
   }
   const int64_t p = std::max(m, n), q = std::min(m, n);
@@ -1540,7 +1573,7 @@ static int svd_any(tenet_ctx ctx, hipStream_t s, int dtype, int64_t m, int64_t n
   void* UR = bm.take((size_t)q * q * 16);
   void* VRh = bm.take((size_t)q * q * 16);
   void* qr_ws = bm.take(align_up(qr_ws_bytes(p, q), 256));
-  void* svd_ws = bm.take(svd_ws_bytes(svd_shape(q, q, true, true)));
+  void* svd_ws = bm.take(svd_ws_bytes(svd_shape(q, q, SVD_ONE_LAUNCH, true)));
   void* Tp = bm.take((size_t)p * q * 16);
   double* nrm = (double*)bm.take((size_t)q * 8);
   int32_t* perm = (int32_t*)bm.take((size_t)q * 4);
@@ -1549,7 +1582,7 @@ static int svd_any(tenet_ctx ctx, hipStream_t s, int dtype, int64_t m, int64_t n
   // the Jacobi on R^H of TEBD bond matrices then needs ~30% fewer sweeps)
   TRY(launch_pre1_order_pack(A, lda, (int)p, (int)q, tall ? 0 : 1, TENET_C128, nrm, perm, (double*)Tp, s));
   TRY(qr_run(ctx, s, TENET_C128, 0, p, q, Tp, p, Q, p, R, q, qr_ws));
-  int st = svd_run(ctx, s, TENET_C128, q, q, R, q, UR, q, S, VRh, q, maxdim, thr, k_dev, disc_dev, svd_ws, true, true);
+  int st = svd_run(ctx, s, TENET_C128, q, q, R, q, UR, q, S, VRh, q, maxdim, thr, k_dev, disc_dev, svd_ws, SVD_ONE_LAUNCH, true);
   if (st != TENET_OK && st != TENET_ERR_NOCONV) return st;
   if (tall) {
     // A[:, perm] = Q U_R S V_R^H: U = Q U_R, V^H[:, perm[c]] = V_R^H[:, c]
@@ -1608,7 +1641,9 @@ extern "C" int tenet_svd_thin_noalloc(tenet_ctx ctx, tenet_stream stream, int dt
   if (S) TRY(check_span(ctx, S, (size_t)k * 8, "S"));
   // the plain Jacobi path (no QR preconditioning: its contractions build
   // plans, which allocate); its whole workspace must fit the scratch array
-  const size_t need = k <= 4096 ? svd_ws_bytes(svd_shape(m, n, true)) : SIZE_MAX;
+  SvdSplit split = SVD_ONE_LAUNCH;
+  if (k <= 4096 && svd_ws_bytes(svd_shape(m, n, split)) > TENET_SVD_NOALLOC_SCRATCH_BYTES) split = SVD_TWO_PHASE;
+  const size_t need = k <= 4096 ? svd_ws_bytes(svd_shape(m, n, split)) : SIZE_MAX;
   if (need > TENET_SVD_NOALLOC_SCRATCH_BYTES) {
     set_error("tenet_svd_thin_noalloc: a " + std::to_string(m) + " x " + std::to_string(n) + " SVD needs " +
               std::to_string(need) + " bytes of workspace, above the " +
@@ -1622,7 +1657,7 @@ extern "C" int tenet_svd_thin_noalloc(tenet_ctx ctx, tenet_stream stream, int dt
     return TENET_ERR_HIP;
   }
   return svd_run(ctx, pick(ctx, stream), dtype, m, n, A, lda, U, ldu, S, Vh, ldvh, maxdim, threshold, k_dev,
-                 discarded_dev, g_scratch_ptr[ctx->device], true);
+                 discarded_dev, g_scratch_ptr[ctx->device], split);
 }
 
 // workspace of one tenet_simple_update with bond matrix m x n
@@ -2588,13 +2623,14 @@ struct tenet_gsvd_s {
   int64_t max_rounds = 0, max_pairs = 0, max_ncp = 0, max_elems = 0, max_out = 0;
   // per round (0: the fixed-pair round, 1 + r: cross round r) the
   // (problem, pair) units that have work in it, largest problems first
-  std::vector<int32_t> units;  // pairs of int32
+  std::vector<int4> units;
   std::vector<int64_t> uoff, ucnt;
-  int2* units_dev = nullptr;
+  int4* units_dev = nullptr;
   // QR-preconditioned problems (pre set): their batched-QR table, sizes
   std::vector<QrBatchProb> qr_probs;
   QrBatchProb* qr_dev = nullptr;
   int64_t pre_max_m = 0, pre_max_n = 0, pre_max_elems = 0;
+  std::vector<char> two_buffers;  // per problem: some round splits its pairs' rows
   // operands, for the single-matrix fallback of problems the sweeps leave unconverged
   std::vector<int64_t> ms, ns, maxdims;
   std::vector<const void*> As;
@@ -2604,6 +2640,109 @@ struct tenet_gsvd_s {
   int64_t* k_dev = nullptr;
   double* disc_dev = nullptr;
 };
+
+// The round unit lists.  A problem of nblk blocks has npairs pairs in the
+// fixed-pair round (r = -1) and, when nblk > 2, in cross rounds 0 .. nblk - 2.
+//
+// A round lasts as long as its longest workgroup or as its workgroups share
+// the chip, so its pairs are cut into chunks of at most L strips for the L
+// that the model below prices lowest; every chunk repeats the pair's Gram and
+// inner solve.  In cycles: a Gram row is 28 and a strip 768 of a CU's matrix
+// cores, a workgroup takes 36000 besides (launch, loads, inner solve); two
+// workgroups of a CU slow each other by half, and a chip full of them reaches
+// half of the products' rate (memory).  Measured with whole pairs, as cut
+// and, for comparison, cut wherever a CU would be idle: 8 of 512 x 512 without
+// U 17.5, 14.6 and 18.4 ms, 16 of 512 x 400 in complex64 17.8, 17.6 and 21.2,
+// 256 of 8 to 512 a side 19.4, 16.4 and 16.5.
+// Where X ends a round in its other buffer the next round starts from there;
+// a sweep that would leave it there has one of its unsplit rounds change
+// buffers too.
+static void gsvd_units(tenet_gsvd g, const std::vector<int64_t>& order, const std::vector<char>& accum) {
+  constexpr double ROW = 28.0, STRIP_COST = 768.0, ALONE = 36000.0, SHARED = 1.5, FULL = 2.0;
+  const int64_t R = g->max_rounds + 1;
+  g->uoff.assign((size_t)R, 0);
+  g->ucnt.assign((size_t)R, 0);
+  auto in_round = [&](int64_t i, int64_t r) {
+    const SvdShape& sh = g->shapes[(size_t)i];
+    return r == 0 || (sh.nblk > 2 && r - 1 < sh.nblk - 1);
+  };
+  auto strips = [&](int64_t i) {
+    const SvdShape& sh = g->shapes[(size_t)i];
+    return (sh.nr + SVD_STRIP - 1) / SVD_STRIP + (accum[(size_t)i] ? (sh.ncp + SVD_STRIP - 1) / SVD_STRIP : 0);
+  };
+  auto chunks = [&](int64_t i, int64_t L) -> int64_t {
+    const SvdShape& sh = g->shapes[(size_t)i];
+    if (L == 0 || sh.nblk == 2 || sh.nr > SVD_ONE_LAUNCH_ROWS) return 1;
+    return (strips(i) + L - 1) / L;
+  };
+  // the strips per chunk of each round (0: whole pairs)
+  std::vector<int64_t> cut((size_t)R, 0);
+  for (int64_t r = 0; r < R; ++r) {
+    double whole = 0.0, best = 0.0;
+    for (const int64_t L : {0, 32, 24, 16, 8, 4}) {
+      double longest = 0.0, slots = 0.0, mfma = 0.0;
+      for (const int64_t i : order) {
+        if (!in_round(i, r)) continue;
+        const SvdShape& sh = g->shapes[(size_t)i];
+        const double q = (double)chunks(i, L), S = (double)strips(i), gram = ROW * sh.nr;
+        longest = std::max(longest, ALONE + gram + STRIP_COST * std::ceil(S / q));
+        slots += sh.npairs * (q * (ALONE + gram) + STRIP_COST * S);
+        mfma += sh.npairs * (q * gram + STRIP_COST * S);
+      }
+      const double t = std::max(longest, std::max(SHARED * slots / (2 * SVD_CUS), FULL * mfma / SVD_CUS));
+      // whole pairs, in place, unless cutting them is clearly faster
+      if (L == 0) whole = best = t;
+      if (t < best && t < 0.9 * whole) {
+        best = t;
+        cut[(size_t)r] = L;
+      }
+    }
+  }
+  // buffer changes: flips[i * R + r], made even in number
+  g->two_buffers.assign((size_t)g->count, 0);
+  std::vector<char> flips((size_t)(g->count * R), 0);
+  for (int64_t i = 0; i < g->count; ++i) {
+    int64_t n = 0, whole = -1;
+    for (int64_t r = 0; r < R; ++r) {
+      if (!in_round(i, r)) continue;
+      const bool split = chunks(i, cut[(size_t)r]) > 1;
+      flips[(size_t)(i * R + r)] = split;
+      n += split;
+      if (!split) whole = r;
+    }
+    // nblk rounds, an even number, so an odd count of split ones leaves a whole one
+    if (n % 2) flips[(size_t)(i * R + whole)] = 1;
+    g->two_buffers[(size_t)i] = n > 0;
+  }
+  std::vector<char> at((size_t)g->count, 0);  // X's buffer
+  for (int64_t r = 0; r < R; ++r) {
+    g->uoff[(size_t)r] = (int64_t)g->units.size();
+    // a pair's chunks eight apart (one XCD), the pairs largest first to the
+    // XCD with the least strips so far
+    std::vector<int4> lane[8];
+    int64_t load[8] = {};
+    for (const int64_t i : order) {
+      if (!in_round(i, r)) continue;
+      const SvdShape& sh = g->shapes[(size_t)i];
+      const int64_t q = chunks(i, cut[(size_t)r]);
+      const int f = flips[(size_t)(i * R + r)], from = at[(size_t)i];
+      for (int64_t p = 0; p < sh.npairs; ++p) {
+        const int x = (int)(std::min_element(load, load + 8) - load);
+        load[x] += strips(i) + q * (sh.nr / SVD_STRIP + 16);
+        for (int64_t c = 0; c < q; ++c)
+          lane[x].push_back(make_int4((int)i, (int)p, (int)(c | q << 16), from | (from ^ f) << 1));
+      }
+      at[(size_t)i] = (char)(from ^ f);
+    }
+    size_t longest = 0;
+    for (const auto& l : lane) longest = std::max(longest, l.size());
+    for (size_t k = 0; k < longest; ++k)
+      for (const auto& l : lane) g->units.push_back(k < l.size() ? l[k] : make_int4(-1, 0, 0, 0));
+    while (!g->units.empty() && (int64_t)g->units.size() > g->uoff[(size_t)r] && g->units.back().x < 0)
+      g->units.pop_back();
+    g->ucnt[(size_t)r] = (int64_t)g->units.size() - g->uoff[(size_t)r];
+  }
+}
 
 static int gsvd_build(tenet_ctx ctx, int dtype, int64_t count, const int64_t* ms, const int64_t* ns,
                       const void* const* As, void* const* Us, double* const* Ss, void* const* Vhs,
@@ -2643,7 +2782,7 @@ static int gsvd_build(tenet_ctx ctx, int dtype, int64_t count, const int64_t* ms
     if (Ss && Ss[i]) TRY(check_span(ctx, Ss[i], (size_t)k * s_es, "S"));
     // Without U and with m <= n, the Jacobi runs on X = A^H: V^H comes from X
     // itself and the rotations need not be accumulated
-    g->shapes[(size_t)i] = pre[(size_t)i] ? svd_shape(n, n, false, true) : svd_shape(m, n, false, !Us[i] && m <= n);
+    g->shapes[(size_t)i] = pre[(size_t)i] ? svd_shape(n, n, SVD_WHOLE, true) : svd_shape(m, n, SVD_WHOLE, !Us[i] && m <= n);
     const SvdShape& sh = g->shapes[(size_t)i];
     total += svd_ws_bytes(sh);
     if (pre[(size_t)i])
@@ -2664,40 +2803,31 @@ static int gsvd_build(tenet_ctx ctx, int dtype, int64_t count, const int64_t* ms
     g->Vhs.push_back(Vhs[i]);
     g->Ss.push_back(Ss ? Ss[i] : nullptr);
   }
-  // round unit lists: a problem of nblk blocks has npairs units in the
-  // fixed-pair round and, when nblk > 2, in cross rounds 0 .. nblk - 2 (the
-  // rounds launch only these units, not a pairs x problems rectangle)
+  std::vector<char> accum((size_t)count);
+  for (int64_t i = 0; i < count; ++i)
+    accum[(size_t)i] = !pre[(size_t)i] && (Us[i] || !g->shapes[(size_t)i].transposed);
   {
     std::vector<int64_t> order((size_t)count);
     for (int64_t i = 0; i < count; ++i) order[(size_t)i] = i;
     std::stable_sort(order.begin(), order.end(), [&](int64_t x, int64_t y) {
       return g->shapes[(size_t)x].nr * g->shapes[(size_t)x].ncp > g->shapes[(size_t)y].nr * g->shapes[(size_t)y].ncp;
     });
-    g->uoff.assign((size_t)g->max_rounds + 1, 0);
-    g->ucnt.assign((size_t)g->max_rounds + 1, 0);
-    for (int64_t r = -1; r < g->max_rounds; ++r) {
-      g->uoff[(size_t)(r + 1)] = (int64_t)g->units.size() / 2;
-      for (int64_t i : order) {
-        const SvdShape& sh = g->shapes[(size_t)i];
-        if (r >= 0 && (sh.nblk <= 2 || r >= sh.nblk - 1)) continue;
-        for (int64_t p = 0; p < sh.npairs; ++p) {
-          g->units.push_back((int32_t)i);
-          g->units.push_back((int32_t)p);
-        }
-      }
-      g->ucnt[(size_t)(r + 1)] = (int64_t)g->units.size() / 2 - g->uoff[(size_t)(r + 1)];
-    }
-    total += align_up(std::max<size_t>(g->units.size(), 2) * 4, 256);
+    gsvd_units(g, order, accum);
+    for (int64_t i = 0; i < count; ++i)
+      if (g->two_buffers[(size_t)i])
+        total += align_up((size_t)g->shapes[(size_t)i].nr * g->shapes[(size_t)i].ncp * 16, 256);
+    total += align_up(std::max<size_t>(g->units.size(), 1) * sizeof(int4), 256);
   }
   TRY(tenet_malloc(ctx, total, &g->dev));
   Bump bm(g->dev);
   g->dprobs = (SvdProblem*)bm.take((size_t)count * sizeof(SvdProblem));
-  g->units_dev = (int2*)bm.take(std::max<size_t>(g->units.size(), 2) * 4);
+  g->units_dev = (int4*)bm.take(std::max<size_t>(g->units.size(), 1) * sizeof(int4));
   g->probs.resize((size_t)count);
   for (int64_t i = 0; i < count; ++i) {
     const SvdShape& sh = g->shapes[(size_t)i];
     SvdProblem& P = g->probs[(size_t)i];
     P.X = (double*)bm.take((size_t)sh.nr * sh.ncp * 16);
+    if (g->two_buffers[(size_t)i]) P.X2 = (double*)bm.take((size_t)sh.nr * sh.ncp * 16);
     P.V = (double*)bm.take((size_t)sh.ncp * sh.ncp * 16);
     P.Gpart = (double*)bm.take((size_t)sh.npairs * sh.q * (2 * sh.b) * (2 * sh.b) * 16);
     P.sigma = (double*)bm.take((size_t)sh.ncp * 8);
@@ -2711,7 +2841,7 @@ static int gsvd_build(tenet_ctx ctx, int dtype, int64_t count, const int64_t* ms
     P.m = (int32_t)ms[i];
     P.n = (int32_t)ns[i];
     P.transposed = sh.transposed ? 1 : 0;
-    P.accum = (Us[i] || !sh.transposed) ? 1 : 0;
+    P.accum = accum[(size_t)i];
     P.s_mode = s_mode;
     P.A = As[i];
     P.lda = ms[i];
@@ -2728,7 +2858,6 @@ static int gsvd_build(tenet_ctx ctx, int dtype, int64_t count, const int64_t* ms
     if (pre[(size_t)i]) {
       const int64_t m = ms[i], n = ns[i];
       P.pre = 1;
-      P.accum = 0;
       P.ldvh = n;
       P.W = (double*)bm.take((size_t)m * n * 16);
       P.cperm = (int32_t*)bm.take((size_t)n * 4);
@@ -2744,8 +2873,7 @@ static int gsvd_build(tenet_ctx ctx, int dtype, int64_t count, const int64_t* ms
     }
   }
   if (!g->qr_probs.empty()) g->qr_dev = (QrBatchProb*)bm.take(g->qr_probs.size() * sizeof(QrBatchProb));
-  // per problem 8 int32: rotated, converged, sweeps, spare, then the sweep's
-  // largest squared relative off-diagonal (8 bytes at flag + 4)
+  // per problem 8 int32: rotated, converged, sweeps, not yet converging, spare
   g->flags_base = (int32_t*)bm.take((size_t)count * 32);
   double* fro_base = (double*)bm.take((size_t)count * 8);
   for (int64_t i = 0; i < count; ++i) {
@@ -2755,7 +2883,7 @@ static int gsvd_build(tenet_ctx ctx, int dtype, int64_t count, const int64_t* ms
   // ordered on the stream after earlier work (the pool block may have been
   // freed by a caller while that work still used it)
   TRY(upload_async(ctx, s, g->dprobs, g->probs.data(), g->probs.size() * sizeof(SvdProblem)));
-  TRY(upload_async(ctx, s, g->units_dev, g->units.data(), g->units.size() * 4));
+  TRY(upload_async(ctx, s, g->units_dev, g->units.data(), g->units.size() * sizeof(int4)));
   TRY(upload_async(ctx, s, g->qr_dev, g->qr_probs.data(), g->qr_probs.size() * sizeof(QrBatchProb)));
   return TENET_OK;
 }
