@@ -2678,6 +2678,11 @@ static void gsvd_units(tenet_gsvd g, const std::vector<int64_t>& order, const st
   // the strips per chunk of each round (0: whole pairs)
   std::vector<int64_t> cut((size_t)R, 0);
   for (int64_t r = 0; r < R; ++r) {
+    // twice as many pairs as the chip holds: cutting would only add Grams
+    int64_t pairs = 0;
+    for (const int64_t i : order)
+      if (in_round(i, r)) pairs += g->shapes[(size_t)i].npairs;
+    if (pairs > 4 * SVD_CUS) continue;
     double whole = 0.0, best = 0.0;
     for (const int64_t L : {0, 32, 24, 16, 8, 4}) {
       double longest = 0.0, slots = 0.0, mfma = 0.0;
@@ -2717,6 +2722,17 @@ static void gsvd_units(tenet_gsvd g, const std::vector<int64_t>& order, const st
   std::vector<char> at((size_t)g->count, 0);  // X's buffer
   for (int64_t r = 0; r < R; ++r) {
     g->uoff[(size_t)r] = (int64_t)g->units.size();
+    if (cut[(size_t)r] == 0) {
+      for (const int64_t i : order) {
+        if (!in_round(i, r)) continue;
+        const int f = flips[(size_t)(i * R + r)], from = at[(size_t)i];
+        for (int64_t p = 0; p < g->shapes[(size_t)i].npairs; ++p)
+          g->units.push_back(make_int4((int)i, (int)p, 1 << 16, from | (from ^ f) << 1));
+        at[(size_t)i] = (char)(from ^ f);
+      }
+      g->ucnt[(size_t)r] = (int64_t)g->units.size() - g->uoff[(size_t)r];
+      continue;
+    }
     // a pair's chunks eight apart (one XCD), the pairs largest first to the
     // XCD with the least strips so far
     std::vector<int4> lane[8];
