@@ -53,7 +53,7 @@ PEAK_FP64_TFLOPS = 78.6
 # HBM bytes per round-kernel dispatch (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 KiB,
 # factors from the scale kernel over 256 MiB) for each TEBD form, from
 # rocprofv3 --pmc passes over one sweep; None where not measured.
-ROUND_TRAFFIC_BYTES = {"fp64": 17_005_568, "vidal": 216_834_819, "vidal_graph": 216_834_819}
+ROUND_TRAFFIC_BYTES = {"vidal": 216_834_819, "vidal_graph": 216_834_819}
 
 FORMS = {"fp64": 0, "fp32": 1, "split_bf16": 2, "split_fp16": 3, "vidal": 0, "vidal_graph": 0}
 DEFAULT_FORMS = "vidal,vidal_graph,fp64,split_bf16,split_fp16,fp32"
@@ -703,8 +703,8 @@ def bench_tebd(args):
                 "kernel": ("svd_round_mfma_kernel (grouped one-sided Jacobi rounds: every SVD of a brickwork layer "
                            "per launch; Gram and rotation on v_mfma_f64_16x16x4, inner 32x32 solve on FP64 VALU)"
                            if head in VIDAL_FORMS else
-                           "svd_round_kernel (one-sided Jacobi round of one SVD: pair Grams, rotations, apply; "
-                           "FP64 VALU)"),
+                           "svd_round_mfma_kernel (one-sided Jacobi round of one SVD, a pair's rows over several "
+                           "workgroups; Gram and rotation on v_mfma_f64_16x16x4, inner 32x32 solve on FP64 VALU)"),
                 "achieved_basis": "nominal SVD flops 4(4p^2q+8pq^2+9q^3) of the sweep / round-kernel time",
                 "peak_basis": "FP64 (vector and matrix peaks are both 78.6 TFLOP/s on MI355X)",
                 "executed_tflops": round(executed, 3), "executed_frac": round(executed / PEAK_FP64_TFLOPS, 4),
