@@ -855,9 +855,12 @@ __device__ __forceinline__ svd_d4v mfma_f64(double a, double b, svd_d4v c) {
 // round before).  The waves' sums are added in LDS in a fixed order, halving
 // the waves.  A chunk of 64 rows is bound by the products: 1800 cycles of the
 // matrix cores.
+//
+// Returns false, with nothing formed, for a converged problem: its flag is
+// looked at when the first loads are under way, not before them.
 template <int D>
-__device__ __forceinline__ void gram_mfma(SvSmem& sm, const double* X, int64_t ld, int r0, int r1, int I, int J,
-                                          int b) {
+__device__ __forceinline__ bool gram_mfma(SvSmem& sm, const double* X, int64_t ld, int r0, int r1, int I, int J, int b,
+                                          int converged) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int kr = lane >> 4, kc = lane & 15;
   const int n2 = 2 * b, tr = lane & (GT - 1), tc = lane / GT;
@@ -876,6 +879,7 @@ __device__ __forceinline__ void gram_mfma(SvSmem& sm, const double* X, int64_t l
     if (r0 + d * RS < r1)
 #pragma unroll
       for (int u = 0; u < 4; ++u) v[d][u] = X2[col[u] + min(own + d * RS, r1 - 1)];
+  if (converged) return false;
   for (int r2 = r0; r2 < r1; r2 += D * RS) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -945,6 +949,7 @@ __device__ __forceinline__ void gram_mfma(SvSmem& sm, const double* X, int64_t l
     if ((i < 16) == (j < 16)) sm.gr[i][j] -= pij + pji;  // Re G = S^T S - P - P^T
   }
   __syncthreads();
+  return true;
 }
 
 // M <- M W by MFMA, with no LDS staging, in strips of 16 rows: one wave takes a
@@ -1096,7 +1101,7 @@ __device__ __forceinline__ void round_pair(int p, int round, int mode, int nb, i
 // the whole round: 63 us at 512 rows of each, 30 us cut.  Such a round is a
 // chain: launch 3 us, Gram 8 us at 256 rows (loads, then 2450 cycles per 64
 // rows), inner solve 9 us (a sweep's first, fixed-pair round 17), rotation 2 us
-// (one 256 x 256 matrix: 22.5 us a round; with two launches, the partial Grams
+// (one 256 x 256 matrix: 21.5 us a round; with two launches, the partial Grams
 // on the VALU, it was 36).  With two workgroups on each CU (ALONE = false:
 // 496 pairs of 512 rows, 63 us) the rounds run at 6.3 TB/s over X, read twice
 // and written once, from beyond the L2s.
@@ -1104,11 +1109,15 @@ __device__ __forceinline__ void round_pair(int p, int round, int mode, int nb, i
 constexpr int NXCD = 8;
 constexpr unsigned NCU = 256;
 
-template <bool ALONE>
+//
+// UNITS: a batch's unit list and problem table, else the one problem among the
+// kernel's arguments (a choice at run time made every field a branch and a
+// scalar load that the next one waited for).
+template <bool ALONE, bool UNITS>
 __global__ __launch_bounds__(SR_THREADS, ALONE ? 2 : 4) void svd_round_mfma_kernel(SvdBatch Bt, int round, int mode) {
   __shared__ SvSmem sm;
   int prob = 0, p, c, q, flip;
-  if (Bt.units) {
+  if constexpr (UNITS) {
     const int4 u = Bt.units[blockIdx.x];
     if (u.x < 0) return;  // padding of the list
     prob = u.x;
@@ -1123,8 +1132,8 @@ __global__ __launch_bounds__(SR_THREADS, ALONE ? 2 : 4) void svd_round_mfma_kern
     c = k % q;
     flip = q > 1 ? 2 : 0;
   }
-  const SvdProblem& P = Bt.arr ? Bt.arr[prob] : Bt.one;
-  if (P.flag[1]) return;  // converged
+  const SvdProblem& P = UNITS ? Bt.arr[prob] : Bt.one;
+  const int converged = P.flag[1];
   const int nb = P.nblk;
   if (mode == 1 && (nb <= 2 || round >= nb - 1)) return;
   if (p >= nb / 2) return;
@@ -1134,7 +1143,7 @@ __global__ __launch_bounds__(SR_THREADS, ALONE ? 2 : 4) void svd_round_mfma_kern
   const double* Xs = (flip & 1) ? P.X2 : P.X;
   double* Xd = (flip & 2) ? P.X2 : P.X;
   const double abs_tol = fmax(4.930380657631324e-32 * (*P.fro2), 1e-300), tol = P.tol;
-  gram_mfma<ALONE ? 4 : 2>(sm, Xs, P.nr, 0, P.nr, I, J, b);
+  if (!gram_mfma<ALONE ? 4 : 2>(sm, Xs, P.nr, 0, P.nr, I, J, b, converged)) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int S = strip_count(P);
   const int lo = (int)((int64_t)c * S / q), hi = (int)((int64_t)(c + 1) * S / q);
@@ -1827,7 +1836,10 @@ int launch_svd_round(const SvdBatch& b, int64_t nprob, int max_items, int round,
   const dim3 grid = b.units ? dim3((unsigned)max_items)
                             : (phase == 2 ? dim3((unsigned)dealt) : dim3((unsigned)max_items, (unsigned)nprob));
   if (phase == 2) {
-    const auto kernel = grid.x <= NCU ? svd_round_mfma_kernel<true> : svd_round_mfma_kernel<false>;
+    // one matrix has at most NCU workgroups with work (q <= NCU / pairs)
+    const auto kernel = !b.units         ? svd_round_mfma_kernel<true, false>
+                        : grid.x <= NCU ? svd_round_mfma_kernel<true, true>
+                                        : svd_round_mfma_kernel<false, true>;
     if (ev0)
       hipExtLaunchKernelGGL(kernel, grid, dim3(SR_THREADS), 0, s, ev0, ev1, 0, b, round, mode);
     else
