@@ -737,14 +737,80 @@ __global__ __launch_bounds__(64 * QB) void qr_panel_v4_batched_kernel(const QrBa
                 reinterpret_cast<const double2*>(q.W) + (size_t)j0 * q.m + j0, q.m);
 }
 
+// Q (m x k) = [I; 0] in FP64
+__global__ void qr_eye_kernel(double* __restrict__ Q, int m, int k) {
+  const size_t total = (size_t)m * k;
+  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < total; e += (size_t)gridDim.x * blockDim.x) {
+    const int r = (int)(e % m), c = (int)(e / m);
+    double2 v;
+    v.x = (r == c) ? 1.0 : 0.0;
+    v.y = 0.0;
+    reinterpret_cast<double2*>(Q)[e] = v;
+  }
+}
+
+// Copy Q (FP64, m x k) and R (upper triangle of W) to the outputs
+template <typename S2>
+__global__ void qr_store_kernel(const double* __restrict__ W, const double* __restrict__ Q, int m, int n, void* Qout,
+                                int64_t ldq, void* Rout, int64_t ldr, int flags) {
+  const int k = min(m, n);
+  const size_t nq = (size_t)m * k, nr = (size_t)k * n;
+  const bool qadj = (flags & TENET_QR_Q_ADJ) != 0, radj = (flags & TENET_QR_R_ADJ) != 0;
+  S2* Qo = static_cast<S2*>(Qout);
+  S2* Ro = static_cast<S2*>(Rout);
+  for (size_t e = (size_t)blockIdx.x * blockDim.x + threadIdx.x; e < nq + nr; e += (size_t)gridDim.x * blockDim.x) {
+    if (e < nq) {
+      const int r = (int)(e % m), c = (int)(e / m);
+      const double2 v = reinterpret_cast<const double2*>(Q)[e];
+      S2 o;
+      o.x = v.x;
+      o.y = qadj ? -v.y : v.y;
+      if (qadj)
+        Qo[(size_t)r * ldq + c] = o;
+      else
+        Qo[(size_t)c * ldq + r] = o;
+    } else {
+      const size_t f = e - nq;
+      const int r = (int)(f % k), c = (int)(f / k);
+      double2 v;
+      v.x = 0.0;
+      v.y = 0.0;
+      if (r <= c) v = reinterpret_cast<const double2*>(W)[(size_t)c * m + r];
+      S2 o;
+      o.x = v.x;
+      o.y = radj ? -v.y : v.y;
+      if (radj)
+        Ro[(size_t)r * ldr + c] = o;
+      else
+        Ro[(size_t)c * ldr + r] = o;
+    }
+  }
+}
+
+constexpr int QS_ROWS = 512;  // rows of a panel that qr_step_kernel holds
+
+// Above 512 rows the trailing columns of a panel and Q go through the 16-wave
+// workgroups' kernels (qr_update_kernel, qr_form_kernel) or, cut into chunks of
+// 64 rows over many workgroups, through qr_apply_chunked.  One workgroup per
+// column block is bound by its CU's address unit (24 us a panel at 768 rows, 32
+// at 1024, however many blocks); the chunks' two launches take 17 us while few
+// blocks share the chip.  Measured lines: 32 column blocks for the trailing
+// update (1024 x 512 4083 -> 3900 us, 768 x 256 1928 -> 1815; 1024 x 1024 5460
+// against 5742 with all panels in chunks); Q in chunks above 768 rows up to 16
+// blocks (1024 x 64 480 -> 461, 1024 x 256 1922 -> 1885, 1024 x 400 3045
+// against 3088, 700 x 64 449 against 452).
+constexpr int QA_MAX_BLOCKS = 32;
+static bool qr_chunked_q(int64_t m, int64_t k) { return m > 768 && k <= 16 * QB; }
+
 bool qr_blocked_fits(int64_t m) { return m <= QP_MAX_ROWS; }
 
-// Row-chunked application of one block reflector on a batch of matrices,
-// M <- (I - V T^H V^H) M on rows [j0, m) and columns [col_begin, col_end), a
-// workgroup per (16-column block, 64-row chunk):
+// Row-chunked application of one block reflector, M <- (I - V T' V^H) M on rows
+// [j0, m) and columns [col_begin, col_end), a workgroup per (16-column block,
+// 64-row chunk):
 //   phase Y: Ypart[chunk][block] = V[chunk]^H M[chunk, block]   (16 x 16)
-//   phase Z: Z = T^H sum_chunks Ypart, once per column block
-//   phase X: M[chunk, block] -= V[chunk] Z
+//   phase Z (batched): Z = T^H sum_chunks Ypart, once per column block
+//   phase X: M[chunk, block] -= V[chunk] Z (one matrix: Z = T' sum_chunks Ypart
+//            formed by each workgroup, in a fixed order)
 constexpr int QA_RC = 64;
 
 __device__ __forceinline__ void qa_load_v(const double2* __restrict__ Wc, int m, int j0, int jb, int rb, int rows,
@@ -848,6 +914,95 @@ __device__ __forceinline__ void qa_y_body(const double* __restrict__ W, const do
     out[2 * e] = yred[0][e][0] + yred[1][e][0] + yred[2][e][0] + yred[3][e][0];
     out[2 * e + 1] = yred[0][e][1] + yred[1][e][1] + yred[2][e][1] + yred[3][e][1];
   }
+}
+
+__global__ __launch_bounds__(QR_THREADS) void qr_apply_y_kernel(const double* __restrict__ W,
+                                                                 const double* __restrict__ M, double* __restrict__ Yp,
+                                                                 int m, int ldm, int j0, int jb, int col_begin,
+                                                                 int col_end) {
+  qa_y_body(W, M, Yp, m, ldm, j0, jb, col_begin, col_end, blockIdx.x, blockIdx.y, gridDim.x);
+}
+
+__device__ __forceinline__ void qa_x_body(const double* __restrict__ W, const double* __restrict__ T,
+                                          const double* __restrict__ Yp, double* __restrict__ M, int m, int ldm,
+                                          int j0, int jb, int col_begin, int col_end, int nchunks, int adj, int blk,
+                                          int chunk, int nblk) {
+  __shared__ double vr[QA_RC][QB + 1], vi[QA_RC][QB + 1];
+  __shared__ double yr[QB][QB + 1], yi[QB][QB + 1];
+  __shared__ double zr[QB][QB + 1], zi[QB][QB + 1];
+  const int tid = threadIdx.x;
+  const int cb0 = col_begin + blk * QB;
+  const int nc = min(QB, col_end - cb0);
+  const int rb = j0 + chunk * QA_RC;
+  const int rows = min(QA_RC, m - rb);
+  if (nc <= 0 || rows <= 0) return;
+  const double2* Wc = reinterpret_cast<const double2*>(W);
+  double2* Mc = reinterpret_cast<double2*>(M);
+  qa_load_v(Wc, m, j0, jb, rb, rows, vr, vi);
+  {
+    // Y = sum over chunks (fixed order), one entry per thread
+    const int a = tid / QB, c = tid % QB;
+    double sr = 0.0, si = 0.0;
+    for (int ch = 0; ch < nchunks; ++ch) {
+      const double* in = Yp + ((size_t)ch * nblk + blk) * QB * QB * 2;
+      sr += in[2 * (a * QB + c)];
+      si += in[2 * (a * QB + c) + 1];
+    }
+    yr[a][c] = sr;
+    yi[a][c] = si;
+  }
+  __syncthreads();
+  {
+    // Z = T' Y
+    const int a = tid / QB, c = tid % QB;
+    double sr = 0.0, si = 0.0;
+    for (int b = 0; b < jb; ++b) {
+      double tr, ti;
+      if (adj) {
+        tr = T[2 * (a * QB + b)];
+        ti = -T[2 * (a * QB + b) + 1];
+      } else {
+        tr = T[2 * (b * QB + a)];
+        ti = T[2 * (b * QB + a) + 1];
+      }
+      sr += tr * yr[b][c] - ti * yi[b][c];
+      si += tr * yi[b][c] + ti * yr[b][c];
+    }
+    zr[a][c] = (a < jb) ? sr : 0.0;
+    zi[a][c] = (a < jb) ? si : 0.0;
+  }
+  __syncthreads();
+  // M[chunk rows] -= V Z: thread owns row tid % 64 and 4 columns
+  const int rsub = tid % QA_RC, cq = 4 * (tid / QA_RC);
+  if (rsub < rows) {
+    double sr[4] = {0, 0, 0, 0}, si[4] = {0, 0, 0, 0};
+#pragma unroll
+    for (int b = 0; b < QB; ++b) {
+      const double pr = vr[rsub][b], pi = vi[rsub][b];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        sr[j] += pr * zr[b][cq + j] - pi * zi[b][cq + j];
+        si[j] += pr * zi[b][cq + j] + pi * zr[b][cq + j];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      if (cq + j < nc) {
+        double2 x = Mc[(size_t)(cb0 + cq + j) * ldm + rb + rsub];
+        x.x -= sr[j];
+        x.y -= si[j];
+        Mc[(size_t)(cb0 + cq + j) * ldm + rb + rsub] = x;
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(QR_THREADS) void qr_apply_x_kernel(const double* __restrict__ W,
+                                                                 const double* __restrict__ T,
+                                                                 const double* __restrict__ Yp, double* __restrict__ M,
+                                                                 int m, int ldm, int j0, int jb, int col_begin,
+                                                                 int col_end, int nchunks, int adj) {
+  qa_x_body(W, T, Yp, M, m, ldm, j0, jb, col_begin, col_end, nchunks, adj, blockIdx.x, blockIdx.y, gridDim.x);
 }
 
 // Batched form: Z = T^H sum_chunks Ypart formed once per (problem, column
@@ -1306,6 +1461,21 @@ __global__ __launch_bounds__(QR_THREADS, 2) void qr_wfused_batched_kernel(const 
   }
 }
 
+// M <- (I - V T' V^H) M (adj = 1: T' = T^H, forward application during the
+// factorisation; adj = 0: T' = T, backward accumulation of Q)
+static int qr_apply_chunked(const double* W, const double* T, double* M, int m, int ldm, int j0, int jb, int c_begin,
+                            int c_end, int adj, double* Yp, hipStream_t s) {
+  if (c_end <= c_begin || m <= j0) return TENET_OK;
+  const unsigned nblk = (unsigned)((c_end - c_begin + QB - 1) / QB);
+  const unsigned nch = (unsigned)((m - j0 + QA_RC - 1) / QA_RC);
+  hipLaunchKernelGGL(qr_apply_y_kernel, dim3(nblk, nch), dim3(QR_THREADS), 0, s, W, M, Yp, m, ldm, j0, jb, c_begin,
+                     c_end);
+  TENET_HIP_CHECK(hipGetLastError());
+  hipLaunchKernelGGL(qr_apply_x_kernel, dim3(nblk, nch), dim3(QR_THREADS), 0, s, W, T, Yp, M, m, ldm, j0, jb, c_begin,
+                     c_end, (int)nch, adj);
+  TENET_HIP_CHECK(hipGetLastError());
+  return TENET_OK;
+}
 
 // Householder QR of every problem of a batch in place (R on and above the
 // diagonal of W, the reflectors below; tau and the panels' T factors kept):
@@ -1371,7 +1541,10 @@ int launch_qr_batched(const QrBatchProb* probs, int64_t nprob, int max_m, int ma
 size_t qr_blocked_ws_bytes(int64_t m, int64_t n) {
   const int64_t k = std::min(m, n);
   const int64_t np = (k + QB - 1) / QB;
-  return (size_t)m * n * 16 + (size_t)k * 16 + (size_t)np * QB * QB * 16 + 2048;
+  size_t b = (size_t)m * n * 16 + (size_t)k * 16 + (size_t)np * QB * QB * 16 + 2048;
+  if (m > QS_ROWS) b += (size_t)((m + QA_RC - 1) / QA_RC) * QA_MAX_BLOCKS * QB * QB * 16;  // chunk partials
+  if (qr_chunked_q(m, k)) b += (size_t)m * k * 16;                                         // Q scratch
+  return b;
 }
 
 // ---------------------------------------------------------------------------
@@ -1725,8 +1898,6 @@ int launch_qr_small(const void* A, int64_t lda, int64_t m, int64_t n, void* Qout
   return TENET_OK;
 }
 
-// W (m x n, FP64 complex, already packed) -> Q, R outputs.  Workspace after W:
-// Q scratch (m x k), tau (k), T blocks.
 // ---- one matrix: a launch per panel, and one for Q ----------------------------
 // The 16 x 16 x 4 FP64 MFMA leaves row 4 r + l / 16, column l % 16 of its result
 // in register r of lane l, which is the layout its B operand wants for the
@@ -2049,11 +2220,16 @@ static void launch_qr_form(const double* W, const double* Tb, int m, int n, int 
     hipLaunchKernelGGL((qr_form_kernel<S2, 4>), grid, block, 0, s, W, Tb, m, n, k, np, Q, ldq, R, ldr, flags);
 }
 
+// W (m x n, FP64 complex, already packed) -> Q, R outputs.  Workspace after W:
+// tau (k), the T blocks, above 512 rows the chunk partials and, where Q is
+// formed in chunks, Q (m x k).
 int launch_qr_blocked(double* W, int64_t m64, int64_t n64, void* Qout, int64_t ldq, void* Rout, int64_t ldr, int dtype,
                       int flags, hipStream_t s) {
   const int m = (int)m64, n = (int)n64, k = std::min(m, n), np = (k + QB - 1) / QB;
   double* tau = W + (size_t)m * n * 2;
   double* Tb = tau + (size_t)k * 2;
+  double* Yp = Tb + (size_t)np * QB * QB * 2;  // chunk partials of V^H M (above QS_ROWS rows)
+  double* Q = Yp + (size_t)((m + QA_RC - 1) / QA_RC) * QA_MAX_BLOCKS * QB * QB * 2;  // (qr_chunked_q)
   // the first panel, then one launch per further panel
   {
     const int jb = std::min(QB, k);
@@ -2082,8 +2258,13 @@ int launch_qr_blocked(double* W, int64_t m64, int64_t n64, void* Qout, int64_t l
       hipLaunchKernelGGL(qr_step_kernel<8>, grid, block, 0, s, W, tau, Tb, m, n, k, p);
     else {
       // more than 512 rows: the panel's rows do not fit the 16-wave kernel
-      hipLaunchKernelGGL(qr_update_kernel, grid, block, 0, s, W, Tb, m, n, p, QB, j1);
-      TENET_HIP_CHECK(hipGetLastError());
+      if (grid.x <= QA_MAX_BLOCKS) {
+        const int st = qr_apply_chunked(W, Tb + (size_t)p * QB * QB * 2, W, m, m, p * QB, QB, j1, n, 1, Yp, s);
+        if (st != TENET_OK) return st;
+      } else {
+        hipLaunchKernelGGL(qr_update_kernel, grid, block, 0, s, W, Tb, m, n, p, QB, j1);
+        TENET_HIP_CHECK(hipGetLastError());
+      }
       hipLaunchKernelGGL(qr_panel_v3_kernel<4>, dim3(1), dim3(QP3_THREADS), 0, s, W, tau,
                          Tb + (size_t)(p + 1) * QB * QB * 2, m, j1, std::min(QB, k - j1));
     }
@@ -2094,6 +2275,25 @@ int launch_qr_blocked(double* W, int64_t m64, int64_t n64, void* Qout, int64_t l
     const dim3 grid((unsigned)((n - k + QB - 1) / QB)), block(64 * QB);
     hipLaunchKernelGGL(qr_update_kernel, grid, block, 0, s, W, Tb, m, n, np - 1, jbl, k);
     TENET_HIP_CHECK(hipGetLastError());
+  }
+  if (qr_chunked_q(m, k)) {
+    const unsigned ge = (unsigned)std::max<size_t>(1, std::min<size_t>(((size_t)m * k + 255) / 256, 4096));
+    hipLaunchKernelGGL(qr_eye_kernel, dim3(ge), dim3(256), 0, s, Q, m, k);
+    TENET_HIP_CHECK(hipGetLastError());
+    for (int p = np - 1; p >= 0; --p) {
+      const int j0 = p * QB;
+      const int st =
+          qr_apply_chunked(W, Tb + (size_t)p * QB * QB * 2, Q, m, m, j0, std::min(QB, k - j0), j0, k, 0, Yp, s);
+      if (st != TENET_OK) return st;
+    }
+    const size_t total = (size_t)m * k + (size_t)k * n;
+    const unsigned gs = (unsigned)std::max<size_t>(1, std::min<size_t>((total + 255) / 256, 4096));
+    if (dtype == TENET_C128)
+      hipLaunchKernelGGL(qr_store_kernel<double2>, dim3(gs), dim3(256), 0, s, W, Q, m, n, Qout, ldq, Rout, ldr, flags);
+    else
+      hipLaunchKernelGGL(qr_store_kernel<float2>, dim3(gs), dim3(256), 0, s, W, Q, m, n, Qout, ldq, Rout, ldr, flags);
+    TENET_HIP_CHECK(hipGetLastError());
+    return TENET_OK;
   }
   if (dtype == TENET_C128)
     launch_qr_form<double2>(W, Tb, m, n, k, np, Qout, ldq, Rout, ldr, flags, s);

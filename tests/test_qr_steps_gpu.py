@@ -45,3 +45,13 @@ def test_factors(ctx, m, n, dt, tol):
         q, r = q.to_host().astype(np.complex128), r.to_host().astype(np.complex128)
         assert np.linalg.norm(q.conj().T @ q - np.eye(k)) <= tol * np.sqrt(k)
         assert np.linalg.norm(q @ r - a) <= tol * np.linalg.norm(a)
+
+
+@pytest.mark.parametrize("dt,tol", [(np.complex128, 1e-12), (np.complex64, 1e-6)])
+@pytest.mark.parametrize("m,n", [(768, 256), (769, 5), (769, 256), (769, 257), (1024, 240), (600, 527), (600, 529),
+                                 (640, 1000), (1024, 1)])
+def test_above_512_rows(ctx, m, n, dt, tol):
+    """Either side of the lines between the row chunks and the 16-wave
+    workgroups: 768 rows and 256 columns for Q, 32 column blocks right of a
+    panel for its update."""
+    test_factors(ctx, m, n, dt, tol)
