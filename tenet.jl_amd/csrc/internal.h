@@ -157,6 +157,18 @@ int launch_qr_blocked(double* W, int64_t m, int64_t n, void* Qout, int64_t ldq, 
                       int flags, hipStream_t s);
 
 // ---- K3: one-sided block Jacobi SVD -----------------------------------------
+// Workgroups that share the rows of each of one matrix's npairs pairs in a
+// one-launch round.  Pairs are dealt over the XCDs and all of a pair's
+// workgroups lie on its XCD, one to a CU, so what the busiest XCD holds must
+// fit its 32 CUs: a workgroup more waits for a whole round (600 x 600, 19
+// pairs: 13 shares 28.2 ms, 10 shares 17.2; two launches a round 20.9).  With
+// at most four strips of 16 rows a share more workgroups bring nothing.
+constexpr int SVD_XCDS = 8, SVD_XCD_CUS = 32;
+inline int64_t svd_row_shares(int64_t npairs, int64_t strips) {
+  const int64_t busiest = (npairs + SVD_XCDS - 1) / SVD_XCDS;
+  const int64_t fit = SVD_XCD_CUS / busiest, most = (strips + 3) / 4, q = fit < most ? fit : most;
+  return q > 1 ? q : 1;
+}
 struct SvdProblem {
   double* X;      // nr x ncp work matrix (complex, column-major)
   double* X2;     // second X buffer of rounds that split a pair's rows (NULL: none do)

@@ -1106,8 +1106,8 @@ __device__ __forceinline__ void round_pair(int p, int round, int mode, int nb, i
 // 496 pairs of 512 rows, 63 us) the rounds run at 6.3 TB/s over X, read twice
 // and written once, from beyond the L2s.
 // mode 0: full inner sweep on the fixed pairs; mode 1: cross-block inner steps.
-constexpr int NXCD = 8;
-constexpr unsigned NCU = 256;
+constexpr int NXCD = SVD_XCDS;
+constexpr unsigned NCU = SVD_XCDS * SVD_XCD_CUS;
 
 //
 // UNITS: a batch's unit list and problem table, else the one problem among the
@@ -1836,7 +1836,7 @@ int launch_svd_round(const SvdBatch& b, int64_t nprob, int max_items, int round,
   const dim3 grid = b.units ? dim3((unsigned)max_items)
                             : (phase == 2 ? dim3((unsigned)dealt) : dim3((unsigned)max_items, (unsigned)nprob));
   if (phase == 2) {
-    // one matrix has at most NCU workgroups with work (q <= NCU / pairs)
+    // one matrix has at most one workgroup with work per CU (svd_row_shares)
     const auto kernel = !b.units         ? svd_round_mfma_kernel<true, false>
                         : grid.x <= NCU ? svd_round_mfma_kernel<true, true>
                                         : svd_round_mfma_kernel<false, true>;

@@ -1391,7 +1391,7 @@ static SvdShape svd_shape(int64_t m, int64_t n, SvdSplit split, bool force_adj =
   sh.split = split;
   if (split == SVD_ONE_LAUNCH) {
     const int64_t strips = (sh.nr + SVD_STRIP - 1) / SVD_STRIP + (sh.ncp + SVD_STRIP - 1) / SVD_STRIP;
-    sh.q = std::max<int64_t>(1, std::min(SVD_CUS / sh.npairs, (strips + 3) / 4));
+    sh.q = svd_row_shares(sh.npairs, strips);
     if (sh.nblk == 2 || sh.nr > SVD_ONE_LAUNCH_ROWS) sh.split = SVD_TWO_PHASE;
   }
   if (sh.split == SVD_TWO_PHASE) sh.q = std::min<int64_t>(16, std::max<int64_t>(1, (sh.nr + 63) / 64));
