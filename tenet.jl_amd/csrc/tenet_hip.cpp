@@ -968,21 +968,34 @@ static void set_tables(GemmTables& t, int64_t* T, const size_t* off) {
   t.bC = T + off[8];
 }
 
-// Where the vendor library's GEMM beats the direct kernel (measured, library
-// against direct, us).  complex128: large products whose 64 x 64 tiles fill the
-// rounds of 256 CUs (1024^3, N/T 126 : 145, C/N 136 : 145; 4096^3 7640 : 8090);
-// a last round mostly empty costs the library more than the tiles' rate gains
-// (3072 x 768 x 3840, 2.25 rounds, 1300 : 1140; 1536^3 538 : 500).  complex64:
-// a band of sizes, with A contiguous along K around 700^3 (26 : 39; 512^3
-// 17.4 : 16.7, 1024^3 90 : 84, 2048^3 637 : 560), otherwise around 2048^3
-// (538 : 605; 1024^3 157 : 84, 250 x 1250 x 462 42 : 19, 4096^3 4890 : 4440).
-static bool lib_pays(int dtype, rocblas_operation opA, int64_t M, int64_t N, int64_t K, int64_t batch) {
-  const double fl = 8.0 * M * N * K * batch;
-  if (dtype == TENET_C128) {
-    const double rounds = (double)((M + 63) / 64) * ((N + 63) / 64) * batch / 256.0;
-    return fl >= 5e9 && rounds >= 0.92 * std::ceil(rounds);
-  }
-  return opA == rocblas_operation_none ? fl >= 3e10 && fl < 3e11 : fl >= 1.5e9 && fl < 6e9;
+// Where the vendor library's GEMM beats the direct kernel, from both sides'
+// times of 1176 products (148 shapes a type and operand order, 1e8 .. 1e11
+// flops, edges 16 .. 40000, K 8 .. 8192, up to 64 in a batch).
+//  - 768 and more tiles of 64 x 64, three rounds of 256 CUs: its tiles' rate
+//    tells (complex128 4348 x 722 x 146 64 : 85 us, complex64 4896 x 2389 x 161
+//    132 : 182), but for the shortest K (20047 x 1727 x 17 289 : 213); narrow
+//    edges are padded by it (20451 x 23 x 1381 310 : 144).
+//  - complex128 of 5 GFLOP and more whose rounds are nearly full (1024^3 120 :
+//    130; 3072 x 768 x 3840, 2.25 rounds, 1300 : 1140).
+//  - with fewer tiles, the operand orders for which it has small ones: A and B
+//    both as stored in complex128 (500^3 17 : 22, 1226 x 325 x 250 17 : 23) and
+//    A along K in complex64 (640^3 23 : 33, 1137 x 446 x 316 14 : 19), up to the
+//    K where few tiles leave it behind (385 x 2999 x 6279 1382 : 568).
+// Elsewhere it falls far behind (128 x 128 x 65536 7100 : 1000, complex64 256 x
+// 256 x 16384 3555 : 182).  The rule's choice is 1.4% slower than the better of
+// the two in the mean, 45% at worst (43 of 38 x 519 x 37, 10 : 15), where the
+// library alone would be 61% slower and the direct kernel alone 4.5%.
+static bool lib_pays(int dtype, rocblas_operation opA, rocblas_operation opB, int64_t M, int64_t N, int64_t K,
+                     int64_t batch) {
+  const int64_t edge = std::min(M, N);
+  if (edge < 64) return false;
+  const double tiles = (double)((M + 63) / 64) * (double)((N + 63) / 64) * (double)batch;
+  if (tiles >= 768) return K >= (dtype == TENET_C128 ? 32 : 16);
+  if (dtype == TENET_C128 && 8.0 * M * N * K * batch >= 5e9 && tiles >= 0.92 * 256 * std::ceil(tiles / 256))
+    return true;
+  if (opB != rocblas_operation_none || K > 4000) return false;
+  if (dtype == TENET_C128) return opA == rocblas_operation_none && tiles >= 48 && edge >= 180;
+  return opA != rocblas_operation_none && tiles >= 64;
 }
 
 static int build_plan(tenet_ctx ctx, int dtype, int prec, const tenet_tdesc* a, const tenet_tdesc* b,
@@ -1002,7 +1015,7 @@ static int build_plan(tenet_ctx ctx, int dtype, int prec, const tenet_tdesc* a, 
   p->spanC = hp.spanC;
   if (prec == TENET_PREC_NATIVE && 8.0 * hp.M * hp.N * hp.K * hp.batch >= LIB_MIN_FLOPS) {
     p->lib = plain_layout(hp);
-    p->lib.ok = p->lib.ok && lib_pays(dtype, p->lib.opA, hp.M, hp.N, hp.K, hp.batch);
+    p->lib.ok = p->lib.ok && lib_pays(dtype, p->lib.opA, p->lib.opB, hp.M, hp.N, hp.K, hp.batch);
   }
   std::vector<int64_t> host;
   size_t off[9];
@@ -2202,8 +2215,9 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
       const double fl = 8.0 * std::get<2>(key) * std::get<3>(key) * std::get<4>(key) * (double)kv.second.size();
       // a batch of eight or more fills the chip in one library launch; fewer
       // go there only where the library would take one of them alone
-      if (kv.second.size() < 8 && !lib_pays(dtype, (rocblas_operation)std::get<0>(key), std::get<2>(key),
-                                            std::get<3>(key), std::get<4>(key), (int64_t)kv.second.size()))
+      if (kv.second.size() < 8 && !lib_pays(dtype, (rocblas_operation)std::get<0>(key),
+                                            (rocblas_operation)std::get<1>(key), std::get<2>(key), std::get<3>(key),
+                                            std::get<4>(key), (int64_t)kv.second.size()))
         continue;
       if (fl < LIB_MIN_FLOPS || std::get<2>(key) < 16 || std::get<3>(key) < 16 || std::get<4>(key) < 16) continue;
       tenet_gplan_s::LibGroup lg;

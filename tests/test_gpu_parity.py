@@ -602,11 +602,12 @@ def test_einsum_split_i8_batched_conj_alpha_beta(ctx, conj):
 @pytest.mark.parametrize("conj", [(0, 0), (1, 0), (0, 1), (1, 1)])
 @pytest.mark.parametrize("layout", ["nn", "tt"])
 def test_einsum_plain_gemm_library_path(ctx, conj, layout):
-    """Native-precision contractions that are plain column-major GEMMs of at
-    least 1e8 flops run through the vendor library (strided-batched, with a
-    batch label, C = alpha op(A) op(B) + beta C): A.B with both operands
-    untransposed (a conjugated one then stays in the tile kernel) and with
-    both transposed (conjugation folds into op C), against numpy."""
+    """Native-precision contractions that are plain column-major GEMMs of many
+    tiles run through the vendor library (strided-batched, with a batch label,
+    C = alpha op(A) op(B) + beta C): A.B with both operands untransposed (a
+    conjugated one then stays in the direct kernel) and with both transposed
+    (conjugation folds into op C), against numpy.  Which one ran shows in the
+    contraction kernels' launch count: the library's is none of ours."""
     import ctypes as C
 
     import tenet_hip as T
@@ -614,7 +615,7 @@ def test_einsum_plain_gemm_library_path(ctx, conj, layout):
     from tenet_hip.device import tdesc
 
     rng = np.random.default_rng(51 + 2 * conj[0] + conj[1] + (10 if layout == "tt" else 0))
-    m, n, k, z = 160, 144, 200, 3  # 8 m n k z = 1.1e8 flops
+    m, n, k, z = 1030, 1000, 40, 3  # 816 tiles of 64 x 64
     for dt, tol in ((np.complex128, 1e-13), (np.complex64, 2e-6)):
         if layout == "nn":
             a = O.complex_gaussian(rng, (m, k, z)).astype(dt)
@@ -633,9 +634,13 @@ def test_einsum_plain_gemm_library_path(ctx, conj, layout):
                                         C.byref(h)), "plan")
         al = (C.c_double * 2)(0.5, -1.25)
         be = (C.c_double * 2)(-0.75, 0.5)
+        ctx.stats_enable(L.KSTAT_GEMM)
         L.check(L.lib.tenet_einsum_exec(h, None, C.c_void_p(A.ptr), C.c_void_p(B.ptr), C.c_void_p(Cd.ptr), conj[0],
                                         conj[1], al, be), "exec")
+        launches = ctx.stats_read()["launches"]
+        ctx.stats_enable(L.KSTAT_OFF)
         L.lib.tenet_plan_destroy(h)
+        assert launches == (1 if layout == "nn" and any(conj) else 0)
         aa = np.conj(a) if conj[0] else a
         bb = np.conj(b) if conj[1] else b
         ref = (0.5 - 1.25j) * np.einsum(spec, aa.astype(np.complex128), bb.astype(np.complex128)) + \

@@ -320,10 +320,12 @@ def test_grouped_plain_gemm_groups(ctx, dtype, tol):
     """Problems whose operands are plain column-major matrices run as batched
     library GEMMs from tenet_grouped_exec (grouped by shape and operand op):
     A.B, A^T.B, A.B^T, conj(A)^T.B, A.conj(B)^T (a strided view with ld
-    above the rows, as the Vidal output step reads V^H[:k]), next to a
-    permuted (gathered) problem and a small one that stay in the persistent
-    kernel.  Each against the oracle's binary_einsum, and the device-table
-    launch (every problem in the kernel) against the same reference."""
+    above the rows, as the Vidal output step reads V^H[:k]), next to permuted
+    (gathered) problems, small ones and a long contraction cut into K chunks
+    that stay in the persistent kernel, as do fewer copies than a library group
+    takes.  Each against the oracle's binary_einsum, and the device-table
+    launch (every problem in the kernel) against the same reference.  The work
+    the contraction kernels report tells which problems ran there."""
     import ctypes as C
 
     import tenet_hip as T
@@ -331,17 +333,21 @@ def test_grouped_plain_gemm_groups(ctx, dtype, tol):
     from tenet_hip.grouped import GroupedPlan
 
     rng = np.random.default_rng(33)
-    m, n, k = 256, 192, 160  # 63 MFLOP per problem: two make a library group
+    m, n, k = 128, 96, 160  # 15.7 MFLOP per problem: eight make a library group
     # (shape_a, labels_a, shape_b, labels_b, shape_c, labels_c, strides_b, conj, copies)
     cases = [
-        ((m, k), "ik", (k, n), "kj", (m, n), "ij", None, (0, 0), 3),
-        ((k, m), "ki", (k, n), "kj", (m, n), "ij", None, (0, 0), 2),
-        ((m, k), "ik", (n, k), "jk", (m, n), "ij", None, (0, 0), 2),
-        ((k, m), "ki", (k, n), "kj", (m, n), "ij", None, (1, 0), 2),
-        ((m, 2, k // 2), "iqr", (n, 2, k // 2), "jqr", (m, n), "ij", (1, n + 7, 2 * (n + 7)), (0, 1), 2),
-        ((k, m), "ki", (n, k), "jk", (n, m), "ji", None, (0, 0), 2),  # C transposed: kernel
-        ((6, 5), "ik", (5, 7), "kj", (6, 7), "ij", None, (0, 0), 3),  # small: kernel
+        ((m, k), "ik", (k, n), "kj", (m, n), "ij", None, (0, 0), 9),
+        ((k, m), "ki", (k, n), "kj", (m, n), "ij", None, (0, 0), 8),
+        ((m, k), "ik", (n, k), "jk", (m, n), "ij", None, (0, 0), 8),
+        ((k, m), "ki", (k, n), "kj", (m, n), "ij", None, (1, 0), 8),
+        ((m, 2, k // 2), "iqr", (n, 2, k // 2), "jqr", (m, n), "ij", (1, n + 7, 2 * (n + 7)), (0, 1), 8),
+        ((k, m), "ki", (n, k), "jk", (n, m), "ji", None, (0, 0), 8),  # C transposed: kernel
+        ((6, 5), "ik", (5, 7), "kj", (6, 7), "ij", None, (0, 0), 9),  # small: kernel
+        ((2 * m, k), "ik", (k, n), "kj", (2 * m, n), "ij", None, (0, 0), 7),  # seven: kernel
+        ((20, 20000), "ik", (20000, 17), "kj", (20, 17), "ij", None, (0, 0), 1),  # K chunks: kernel
     ]
+    in_kernel = 8.0 * (8 * m * n * k + 9 * 6 * 5 * 7 + 7 * 2 * m * n * k + 20 * 20000 * 17)
+    total = in_kernel + 8.0 * 41 * m * n * k
     probs, hosts, outs, ptrs, conj = [], [], [], [], []
     for sa, la, sb, lb, sc, lc, st_b, cj, copies in cases:
         for _ in range(copies):
@@ -365,6 +371,14 @@ def test_grouped_plain_gemm_groups(ctx, dtype, tol):
             ptrs += [da.ptr, db.ptr, dc.ptr]
             conj.append(cj)
     plan = GroupedPlan(ctx, probs, dtype, conj=conj)
+    assert plan.info()["split_tiles"] > 0
+
+    def counted(launch):
+        ctx.stats_enable(L.KSTAT_GEMM)
+        launch()
+        flops = ctx.stats_read()["flops"]
+        ctx.stats_enable(L.KSTAT_OFF)
+        return flops
 
     def check():
         for (a, b, la_, lb_, lc_, cj), (_, _, dc) in zip(hosts, outs):
@@ -379,14 +393,14 @@ def test_grouped_plain_gemm_groups(ctx, dtype, tol):
         for rep in range(2):
             for _, _, dc in outs:
                 dc.zero_()
-            plan.exec(ptrs)
+            assert counted(lambda: plan.exec(ptrs)) == in_kernel
             check()
         for _, _, dc in outs:
             dc.zero_()
         words = np.zeros(len(ptrs) + len(ptrs) % 2, dtype=np.uint64)
         words[:len(ptrs)] = ptrs
         tab = T.DeviceArray.from_host(ctx, words.view(np.complex128), np.complex128)
-        plan.exec_dev(tab.ptr)
+        assert counted(lambda: plan.exec_dev(tab.ptr)) == total
         check()
     finally:
         plan.close()
@@ -405,7 +419,7 @@ def test_grouped_plain_gemm_strided(ctx, dtype, tol):
     from tenet_hip.grouped import GroupedPlan
 
     rng = np.random.default_rng(34)
-    m, n, k, P = 256, 192, 160, 4
+    m, n, k, P = 256, 192, 160, 8
     for cj, sb, lb, st_b in [((0, 0), (k, n), "kj", None), ((0, 1), (n, k), "jk", (1, n + 5))]:
         a = [O.complex_gaussian(rng, (m, k), dtype) for _ in range(P)]
         bfull = [O.complex_gaussian(rng, (sb[0] + (5 if st_b else 0), sb[1]), dtype) for _ in range(P)]
@@ -424,7 +438,10 @@ def test_grouped_plain_gemm_strided(ctx, dtype, tol):
             pr = pr + (None, st_b)
         plan = GroupedPlan(ctx, [pr] * P, dtype, conj=[cj] * P)
         try:
+            ctx.stats_enable(L.KSTAT_GEMM)
             plan.exec([p for j in range(P) for p in (da[j].ptr, db[j].ptr, dc[j].ptr)])
+            assert ctx.stats_read()["launches"] == 0  # all of it in the library
+            ctx.stats_enable(L.KSTAT_OFF)
             for j in range(P):
                 b2 = np.conj(b[j]) if cj[1] else b[j]
                 ref = O.binary_einsum(O.OTensor(np.asarray(a[j], np.complex128), list("ik")),

@@ -1,0 +1,61 @@
+"""Which plain matrix products of at least 1e8 flops run in the vendor library
+and which in the direct kernel, either side of each line of the rule, and the
+results of both against numpy.  A library GEMM is none of the contraction
+kernels' launches.
+
+Tolerance as for the direct kernel: sums of at most 2 K terms in the dtype's
+precision, four times sqrt(2 K) units of it on the result's norm."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+import tenet_hip as T
+from tenet_hip import _lib as L
+from tenet_hip.device import tdesc
+
+pytestmark = pytest.mark.gpu
+
+Z, F = np.complex128, np.complex64
+
+
+def _gauss(rng, shape, dt):
+    return ((rng.standard_normal(shape) + 1j * rng.standard_normal(shape)) / np.sqrt(2)).astype(dt)
+
+
+# (M, N, K, batch), A and B as stored (n) or transposed (t), library?
+@pytest.mark.parametrize("dt,size,ops,library", [
+    # many tiles, either type and any order, but not along a narrow edge or for a tiny K
+    (Z, (1536, 2048, 33, 1), "nt", True), (Z, (1536, 2048, 31, 1), "nt", False), (F, (1536, 2048, 16, 1), "nn", True),
+    (F, (1536, 1984, 50, 1), "nn", False), (F, (63, 50000, 20, 1), "nt", False), (Z, (250, 255, 40, 48), "tn", True),
+    # complex128, full rounds of 5 GFLOP
+    (Z, (1024, 1024, 600, 1), "tt", True), (Z, (1024, 1024, 590, 1), "tt", False),
+    (Z, (1024, 1152, 600, 1), "tn", False),
+    # few tiles: complex128 as stored, complex64 with A along K
+    (Z, (500, 500, 500, 1), "nn", True), (Z, (500, 500, 500, 1), "tn", False), (Z, (179, 1030, 100, 1), "nn", False),
+    (Z, (384, 440, 100, 1), "nn", False), (F, (640, 640, 640, 1), "tn", True), (F, (640, 640, 640, 1), "nn", False),
+    (F, (448, 570, 60, 1), "tn", False), (F, (512, 512, 60, 1), "tn", True), (Z, (300, 700, 4001, 1), "nn", False),
+    # few tiles and a long K: never
+    (Z, (128, 128, 65536, 1), "nt", False), (F, (64, 64, 20000, 1), "tn", False),
+])
+def test_route_and_result(ctx, dt, size, ops, library):
+    M, N, K, Bt = size
+    rng = np.random.default_rng(M + N + K)
+    a = _gauss(rng, (M, K, Bt) if ops[0] == "n" else (K, M, Bt), dt)
+    b = _gauss(rng, (K, N, Bt) if ops[1] == "n" else (N, K, Bt), dt)
+    A, B, Cd = T.DeviceArray.from_host(ctx, a, dt), T.DeviceArray.from_host(ctx, b, dt), T.DeviceArray(ctx, (M, N, Bt), dt)
+    da = tdesc(a.shape, [1, 2, 4] if ops[0] == "n" else [2, 1, 4])
+    db = tdesc(b.shape, [2, 3, 4] if ops[1] == "n" else [3, 2, 4])
+    dc = tdesc((M, N, Bt), [1, 3, 4])
+    ctx.stats_enable(L.KSTAT_GEMM)
+    L.check(L.lib.tenet_einsum(ctx.h, None, A.code, 0, C.byref(da), C.c_void_p(A.ptr), C.byref(db),
+                               C.c_void_p(B.ptr), C.byref(dc), C.c_void_p(Cd.ptr), 0, 0), "einsum")
+    launches = ctx.stats_read()["launches"]
+    ctx.stats_enable(L.KSTAT_OFF)
+    assert launches == (0 if library else 1)
+    got = Cd.to_host()
+    for z in range(Bt):
+        x = (a if ops[0] == "n" else a.transpose(1, 0, 2))[..., z].astype(np.complex128)
+        y = (b if ops[1] == "n" else b.transpose(1, 0, 2))[..., z].astype(np.complex128)
+        ref = x @ y
+        assert np.linalg.norm(got[..., z] - ref) <= 4 * np.sqrt(2 * K + 2) * np.finfo(dt).eps * np.linalg.norm(ref)
