@@ -981,6 +981,12 @@ static void set_tables(GemmTables& t, int64_t* T, const size_t* off) {
 //    both as stored in complex128 (500^3 17 : 22, 1226 x 325 x 250 17 : 23) and
 //    A along K in complex64 (640^3 23 : 33, 1137 x 446 x 316 14 : 19), up to the
 //    K where few tiles leave it behind (385 x 2999 x 6279 1382 : 568).
+//  - batches of a thousand and more narrow products (400 shapes: edges 2 .. 100,
+//    K 2 .. 200, batch 140 .. 1e6), which it packs and the direct kernel takes
+//    one to a workgroup: complex128 as stored (8 x 8 x 8 by 200000 130 : 288),
+//    in the other orders from an edge of 30 on (47 x 49 x 24 by 2730 49 : 102;
+//    13 x 9 x 12 by 16312, A along K, 180 : 26), complex64 with A along K and few
+//    terms (20 x 20 x 20 by 100000 278 : 406; as stored the direct kernel wins).
 // Elsewhere it falls far behind (128 x 128 x 65536 7100 : 1000, complex64 256 x
 // 256 x 16384 3555 : 182).  The rule's choice is 1.4% slower than the better of
 // the two in the mean, 45% at worst (43 of 38 x 519 x 37, 10 : 15), where the
@@ -988,7 +994,12 @@ static void set_tables(GemmTables& t, int64_t* T, const size_t* off) {
 static bool lib_pays(int dtype, rocblas_operation opA, rocblas_operation opB, int64_t M, int64_t N, int64_t K,
                      int64_t batch) {
   const int64_t edge = std::min(M, N);
-  if (edge < 64) return false;
+  if (edge < 64) {
+    const bool as_stored = opA == rocblas_operation_none && opB == rocblas_operation_none;
+    if (batch < 1000 || edge < 3) return false;
+    if (dtype == TENET_C128) return as_stored || (edge >= 30 && K >= 6 && K <= 64);
+    return opA != rocblas_operation_none && opB == rocblas_operation_none && K <= 24;
+  }
   const double tiles = (double)((M + 63) / 64) * (double)((N + 63) / 64) * (double)batch;
   if (tiles >= 768) return K >= (dtype == TENET_C128 ? 32 : 16);
   if (dtype == TENET_C128 && 8.0 * M * N * K * batch >= 5e9 && tiles >= 0.92 * 256 * std::ceil(tiles / 256))

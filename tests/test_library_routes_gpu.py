@@ -35,6 +35,10 @@ def _gauss(rng, shape, dt):
     (Z, (500, 500, 500, 1), "nn", True), (Z, (500, 500, 500, 1), "tn", False), (Z, (179, 1030, 100, 1), "nn", False),
     (Z, (384, 440, 100, 1), "nn", False), (F, (640, 640, 640, 1), "tn", True), (F, (640, 640, 640, 1), "nn", False),
     (F, (448, 570, 60, 1), "tn", False), (F, (512, 512, 60, 1), "tn", True), (Z, (300, 700, 4001, 1), "nn", False),
+    # batches of narrow products
+    (Z, (8, 8, 8, 30000), "nn", True), (Z, (8, 9, 12, 30000), "tn", False), (Z, (30, 40, 64, 1000), "nt", True),
+    (Z, (30, 40, 65, 1000), "nt", False), (Z, (40, 40, 10, 999), "nn", False), (Z, (2, 9, 20, 50000), "nn", False),
+    (F, (20, 20, 24, 2000), "tn", True), (F, (20, 20, 25, 2000), "tn", False), (F, (20, 20, 24, 2000), "nn", False),
     # few tiles and a long K: never
     (Z, (128, 128, 65536, 1), "nt", False), (F, (64, 64, 20000, 1), "tn", False),
 ])
