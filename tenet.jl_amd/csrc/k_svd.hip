@@ -1106,14 +1106,19 @@ __device__ __forceinline__ void round_pair(int p, int round, int mode, int nb, i
 // 496 pairs of 512 rows, 63 us) the rounds run at 6.3 TB/s over X, read twice
 // and written once, from beyond the L2s.
 // mode 0: full inner sweep on the fixed pairs; mode 1: cross-block inner steps.
-constexpr int NXCD = SVD_XCDS;
-constexpr unsigned NCU = SVD_XCDS * SVD_XCD_CUS;
-
 //
 // UNITS: a batch's unit list and problem table, else the one problem among the
 // kernel's arguments (a choice at run time made every field a branch and a
 // scalar load that the next one waited for).
-template <bool ALONE, bool UNITS>
+// FIRST: the converged flag is waited for before the Gram's first loads go out,
+// not while they are under way.  A captured run's fixed number of sweeps
+// consists mostly of rounds over converged problems, whose loads (all of X at
+// 256 rows) are then not made: the n = 64, chi = 256 Vidal sweep replayed from
+// graphs 349 -> 329 ms, 31 captured 256 x 256 problems 8.2 -> 6.6 ms.
+constexpr int NXCD = SVD_XCDS;
+constexpr unsigned NCU = SVD_XCDS * SVD_XCD_CUS;
+
+template <bool ALONE, bool UNITS, bool FIRST>
 __global__ __launch_bounds__(SR_THREADS, ALONE ? 2 : 4) void svd_round_mfma_kernel(SvdBatch Bt, int round, int mode) {
   __shared__ SvSmem sm;
   int prob = 0, p, c, q, flip;
@@ -1134,6 +1139,7 @@ __global__ __launch_bounds__(SR_THREADS, ALONE ? 2 : 4) void svd_round_mfma_kern
   }
   const SvdProblem& P = UNITS ? Bt.arr[prob] : Bt.one;
   const int converged = P.flag[1];
+  if (FIRST && converged) return;
   const int nb = P.nblk;
   if (mode == 1 && (nb <= 2 || round >= nb - 1)) return;
   if (p >= nb / 2) return;
@@ -1824,7 +1830,7 @@ int launch_svd_init(const SvdBatch& b, int64_t nprob, int64_t max_elems, int max
   return TENET_OK;
 }
 
-int launch_svd_round(const SvdBatch& b, int64_t nprob, int max_items, int round, int phase, int mode,
+int launch_svd_round(const SvdBatch& b, int64_t nprob, int max_items, int round, int phase, int mode, bool flag_first,
                      hipStream_t s, hipEvent_t ev0, hipEvent_t ev1) {
   if (b.units && phase != 2) {
     set_error("SVD round: unit lists need the fused round kernel");
@@ -1837,9 +1843,13 @@ int launch_svd_round(const SvdBatch& b, int64_t nprob, int max_items, int round,
                             : (phase == 2 ? dim3((unsigned)dealt) : dim3((unsigned)max_items, (unsigned)nprob));
   if (phase == 2) {
     // one matrix has at most one workgroup with work per CU (svd_row_shares)
-    const auto kernel = !b.units         ? svd_round_mfma_kernel<true, false>
-                        : grid.x <= NCU ? svd_round_mfma_kernel<true, true>
-                                        : svd_round_mfma_kernel<false, true>;
+    const auto pick = [&](auto first) {
+      constexpr bool F = decltype(first)::value;
+      return !b.units        ? svd_round_mfma_kernel<true, false, F>
+             : grid.x <= NCU ? svd_round_mfma_kernel<true, true, F>
+                             : svd_round_mfma_kernel<false, true, F>;
+    };
+    const auto kernel = flag_first ? pick(std::true_type{}) : pick(std::false_type{});
     if (ev0)
       hipExtLaunchKernelGGL(kernel, grid, dim3(SR_THREADS), 0, s, ev0, ev1, 0, b, round, mode);
     else

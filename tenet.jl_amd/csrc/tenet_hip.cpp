@@ -286,9 +286,10 @@ static int upload_async(tenet_ctx ctx, hipStream_t s, void* dst, const void* src
 
 // launch_svd_round with its timing sample stamped by the dispatch
 static int svd_round_timed(tenet_ctx ctx, hipStream_t s, double flops, double bytes, const SvdBatch& B, int64_t nprob,
-                           int max_items, int round, int phase, int mode) {
+                           int max_items, int round, int phase, int mode, bool flag_first) {
   StatScope st(ctx, s, TENET_KSTAT_SVD_ROUND, flops, bytes, true);
-  const int rc = launch_svd_round(B, nprob, max_items, round, phase, mode, s, st.start_event(), st.stop_event());
+  const int rc =
+      launch_svd_round(B, nprob, max_items, round, phase, mode, flag_first, s, st.start_event(), st.stop_event());
   if (rc == TENET_OK) st.launched();
   return rc;
 }
@@ -1491,6 +1492,10 @@ static int svd_run(tenet_ctx ctx, hipStream_t s, int dtype, int64_t m, int64_t n
   TRY(launch_svd_init(B, 1, sh.nr * sh.ncp + sh.ncp * sh.ncp, (int)sh.ncp, dtype, s));
   const bool sync_ok = !capturing(s);
   const int max_sweeps = sync_ok ? 40 : CAPTURED_SWEEPS;
+  // captured rounds mostly find the matrix converged; below 256 rows waiting for
+  // the flag costs the live rounds more than the idle ones' loads (200 x 120 in
+  // complex128 1863 : 1896 us, 300 x 530 6705 : 6520)
+  const bool flag_first = !sync_ok && sh.nr >= 256;
   bool converged = false;
   // one sweep = a full-inner round on the fixed pairs (2i, 2i+1), then the
   // circle rounds with cross-block inner steps (every column pair once)
@@ -1503,14 +1508,15 @@ static int svd_run(tenet_ctx ctx, hipStream_t s, int dtype, int64_t m, int64_t n
   auto round = [&](int r, int mode) -> int {
     if (sh.split != SVD_TWO_PHASE) {
       TRY(svd_round_timed(ctx, s, gram_fl + apply_fl, 16.0 * sh.npairs * n2 * sh.nr + 2.0 * xv_bytes, B, 1,
-                          (int)sh.npairs, r, 2, mode));
+                          (int)sh.npairs, r, 2, mode, flag_first));
       // a sweep is nblk rounds, an even number: X is back in its own buffer
       // when it ends, also where a captured run's later rounds return at once
       if (sh.split == SVD_ONE_LAUNCH) std::swap(B.one.X, B.one.X2);
       return TENET_OK;
     }
-    TRY(svd_round_timed(ctx, s, gram_fl, 16.0 * sh.npairs * n2 * sh.nr, B, 1, (int)(sh.npairs * sh.q), r, 0, mode));
-    return svd_round_timed(ctx, s, apply_fl, 2.0 * xv_bytes, B, 1, (int)(sh.npairs * sh.q), r, 1, mode);
+    TRY(svd_round_timed(ctx, s, gram_fl, 16.0 * sh.npairs * n2 * sh.nr, B, 1, (int)(sh.npairs * sh.q), r, 0, mode,
+                        flag_first));
+    return svd_round_timed(ctx, s, apply_fl, 2.0 * xv_bytes, B, 1, (int)(sh.npairs * sh.q), r, 1, mode, flag_first);
   };
   for (int sw = 0; sw < max_sweeps && !converged; ++sw) {
     TRY(round(0, 0));
@@ -3036,7 +3042,7 @@ static int gsvd_run(tenet_gsvd g, hipStream_t s) {
   auto round0 = [&]() {
     SvdBatch Bu = B;
     Bu.units = g->units_dev + g->uoff[0];
-    return svd_round_timed(ctx, s, f0, b0, Bu, count, (int)g->ucnt[0], 0, 2, 0);
+    return svd_round_timed(ctx, s, f0, b0, Bu, count, (int)g->ucnt[0], 0, 2, 0, !sync_ok);
   };
   // the cross rounds, the sweep's end and (eagerly) its flags copy
   auto rest = [&](int sw) -> int {
@@ -3044,7 +3050,8 @@ static int gsvd_run(tenet_gsvd g, hipStream_t s) {
     for (int r = 0; r < g->max_rounds; ++r) {
       if (g->ucnt[(size_t)r + 1] == 0) continue;
       Bu.units = g->units_dev + g->uoff[(size_t)r + 1];
-      TRY(svd_round_timed(ctx, s, flr[(size_t)r], byr[(size_t)r], Bu, count, (int)g->ucnt[(size_t)r + 1], r, 2, 1));
+      TRY(svd_round_timed(ctx, s, flr[(size_t)r], byr[(size_t)r], Bu, count, (int)g->ucnt[(size_t)r + 1], r, 2, 1,
+                          !sync_ok));
     }
     TRY(launch_svd_sweep_end(B, count, s));
     if (sync_ok) {
