@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "internal.h"
+#include "tile_model.h"
 
 namespace tenet {
 static thread_local std::string g_err;
@@ -154,8 +155,8 @@ struct tenet_ctx_s {
   size_t stat_used = 0;
   int64_t stat_launches = 0, stat_sampled = 0, stat_every = 17;
   bool svd_precond = true;  // QR-preconditioned Jacobi for complex128 bond matrices (tenet_svd_set_precondition)
-  // grouped-launch tile costs per (tile, K step) relative to 64 x 64, per dtype (0 = unset)
-  double tile_cost[2][3] = {{0, 0, 0}, {0, 0, 0}};
+  // grouped-launch tile shapes: time per modelled cycle relative to 64 x 64, per dtype (1 until tuned)
+  double tile_eff[2][3] = {{1, 1, 1}, {1, 1, 1}};
   double stat_ms = 0.0, stat_flops = 0.0, stat_bytes = 0.0;
   // pinned landing slots for the per-sweep convergence flags of grouped SVD
   // runs (free list; a run takes one for its duration)
@@ -2056,6 +2057,7 @@ struct tenet_gplan_s {
   std::vector<int64_t> spanA, spanB, spanC;
   double flops = 0.0, bytes = 0.0;
   int64_t shape_count[4] = {0, 0, 0, 0};  // 64, 32, 16 tiles; GROUPED_SMALLK
+  double tile_cycles = 0.0;  // modelled cycles of the tiled problems' units
   int64_t split_tiles = 0;
   // Problems that are plain column-major GEMMs (every operand a matrix with
   // unit stride along rows or columns, no batch label), grouped by shape:
@@ -2088,48 +2090,10 @@ static bool plain_gemm(const HostPlan& hp, bool conjA, bool conjB, rocblas_opera
   return true;
 }
 
-static const int TILE_EDGE[3] = {64, 32, 16};
-
-// Cycles of a unit outside its K steps (queue, first loads, epilogue), and the
-// smallest unit worth cutting off a longer one.  Batches of 40..1024 unlike
-// problems time within 2% for 1000..6000 and 8192..32768.
-constexpr double UNIT_CYCLES = 3000.0, MIN_UNIT_CYCLES = 16384.0;
-
-// Cycles of a CU's address unit per wave load of 16 rows x 4 contracted
-// entries, from the cache lines it touches (rows: the runs of adjacent row
-// entries; k: those of the contracted entries; pair: two k steps per load).
-static double gather_cycles(const std::vector<int64_t>& rows, const std::vector<int64_t>& k, bool pair) {
-  auto run = [](const std::vector<int64_t>& t) {
-    if (t.size() < 2) return 1.0;
-    size_t breaks = 0;
-    for (size_t i = 1; i < t.size(); ++i) breaks += t[i] != t[i - 1] + 1;
-    return (double)t.size() / (double)(breaks + 1);
-  };
-  const double rr = rows.size() < 2 ? 16.0 : std::min(16.0, run(rows));
-  const double kr = k.size() < 2 ? 4.0 : std::min(4.0, run(k));
-  const double lines = std::max(4.0, 64.0 / std::max(rr, kr));
-  return (16.0 + 2.0 * lines) * (pair && rr < kr ? 0.5 : 1.0);
-}
-
-// Modelled cycles of one (tile, 16-wide K step) per tile shape: the larger of
-// the MFMA time on each SIMD (64, 16 and 4 blocks x 4 products over the four
-// waves) and the operand loads' address time.  The 32 x 32 shape, whose waves
-// deal K, measured 0.8 of that (five batches of each type, 4% in the mean).
-static void tile_step_cycles(int dtype, double clx, double cly, double c[3]) {
-  const double mf = dtype == TENET_C128 ? 64 : 32;
-  c[0] = std::max(64 * mf, 32 * (clx + cly));
-  c[1] = 0.8 * std::max(16 * mf, 8 * (clx + cly));
-  c[2] = std::max(4 * mf, 4 * (clx + cly));
-}
-
-// The model above with each shape's measured efficiency (tenet_autotune_tiles).
+// The model with each shape's measured efficiency (tenet_autotune_tiles).
 static void tile_costs(tenet_ctx ctx, int dtype, double clx, double cly, double c[3]) {
   tile_step_cycles(dtype, clx, cly, c);
-  const double* t = ctx->tile_cost[dtype == TENET_C128 ? 0 : 1];
-  if (t[0] <= 0) return;
-  double ref[3];  // the model's costs of the measured problem
-  tile_step_cycles(dtype, 24, 24, ref);
-  for (int v = 0; v < 3; ++v) c[v] *= t[v] * ref[0] / (t[0] * ref[v]);
+  for (int v = 0; v < 3; ++v) c[v] *= ctx->tile_eff[dtype == TENET_C128 ? 0 : 1][v];
 }
 
 static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count, const tenet_tdesc* descs,
@@ -2290,6 +2254,7 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
     q.kchunks = (int32_t)ch;
     q.kc = kcs * 16;
     const int64_t tiles = q.tiles_m * q.tiles_n * q.batch;
+    g->tile_cycles += tile_cycles(tile_step_cost[(size_t)i], tiles, ksteps, ch);
     q.part_base = -1;
     if (ch > 1) {
       const int64_t e = TILE_EDGE[q.shape];
@@ -2608,7 +2573,11 @@ extern "C" int tenet_autotune_tiles(tenet_ctx ctx, int dtype, double costs_out[3
     ptrs.push_back(b + ((size_t)P * M * K + (size_t)p * K * N) * es);
     ptrs.push_back(b + ((size_t)P * (M * K + K * N) + (size_t)p * M * N) * es);
   }
-  double cost[3] = {0, 0, 0};
+  const int d = dtype == TENET_C128 ? 0 : 1;
+  double cost[3] = {0, 0, 0}, cycles[3] = {0, 0, 0}, ms3[3] = {0, 0, 0};
+  // measured against the bare model, not against an earlier tuning
+  const double before[3] = {ctx->tile_eff[d][0], ctx->tile_eff[d][1], ctx->tile_eff[d][2]};
+  for (double& e : ctx->tile_eff[d]) e = 1.0;
   for (int v = 0; v < 3 && st == TENET_OK; ++v) {
     tenet_gplan_s g;
     st = grouped_plan_build(ctx, dtype, TENET_PREC_NATIVE, P, descs.data(), v, &g);
@@ -2626,16 +2595,20 @@ extern "C" int tenet_autotune_tiles(tenet_ctx ctx, int dtype, double costs_out[3
       }
       const int64_t e = TILE_EDGE[v];
       cost[v] = (double)best / ((double)P * ((M + e - 1) / e) * ((N + e - 1) / e) * (K / 16));
+      ms3[v] = best;
+      cycles[v] = g.tile_cycles;
     }
     (void)hipStreamSynchronize(s);
     if (g.dev) (void)tenet_free(ctx, g.dev);
   }
   (void)hipFree(buf);
-  TRY(st);
-  const int d = dtype == TENET_C128 ? 0 : 1;
-  for (int v = 0; v < 3; ++v) ctx->tile_cost[d][v] = cost[v] / cost[0];
+  if (st != TENET_OK) {
+    std::copy(before, before + 3, ctx->tile_eff[d]);
+    return st;
+  }
+  tile_efficiency(ms3, cycles, ctx->tile_eff[d]);
   if (costs_out)
-    for (int v = 0; v < 3; ++v) costs_out[v] = ctx->tile_cost[d][v];
+    for (int v = 0; v < 3; ++v) costs_out[v] = cost[v] / cost[0];
   return TENET_OK;
 }
 
