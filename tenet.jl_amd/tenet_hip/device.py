@@ -353,9 +353,13 @@ def tdesc(shape, labels, strides=None):
         for s in shape:
             strides.append(acc)
             acc *= int(s)
+    if type(labels) is not list:
+        labels = list(labels)
+    if type(strides) is not list:
+        strides = list(strides)
     try:
         return _desc_of(_PACK_DESC[rank](rank, 0, *shape, *strides, *labels))
-    except struct.error:  # entries that are not integers, or of unlike lengths
+    except (struct.error, TypeError):  # entries that int() makes integers (0-d arrays too), or unlike lengths
         d = L.TDesc()
         d.rank = rank
         for i, (e, st, lab) in enumerate(zip(shape, strides, labels)):

@@ -25,3 +25,13 @@ def test_fields(shape, labels, strides):
 def test_rank_limit():
     with pytest.raises(ValueError, match="rank above 8"):
         tdesc(range(9), range(9))
+
+
+def test_zero_dimensional_floats_and_generators():
+    """What int() takes is taken: 0-d float arrays (which have an __index__ that
+    refuses), and label and stride sequences that can be read only once."""
+    want = tdesc((2, 3), (5, 6), (1, 2))
+    assert bytes(tdesc((np.array(2.0), np.array(3.0)), (5, 6), (1, 2))) == bytes(want)
+    assert bytes(tdesc((2.0, 3), (x for x in (5, 6)), (x for x in (1, 2)))) == bytes(want)
+    with pytest.raises(TypeError):
+        tdesc((2, None), (5, 6), (1, 2))
