@@ -115,13 +115,10 @@ __global__ __launch_bounds__(256) void gemm_elements_kernel(GemmTables t, const 
 // (K 4..3840, 24 x 38 to 590000 x 20, both types) the choice is 2% slower than
 // the best of the six in the mean, 26% at worst (complex64 300 x 600 x 300,
 // 11.8 against 9.4 us).  From K = 128 on the WK = 1 shapes never won.
-// Shapes whose tiles a grid of 256-thread workgroups cannot number are passed
-// over while a larger one fits (3 x 17 in batches of 8.4e6 and more).
-constexpr double MAX_DIRECT_TILES = 0xffffff;  // HIP: fewer than 2^32 threads along x
 static int choose_direct(double cyc, int64_t I, int64_t J, int64_t K, int64_t batch, bool x_adj, bool y_adj) {
   const double clx = x_adj ? 24 : 48, cly = y_adj ? 24 : 48;
   int best = 0;
-  double best_t = 0.0, best_tiles = 0.0;
+  double best_t = 0.0;
   for (int c = 0; c < DIRECT_CFGS; ++c) {
     const DirectCfg& f = kDirect[c];
     if (f.wk == 1 && K >= 128) continue;
@@ -131,11 +128,9 @@ static int choose_direct(double cyc, int64_t I, int64_t J, int64_t K, int64_t ba
     const double steps = (double)((K + 4 * f.wk - 1) / (4 * f.wk));
     const double step = std::max(4 * cyc * f.ti * f.tj, 4 * (f.ti * clx + f.tj * cly));
     const double t = rounds * (steps * step / f.eff + 200.0 * f.ti * f.tj);
-    const bool fits = tiles <= MAX_DIRECT_TILES, best_fits = best_tiles <= MAX_DIRECT_TILES;
-    if (c == 0 || (fits == best_fits ? t < best_t : fits)) {
+    if (c == 0 || t < best_t) {
       best = c;
       best_t = t;
-      best_tiles = tiles;
     }
   }
   return best;
@@ -201,7 +196,7 @@ static int launch_direct(DirectArgs& p, const GemmLaunch& g, hipStream_t s) {
   p.tiles_i = (p.I + 16 * TI - 1) / (16 * TI);
   p.tiles_j = (p.J + 16 * TJ * WJ - 1) / (16 * TJ * WJ);
   const double total = (double)p.tiles_i * (double)p.tiles_j * (double)g.batch;
-  if (total > MAX_DIRECT_TILES) {
+  if (total > 0x7fffffffLL) {
     set_error("contraction too large for one launch");
     return TENET_ERR_UNSUPPORTED;
   }

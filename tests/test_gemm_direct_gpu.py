@@ -104,17 +104,3 @@ def test_alpha_beta_strided(ctx, size, dt):
     ref[:M] = al * (a[:M, :K] @ b[:K]) + be * c[:M]
     _check(got, ref, K, dt)
     assert np.array_equal(got[M:], c[M:].astype(dt))
-
-
-def test_more_tiles_than_a_grid_numbers(ctx):
-    """An outer product in a batch of 2^23: in tiles of 16 rows it would take two
-    workgroups an entry, one more than a launch can number; a larger tile takes
-    it.  Compared at the batch's ends and in its middle."""
-    Bt, M, N = 1 << 23, 3, 17
-    rng = np.random.default_rng(8)
-    a, b = (np.resize(_gauss(rng, (1021, x), np.complex64), (Bt, x)) for x in (M, N))  # a period of 1021 entries
-    got = T.binary_einsum(T.Tensor.from_host(ctx, a, "zm"), T.Tensor.from_host(ctx, b, "zn"), dims=[],
-                          out_labels=["m", "n", "z"]).to_host()
-    for z in (slice(0, 40), slice(Bt // 2 - 20, Bt // 2 + 20), slice(Bt - 40, Bt)):
-        ref = np.einsum("zm,zn->mnz", a[z].astype(np.complex128), b[z].astype(np.complex128))
-        _check(got[..., z], ref, 1, np.complex64)
