@@ -323,11 +323,10 @@ struct UnitCfg {
 using Tile64 = UnitCfg<2, 2, 2, 1>;
 using Tile32 = UnitCfg<2, 2, 1, 4>;
 using Tile16 = UnitCfg<1, 1, 1, 4>;
-// LDS values of the K-split fold (WK / 2 * TI * TJ * 512), with the slack that
-// puts the queue word behind them at 17408 / 34816 bytes, the offset the
-// kernel's generated code is checked for
-constexpr int FOLD_VALUES = 4352;
-static_assert(FOLD_VALUES >= 4 / 2 * 2 * 2 * 512, "fold buffer");
+// LDS values of the K-split fold of the largest tile whose waves deal K
+// (WK / 2 * TI * TJ * 512)
+constexpr int FOLD_VALUES = Tile32::WK / 2 * Tile32::TI * Tile32::TJ * 512;
+static_assert(FOLD_VALUES >= Tile16::WK / 2 * Tile16::TI * Tile16::TJ * 512, "fold buffer");
 
 // Split-K partials: a result-holding thread stores its registers at
 // ((wave * TI + i) * TJ + j) * 4 + r) * 64 + lane, as (re, im) pairs

@@ -50,5 +50,7 @@ def test_persistent_loop_has_one_cycle_through_the_queue_fetch(isa, kernel):
     assert "This Loop Header: Depth=3" not in body
     hdr = body.index("This Loop Header: Depth=1")
     fetch = body.index("global_atomic_add", hdr)
-    reads = [m.start() for m in re.finditer(r"ds_read_b32 v\d+, v\d+ offset:(17408|34816)\b", body)]
-    assert len(reads) == 1 and fetch < reads[0]
+    # the fetched index's LDS word: written right behind the fetch, read once
+    word = re.search(r"ds_write_b32 v\d+, v\d+ offset:(\d+)\n", body[fetch:])
+    reads = [m.start() for m in re.finditer(rf"ds_read_b32 v\d+, v\d+ offset:{word.group(1)}\b", body)]
+    assert len(reads) == 1 and fetch + word.start() < reads[0]
