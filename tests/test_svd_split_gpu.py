@@ -6,8 +6,9 @@ pair (33), ragged last strips and blocks (100 x 70, 257 x 130), the last row
 count of the one-launch rounds (768) and the next, and a batch whose rounds are
 cut for some problems and not for others.
 
-Tolerance: a column takes part in at most n rotations a sweep and about 16
-sweeps, each adding a few eps of its norm: 100 n eps of FP64; complex64 factors
+Tolerance: each of the n = min(shape) columns takes part in at most n rotations a
+sweep and about 16 sweeps, each adding a few eps of its norm: 100 n eps of FP64;
+norms and products over m = max(shape) rows add at most m eps; complex64 factors
 are rounded to 24 bits at the end: 8 eps of FP32 more."""
 import ctypes as C
 
@@ -26,7 +27,7 @@ def _matrix(rng, m, n, dt):
 
 
 def _check(a, u, s, vh):
-    n, tol = min(a.shape), 100 * max(a.shape) * 2.0 ** -52
+    n, tol = min(a.shape), (100 * min(a.shape) + max(a.shape)) * 2.0 ** -52
     if a.dtype == np.complex64:
         tol += 8 * 2.0 ** -23
     a, vh = a.astype(np.complex128), vh.astype(np.complex128)
