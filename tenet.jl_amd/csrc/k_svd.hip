@@ -539,10 +539,9 @@ __device__ __forceinline__ double from_next_slot(double x, int H, int lane) {
   return H == XB ? from_next_lane(x) : __shfl(x, lane, 64);
 }
 
-//
-// Each role runs its own copy of the loops below (so that its registers are its
-// own), chosen by a scalar branch on the wave's number; every copy passes the
-// same 1 + H barriers a level.
+// The levels and steps of jacobi_levels.  Each role runs its own copy of these
+// loops (so that its registers are its own), chosen by a scalar branch on the
+// wave's number; every copy passes the same 1 + H barriers a level.
 template <typename Init, typename Step, typename Done>
 __device__ __forceinline__ void level_loops(int h0, Init init, Step step, Done done) {
   int par = 0;  // the G buffer and rotation slots of the coming step

@@ -2,9 +2,10 @@
 singular values, the product and the factors' orthonormality.
 
 Shapes sit at the edges of the rule and of the strips: one column over a single
-pair (33), ragged last strips and blocks (100 x 70, 257 x 130), the last row
-count of the one-launch rounds (768) and the next, and a batch whose rounds are
-cut for some problems and not for others.
+pair (33), ragged last strips and blocks (100 x 70, 257 x 130), three and two pairs on
+an XCD (530 x 530, 768 x 300), the last row count of the one-launch rounds (768)
+and the next, and a batch whose rounds are cut for some problems and not for
+others.
 
 Tolerance: each of the n = min(shape) columns takes part in at most n rotations a
 sweep and about 16 sweeps, each adding a few eps of its norm: 100 n eps of FP64;
@@ -41,7 +42,7 @@ def _check(a, u, s, vh):
 
 
 @pytest.mark.parametrize("precondition", [False, True])
-@pytest.mark.parametrize("m,n", [(33, 33), (100, 70), (70, 100), (257, 130), (256, 256), (768, 48), (769, 48)])
+@pytest.mark.parametrize("m,n", [(33, 33), (100, 70), (70, 100), (257, 130), (256, 256), (768, 48), (769, 48), (530, 530), (768, 300)])
 def test_one_matrix(ctx, m, n, precondition):
     a, k = _matrix(np.random.default_rng(m + n), m, n, np.complex128), min(m, n)
     A = T.DeviceArray.from_host(ctx, a)
