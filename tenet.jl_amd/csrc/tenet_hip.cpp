@@ -1011,6 +1011,24 @@ static bool lib_pays(int dtype, rocblas_operation opA, rocblas_operation opB, in
   return opA != rocblas_operation_none && tiles >= 64;
 }
 
+// The same for one to seven equal products among others of a grouped launch,
+// which the persistent kernel takes with the rest at no call more.  The library
+// is ahead of it while their pointers happen to be evenly spaced (complex128 0.6
+// .. 0.95 of its time, complex64 0.55 .. 0.8), but over pointer arrays it falls
+// behind almost everywhere (complex128 1200 x 330 x 250 by 7 297 : 129, 1000 x
+// 1000 x 200 by 3 240 : 118; complex64 2000 x 2000 x 64 by 3 131 : 109), and one
+// 500^3 product taken out of a mixed launch costs it 85 : 78.  A plan does not
+// know its pointers, so only the large full-round products and the complex64
+// bands where it wins alone by the most leave the kernel.
+static bool lib_pays_few(int dtype, rocblas_operation opA, int64_t M, int64_t N, int64_t K, int64_t n) {
+  const double fl = 8.0 * M * N * K * n;
+  if (dtype == TENET_C128) {
+    const double rounds = (double)((M + 63) / 64) * (double)((N + 63) / 64) * (double)n / 256.0;
+    return fl >= 5e9 && rounds >= 0.92 * std::ceil(rounds);
+  }
+  return opA == rocblas_operation_none ? fl >= 3e10 && fl < 3e11 : fl >= 1.5e9 && fl < 6e9;
+}
+
 static int build_plan(tenet_ctx ctx, int dtype, int prec, const tenet_tdesc* a, const tenet_tdesc* b,
                       const tenet_tdesc* c, tenet_plan p) {
   HostPlan hp;
@@ -2193,20 +2211,21 @@ static int grouped_plan_build(tenet_ctx ctx, int dtype, int prec, int64_t count,
     }
     for (auto& kv : groups) {
       const auto& key = kv.first;
-      const double fl = 8.0 * std::get<2>(key) * std::get<3>(key) * std::get<4>(key) * (double)kv.second.size();
-      // a batch of eight or more fills the chip in one library launch; fewer
-      // go there only where the library would take one of them alone
-      if (kv.second.size() < 8 && !lib_pays(dtype, (rocblas_operation)std::get<0>(key),
-                                            (rocblas_operation)std::get<1>(key), std::get<2>(key), std::get<3>(key),
-                                            std::get<4>(key), (int64_t)kv.second.size()))
+      const auto oa = (rocblas_operation)std::get<0>(key);
+      const auto ob = (rocblas_operation)std::get<1>(key);
+      const int64_t M = std::get<2>(key), N = std::get<3>(key), K = std::get<4>(key);
+      const int64_t n = (int64_t)kv.second.size();
+      // a batch of eight or more fills the chip in one library launch; a plan of
+      // one problem goes where the same single product would (500^3 25 : 41)
+      if (n < 8 && !(count == 1 ? lib_pays(dtype, oa, ob, M, N, K, 1) : lib_pays_few(dtype, oa, M, N, K, n)))
         continue;
-      if (fl < LIB_MIN_FLOPS || std::get<2>(key) < 16 || std::get<3>(key) < 16 || std::get<4>(key) < 16) continue;
+      if (8.0 * M * N * K * n < LIB_MIN_FLOPS || M < 16 || N < 16 || K < 16) continue;
       tenet_gplan_s::LibGroup lg;
-      lg.opA = (rocblas_operation)std::get<0>(key);
-      lg.opB = (rocblas_operation)std::get<1>(key);
-      lg.M = std::get<2>(key);
-      lg.N = std::get<3>(key);
-      lg.K = std::get<4>(key);
+      lg.opA = oa;
+      lg.opB = ob;
+      lg.M = M;
+      lg.N = N;
+      lg.K = K;
       lg.lda = std::get<5>(key);
       lg.ldb = std::get<6>(key);
       lg.ldc = std::get<7>(key);

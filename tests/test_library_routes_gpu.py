@@ -63,3 +63,42 @@ def test_route_and_result(ctx, dt, size, ops, library):
         y = (b if ops[1] == "n" else b.transpose(1, 0, 2))[..., z].astype(np.complex128)
         ref = x @ y
         assert np.linalg.norm(got[..., z] - ref) <= 4 * np.sqrt(2 * K + 2) * np.finfo(dt).eps * np.linalg.norm(ref)
+
+
+# (M, N, K), A and B as stored (n) or transposed (t), copies, a small product beside them, library?
+@pytest.mark.parametrize("dt,size,ops,copies,beside,library", [
+    # the only problem of its plan: as the single product
+    (Z, (500, 500, 500), "nn", 1, False, True), (Z, (500, 500, 500), "tn", 1, False, False),
+    (F, (512, 512, 60), "tn", 1, False, True), (F, (2000, 2000, 1000), "nn", 1, False, True),
+    # a few: in the kernel, but for full rounds of 5 GFLOP in complex128 and a band of complex64
+    (Z, (500, 500, 500), "nn", 1, True, False), (Z, (500, 500, 500), "nn", 7, False, False),
+    (Z, (1024, 1024, 600), "tt", 1, True, True), (Z, (512, 512, 640), "nn", 4, False, True),
+    (Z, (512, 576, 640), "nn", 4, False, False),
+    (F, (512, 512, 60), "tn", 2, True, False), (F, (640, 640, 640), "tn", 1, True, True),
+    (F, (640, 640, 640), "nn", 2, True, False), (F, (640, 640, 640), "tn", 3, False, False),
+    (F, (2000, 2000, 1000), "nn", 1, True, True),
+])
+def test_route_of_grouped_products(ctx, dt, size, ops, copies, beside, library):
+    from tenet_hip.grouped import GroupedPlan
+    M, N, K = size
+    rng = np.random.default_rng(M + N + K + copies)
+    probs, hosts, outs, ptrs, small = [], [], [], [], 8.0 * 9 * 11 * 7
+    for m, n, k, o in [(M, N, K, ops)] * copies + [(9, 11, 7, "nn")] * beside:
+        a = _gauss(rng, (m, k) if o[0] == "n" else (k, m), dt)
+        b = _gauss(rng, (k, n) if o[1] == "n" else (n, k), dt)
+        A, B, Cd = T.DeviceArray.from_host(ctx, a, dt), T.DeviceArray.from_host(ctx, b, dt), T.DeviceArray(ctx, (m, n), dt)
+        probs.append((a.shape, "mk" if o[0] == "n" else "km", b.shape, "kn" if o[1] == "n" else "nk", (m, n), "mn"))
+        hosts.append((a if o[0] == "n" else a.T, b if o[1] == "n" else b.T))
+        outs.append((A, B, Cd))
+        ptrs += [A.ptr, B.ptr, Cd.ptr]
+    plan = GroupedPlan(ctx, probs, dt)
+    ctx.stats_enable(L.KSTAT_GEMM)
+    plan.exec(ptrs)
+    flops = ctx.stats_read()["flops"]
+    ctx.stats_enable(L.KSTAT_OFF)
+    got = [o[2].to_host() for o in outs]
+    plan.close()
+    assert flops == (0 if library else 8.0 * M * N * K * copies) + small * beside
+    for (a, b), x in zip(hosts, got):
+        ref = a.astype(np.complex128) @ b.astype(np.complex128)
+        assert np.linalg.norm(x - ref) <= 4 * np.sqrt(2 * a.shape[1] + 2) * np.finfo(dt).eps * np.linalg.norm(ref)
