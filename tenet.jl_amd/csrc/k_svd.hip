@@ -856,8 +856,9 @@ __device__ __forceinline__ svd_d4v mfma_f64(double a, double b, svd_d4v c) {
 // matrix cores.
 //
 // Returns false, with nothing formed, for a converged problem: its flag is
-// looked at when the first loads are under way, not before them.
-template <int D>
+// looked at when the first loads are under way, not before them (FIRST: the
+// caller has looked).
+template <int D, bool FIRST>
 __device__ __forceinline__ bool gram_mfma(SvSmem& sm, const double* X, int64_t ld, int r0, int r1, int I, int J, int b,
                                           int converged) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -878,7 +879,7 @@ __device__ __forceinline__ bool gram_mfma(SvSmem& sm, const double* X, int64_t l
     if (r0 + d * RS < r1)
 #pragma unroll
       for (int u = 0; u < 4; ++u) v[d][u] = X2[col[u] + min(own + d * RS, r1 - 1)];
-  if (converged) return false;
+  if (!FIRST && converged) return false;
   for (int r2 = r0; r2 < r1; r2 += D * RS) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -1101,9 +1102,10 @@ __device__ __forceinline__ void round_pair(int p, int round, int mode, int nb, i
 // chain: launch 3 us, Gram 8 us at 256 rows (loads, then 2450 cycles per 64
 // rows), inner solve 9 us (a sweep's first, fixed-pair round 17), rotation 2 us
 // (one 256 x 256 matrix: 21.5 us a round; with two launches, the partial Grams
-// on the VALU, it was 36).  With two workgroups on each CU (ALONE = false:
-// 496 pairs of 512 rows, 63 us) the rounds run at 6.3 TB/s over X, read twice
-// and written once, from beyond the L2s.
+// on the VALU, it was 36).  With two workgroups on each CU (ALONE = false: 496
+// pairs of 512 rows, 74 us in a whole sweep) a round fetches 193 MB of X, read
+// twice, and writes 93 beyond the L2s (3.9 TB/s) at 24 TFLOP/s: neither is the
+// bound, but the same chain, of which two workgroups hide a part of each other's.
 // mode 0: full inner sweep on the fixed pairs; mode 1: cross-block inner steps.
 //
 // UNITS: a batch's unit list and problem table, else the one problem among the
@@ -1148,7 +1150,7 @@ __global__ __launch_bounds__(SR_THREADS, ALONE ? 2 : 4) void svd_round_mfma_kern
   const double* Xs = (flip & 1) ? P.X2 : P.X;
   double* Xd = (flip & 2) ? P.X2 : P.X;
   const double abs_tol = fmax(4.930380657631324e-32 * (*P.fro2), 1e-300), tol = P.tol;
-  if (!gram_mfma<ALONE ? 4 : 2>(sm, Xs, P.nr, 0, P.nr, I, J, b, converged)) return;
+  if (!gram_mfma<(ALONE ? 4 : 2), FIRST>(sm, Xs, P.nr, 0, P.nr, I, J, b, converged)) return;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int S = strip_count(P);
   const int lo = (int)((int64_t)c * S / q), hi = (int)((int64_t)(c + 1) * S / q);
