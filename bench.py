@@ -53,7 +53,7 @@ PEAK_FP64_TFLOPS = 78.6
 # HBM bytes per round-kernel dispatch (FETCH_SIZE x 2.0 + WRITE_SIZE x 1.0 KiB,
 # factors from the scale kernel over 256 MiB) for each TEBD form, from
 # rocprofv3 --pmc passes over one sweep; None where not measured.
-ROUND_TRAFFIC_BYTES = {"vidal": 216_834_819, "vidal_graph": 216_834_819}
+ROUND_TRAFFIC_BYTES = {"fp64": 15_469_103, "vidal": 216_997_291}
 
 FORMS = {"fp64": 0, "fp32": 1, "split_bf16": 2, "split_fp16": 3, "vidal": 0, "vidal_graph": 0}
 DEFAULT_FORMS = "vidal,vidal_graph,fp64,split_bf16,split_fp16,fp32"
@@ -601,13 +601,13 @@ def bench_serving(args):
     if sat["amp_launches"] and sat["amp_kernel_ms"] > 0:
         ach = sat["amp_bytes"] / (sat["amp_kernel_ms"] * 1e-3) / 1e9
         roof = {"bound": "hbm", "achieved": round(ach, 2), "peak": 8000.0, "unit": "GB/s", "frac": round(ach / 8000, 5),
-                "traffic": None, "kernel": "amp_site_kernel (site-parallel amplitudes: one launch per site position, each "
-                                           "request's slice product over ceil(chi/16) workgroups)",
+                "traffic": None, "kernel": "amp_tile_kernel (site-parallel amplitudes: one launch per site position, tiles "
+                                           "of up to 16 requests sharing a slice by 16 columns of it)",
                 "measured_on": f"saturated leg: {sat['requests']} amplitude requests present at t = 0 "
                                f"(batches of up to 512), {sat['served_rps']} req/s",
-                "achieved_basis": "one selected slice per request and site (c64) / amplitude kernel time; a batch "
-                                  "of 512 requests over 32 states reads each slice ~8 times, the repeats from "
-                                  "L2 / Infinity Cache",
+                "achieved_basis": "nominal: one selected slice (c64) per request and site / amplitude kernel time; the "
+                                  "requests of a tile share its slice, which the kernel loads once for them all, "
+                                  "so fewer bytes than these move",
                 "launches": sat["amp_launches"], "avg_launch_us": round(sat["amp_kernel_ms"] * 1e3 / sat["amp_launches"], 1)}
     cpu = None
     if not args.no_cpu:
