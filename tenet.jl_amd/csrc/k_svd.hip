@@ -1115,7 +1115,7 @@ __device__ __forceinline__ void round_pair(int p, int round, int mode, int nb, i
 // not while they are under way.  A captured run's fixed number of sweeps
 // consists mostly of rounds over converged problems, whose loads (all of X at
 // 256 rows) are then not made: the n = 64, chi = 256 Vidal sweep replayed from
-// graphs 349 -> 329 ms, 31 captured 256 x 256 problems 8.2 -> 6.6 ms.
+// graphs 349 -> 326 ms, 31 captured 256 x 256 problems 8.2 -> 6.6 ms.
 constexpr int NXCD = SVD_XCDS;
 constexpr unsigned NCU = SVD_XCDS * SVD_XCD_CUS;
 
